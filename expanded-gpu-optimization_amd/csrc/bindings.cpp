@@ -99,8 +99,8 @@ std::vector<torch::Tensor> fused_forward_laplacian_backward(torch::Tensor coordi
   return {grad_parameters, grad_coordinates};
 }
 
-// The forward of the autograd glue's "saved" mode: (u, Laplacian, saved layers), the last an
-// opaque uint8 buffer of fhoad_saved_layers_size(batch) bytes for backward_for_autograd.
+// The saved-layer pair's forward: (u, Laplacian, buffer), the last an opaque uint8 buffer of
+// fhoad_saved_layers_size(batch) bytes for backward_for_autograd.
 std::vector<torch::Tensor> forward_saving(torch::Tensor coordinates, torch::Tensor parameters,
                                           int64_t version) {
   TORCH_CHECK(version >= 0 && version <= 5, "version must be 0 to 5");
@@ -128,8 +128,7 @@ std::vector<torch::Tensor> forward_saving(torch::Tensor coordinates, torch::Tens
 // upstream gradient may be None (zero, so no zeros tensor is made), and grad_coordinates is
 // computed only when want_coordinates is set (otherwise None is returned and nothing is
 // written). Same checks and kernels as fused_forward_laplacian_backward. saved:
-// forward_saving's buffer for the same coordinates and parameters (the backward then reads the
-// hidden layers instead of re-running the forward), or None.
+// forward_saving's buffer for the same coordinates and parameters (checked, not read), or None.
 std::vector<c10::optional<torch::Tensor>> backward_for_autograd(
     torch::Tensor coordinates, torch::Tensor parameters, c10::optional<torch::Tensor> grad_output,
     c10::optional<torch::Tensor> grad_laplacian, bool want_coordinates, int64_t version,
@@ -207,8 +206,9 @@ static_assert(fhoad::kOutputBase + fhoad::kHidden + 1 == kParameterCount, "packe
 // per-step host work (the Python apply, the backward's Python frame, the differentiable
 // torch.cat pack and its backward, or the ten gradient views built in Python). Inputs:
 // coordinates; the packed buffer when the model's parameters are its views
-// (flatten_poisson_parameters_), else None; the forward and backward versions; whether to keep
-// the hidden layers for the backward ("saved"); and the ten parameters in layout order (weight
+// (flatten_poisson_parameters_), else None; the forward and backward versions; save_layers (the
+// "saved" mode; nothing is kept, since the backward re-runs the forward faster than it could read
+// the layers back); and the ten parameters in layout order (weight
 // then bias of each linear layer), the Function's differentiable inputs. Without a buffer the
 // parameters are packed into a new one (one copy kernel, outside autograd). Each parameter gets
 // a view of the packed gradient with its own shape. An unused output's gradient arrives
@@ -219,7 +219,7 @@ struct ModelLaplacian : public torch::autograd::Function<ModelLaplacian> {
                                                 const torch::Tensor& coordinates,
                                                 const c10::optional<torch::Tensor>& packed,
                                                 int64_t version, int64_t backward_version,
-                                                bool save_layers, torch::TensorList parameters) {
+                                                bool /*save_layers*/, torch::TensorList parameters) {
     TORCH_CHECK(backward_version >= 1 && backward_version <= 6, "backward version must be 1 to 6");
     TORCH_CHECK(parameters.size() == kPackedSlices.size(), "expected the model's 10 parameters");
     for (size_t k = 0; k < kPackedSlices.size(); ++k) {
@@ -250,17 +250,14 @@ struct ModelLaplacian : public torch::autograd::Function<ModelLaplacian> {
     ctx->set_materialize_grads(false);
     ctx->saved_data["backward_version"] = backward_version;
     ctx->saved_data["packed_given"] = packed.has_value();
-    ctx->saved_data["save_layers"] = save_layers;
-    std::vector<torch::Tensor> out = save_layers ? forward_saving(coordinates, flat, version)
-                                                 : fused_forward_laplacian(coordinates, flat, version);
-    // Saved: coordinates, the packed buffer, the saved layers ("saved" mode) and, when the
+    std::vector<torch::Tensor> out = fused_forward_laplacian(coordinates, flat, version);
+    // Saved: coordinates, the packed buffer and, when the
     // buffer is the model's (its parameters are views of it), the ten parameters as well: each
     // view has its own version counter, so an in-place update of a parameter between this
     // forward and the backward (an optimizer step before a retain_graph backward) leaves the
     // buffer's counter alone; saving the views makes autograd's check of their counters raise
     // PyTorch's in-place-modification error there, as nn.Linear would. Saving copies nothing.
     std::vector<torch::Tensor> to_save{coordinates, flat};
-    if (save_layers) to_save.push_back(out[2]);
     if (packed.has_value()) to_save.insert(to_save.end(), parameters.begin(), parameters.end());
     ctx->save_for_backward(to_save);
     return {out[0], out[1]};
@@ -286,9 +283,7 @@ struct ModelLaplacian : public torch::autograd::Function<ModelLaplacian> {
     };
     const auto out = backward_for_autograd(
         saved[0], saved[1], upstream(grads[0]), upstream(grads[1]), needs_coordinates,
-        ctx->saved_data["backward_version"].toInt(),
-        ctx->saved_data["save_layers"].toBool() ? c10::optional<torch::Tensor>(saved[2])
-                                                : c10::nullopt);
+        ctx->saved_data["backward_version"].toInt(), c10::nullopt);
     if (needs_coordinates) result[0] = *out[1];
     if (needs_parameters) {
       const torch::Tensor& grad_flat = *out[0];

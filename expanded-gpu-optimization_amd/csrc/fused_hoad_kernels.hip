@@ -10,16 +10,16 @@
 //   output:  u = w_out . v + b_out,  lap = w_out . L
 //
 // Register layout. A wave owns a tile of 16 points. Each hidden layer is the product
-// Z[64 x 64] = W[64 x 64] * H[64 x (4 components x 16 points)], done with
-// v_mfma_f32_16x16x4f32 (FP32 in, FP32 accumulate). With m = lane % 16 and g = lane / 16, the
-// MFMA accumulator of output block mb and component c holds, in register r,
+// Z[64 x 64] = W[64 x 64] * H[64 x (4 components x 16 points)], done on the bf16 matrix cores with
+// operands split into three bf16 parts (float32 precision: see split_pair). With m = lane % 16
+// and g = lane / 16, the MFMA accumulator of output block mb and component c holds, in register r,
 //     Z[o = 16 mb + 4 g + r][c][point m].
-// The contraction order is free, so k-step (ob, j) assigns lane group g the input neuron
-// i = 16 ob + 4 g + j. Then the B operand a lane must supply at that step,
-//     H[16 ob + 4 g + j][c][point m],
-// is register j of the previous layer's accumulator (ob, c) in the same lane: a layer's output
-// is already in the operand layout of the next layer, and the tanh-jet update (which needs the
-// 4 components of one (neuron, point)) is local to a lane. Only the weights come from LDS.
+// The contraction order is free, so half t of it (32 neurons, one v_mfma_f32_16x16x32_bf16 per
+// product of parts) assigns lane group g the input neurons i = 32 t + 16 (e / 4) + 4 g + e % 4,
+// e = 0..7. Then the B operand a lane must supply, H[i][c][point m], is the previous layer's
+// accumulators of blocks 2 t and 2 t + 1 in the same lane: a layer's output, split, is already in
+// the operand layout of the next layer, and the tanh-jet update (which needs the 4 components of one
+// (neuron, point)) is local to a lane. Only the weights come from LDS.
 //
 // Scaled jet. With c = -2 log2(e) and lambda = log2(e), kernels carry the layer outputs as
 //   (v', J0', J1', L') = (c v / 4, J0 / 2, J1 / 2, lambda L / 4)
@@ -33,16 +33,16 @@
 // uses z'_J = 2 W0 columns; w_out is staged as 4 w_out / c and 4 w_out / lambda for u and lap.
 // The backward is backpropagation through this scaled network (weights 4 W): its dW sums are
 // of d/d(4 W), so the partial rows take a factor 4; bias gradients take c; layer-0 weight
-// gradients c for the x terms and 2 for the z_J terms. FP32 MFMA runs on the same SIMD issue
-// slots as VALU work on gfx950 (measured: they do not co-execute), so every VALU instruction
-// saved in the jet update is MFMA time recovered.
+// gradients c for the x terms and 2 for the z_J terms.
 //
-// LDS weight layouts. The forward kernel keeps W in MFMA operand order (one 16-byte read per
-// k-step, see stage_operand_weights); its small-batch form (forward_split_kernel) keeps only a
-// wave's 16 rows, in registers. The backward kernels (backward_kernel, and
-// backward_split_kernel for small batches) need both W and W^T operands from one copy:
-// W[o][i] at 68 o + i, read as W[16 mb + m][16 ob + 4 g + j], j = 0..3 (16 bytes) for the forward
-// recompute and as W[16 ob + 4 g + j][16 ib + m] (4 bytes) for W^T zbar.
+// What bounds the kernels: instruction issue and power. A wave's VALU instruction takes 4.4 clocks
+// of its SIMD (exp and rcp 8.5), a bf16 MFMA 8.5 clocks of issue and 16 (16 x 16 x 32) or 32
+// (32 x 32 x 16) of the matrix core, whose rest the VALU can use (v_dot2 instructions cannot). With
+// random data in all the matrix cores the shader clock falls from 2.4 to about 2.1 GHz.
+//
+// LDS weight layout: every kernel but forward_split_kernel (which keeps a wave's 16 rows in
+// registers) holds one copy of the split hidden weights in operand order (stage_operand_weights);
+// the backward kernels read W^T operands from the same copy with transposed LDS reads.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -62,8 +62,6 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWave = 64;
 constexpr int kTile = 16;     // points per wave tile (the MFMA N dimension)
-constexpr int kWRow = 68;     // LDS row pitch of the backward's 64-wide rows
-constexpr int kPlane = 4352;  // floats per 64 x 68 LDS plane
 
 // Scale factors of the carried jet (see the header comment).
 constexpr float kC = -2.8853900817779268f;       // c = -2 log2(e)
@@ -84,31 +82,159 @@ constexpr int kSmallWoutL = kSmallWoutV + kHidden;   // 4 w_out / lambda
 constexpr int kSmallBout = kSmallWoutL + kHidden;    // b_out
 constexpr int kSmallFloats = kSmallBout + 4;
 
-// Lane-dependent parts of the backward's two LDS access patterns on pitch-68 planes (value
-// (row, col) at 68 row + col): reading 4 consecutive columns of row m (16 bytes at
-// 68 m + 4 g) and reading one column m of rows 4 g + j (4 bytes at 272 g + m + 68 j). In both,
-// the 64 lanes cover distinct banks per 16-lane group, and the remaining offsets are immediates.
-__device__ __forceinline__ int lane_rows(int m, int g) { return kWRow * m + 4 * g; }
-__device__ __forceinline__ int lane_cols(int m, int g) { return 272 * g + m; }
+__device__ __forceinline__ f4 lds4(const float* p) { return *reinterpret_cast<const f4*>(p); }
 
-// The backward's dW staging buffer: six planes of [neuron row R][tile point p] in the weight
-// planes' layout, (R, p) at 68 R + p. Planes 0..2 hold zbar of the three "early" jet
-// components (early_component(e) in plane e), planes 3..5 h_prev of the same components; the
-// "late" component (J1) goes into planes 0 and 3 once the products of plane pair (0, 3) are done.
-// They are written 4 bytes per lane (lane (m, g) of wave w: rows 4 g + r of a 16-row block, point
-// 16 w + m; base lane_cols(m, g) + 16 w, conflict-free) and read 16 bytes per lane (row m,
-// points 4 g .. 4 g + 3 of a 16-point block; base lane_rows(m, g); 4 bank-conflict cycles per
-// read on gfx950, which overlap the MFMAs that consume them). Six planes at pitch 68 (104 KB)
-// fit beside the 52 KB of weight planes; at the conflict-free pitch 80 only four would.
-constexpr int kStagePlanes = 6;
-__device__ __forceinline__ constexpr int early_component(int e) { return e == 0 ? 0 : e == 1 ? 3 : 1; }
-constexpr int kLateComponent = 2;
+// ---------------------------------------------------------------------------------------------
+// Hidden products on the bf16 matrix cores at float32 precision. A float32 value is the exact
+// sum of three bf16 values, x = hi + mid + lo (round to nearest even each time: 8 + 8 + 8
+// significant bits and the signs of the remainders), so a product of two values is the sum of
+// nine bf16 products, each exact in float32. Six of them are formed (lo lo, lo mid and mid lo
+// are at most 2^-26 of the product and left out) on v_mfma_f32_16x16x32_bf16, which accumulates
+// in float32: 16 clocks for a 16 x 16 x 32 product against 256 for v_mfma_f32_16x16x4f32 (32
+// clocks, K = 4), so the six cost 3/8 of the float32 product. Against float64, a 64-term product
+// of random values is off by 0.9e-7 of its norm this way and by 1.45e-7 with
+// v_mfma_f32_16x16x4f32 (fewer roundings along the accumulation).
+// An infinite value, or one that rounds to an infinite bf16 (above 3.39e38), has an infinite hi
+// and a NaN remainder: what follows from it is NaN.
+typedef unsigned u4 __attribute__((ext_vector_type(4)));  // 8 bf16 values, two to a register
+typedef unsigned u2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
-__device__ __forceinline__ f4 mfma(float a, float b, f4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+constexpr int kParts = 3;  // hi, mid, lo
+
+// Two values rounded to bf16, a in the low half.
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((f2{a, b}), bf2));
 }
 
-__device__ __forceinline__ f4 lds4(const float* p) { return *reinterpret_cast<const f4*>(p); }
+// The three parts of two values, each part packed as bf16_pair packs them.
+__device__ __forceinline__ void split_pair(float a, float b, unsigned& hi, unsigned& mid,
+                                           unsigned& lo) {
+#pragma clang fp contract(off)  // x - hi of the float32 x, also where x is a product just formed
+  hi = bf16_pair(a, b);
+  a -= __builtin_bit_cast(float, hi << 16);
+  b -= __builtin_bit_cast(float, hi & 0xffff0000u);
+  mid = bf16_pair(a, b);
+  a -= __builtin_bit_cast(float, mid << 16);
+  b -= __builtin_bit_cast(float, mid & 0xffff0000u);
+  lo = bf16_pair(a, b);
+}
+
+// The parts of four values as the halves (two registers each) of operands.
+__device__ __forceinline__ void split4(const f4 x, u2 (&part)[kParts]) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    unsigned hi, mid, lo;
+    split_pair(x[2 * i], x[2 * i + 1], hi, mid, lo);
+    part[0][i] = hi;
+    part[1][i] = mid;
+    part[2][i] = lo;
+  }
+}
+
+__device__ __forceinline__ f4 mfma_bf16(u4 a, u4 b, f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, a),
+                                                 __builtin_bit_cast(bf8, b), c, 0, 0, 0);
+}
+
+// The six products in the order they accumulate, smallest first: parts of A and of B.
+constexpr int kProducts = 6;
+__device__ __forceinline__ constexpr int part_a(int k) { return k == 0 ? 2 : k == 1 || k == 3 ? 1 : 0; }
+__device__ __forceinline__ constexpr int part_b(int k) { return k == 2 ? 2 : k == 1 || k == 4 ? 1 : 0; }
+
+// A layer's output as the next product's B operand: half t (32 neurons) of the contraction, jet
+// component c, part s. The 32 k of a step are free to order, so lane group g's 8 are rows
+// 16 (2 t + e / 4) + 4 g + e % 4: the 4 values that the lane holds of output blocks 2 t and
+// 2 t + 1.
+struct JetOperand {
+  u4 part[2][4][kParts];
+};
+
+// -I as the A operand of v_mfma_f32_16x16x16_bf16 (lane (m, g) holds k = 4 g .. 4 g + 3 of row m).
+__device__ __forceinline__ u2 minus_identity(int m, int g) {
+  const int e = m - 4 * g;
+  return u2{e == 0 ? 0x0000bf80u : e == 1 ? 0xbf800000u : 0u,
+            e == 2 ? 0x0000bf80u : e == 3 ? 0xbf800000u : 0u};
+}
+
+// x - part for an output block's component in accumulator layout: its part, packed, is also the
+// B operand of a K = 16 product whose k are the block's rows. Exact, like the subtraction (one
+// nonzero product per row, and the difference is a float32 value).
+__device__ __forceinline__ f4 remainder_mfma(u2 minus_one, u2 part, f4 x) {
+  typedef short s4 __attribute__((ext_vector_type(4)));
+  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s4, minus_one),
+                                                   __builtin_bit_cast(s4, part), x, 0, 0, 0);
+}
+
+// The parts of an output block (16 rows x 4 components, accumulator layout). The kernels here
+// are bound by instruction issue (a VALU instruction takes 4.4 clocks of a SIMD's issue, an MFMA
+// 8.5 of its 16), so the two remainders of each value are formed on the matrix cores: 6 VALU
+// and 2 MFMA instructions per 4 values against 22 VALU (split4).
+__device__ __forceinline__ void split_block(u2 minus_one, const f4 (&x)[4], u2 (&part)[4][kParts]) {
+  f4 rest[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) rest[c] = x[c];
+#pragma unroll
+  for (int s = 0; s < kParts; ++s) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      part[c][s] = u2{bf16_pair(rest[c][0], rest[c][1]), bf16_pair(rest[c][2], rest[c][3])};
+      if (s + 1 < kParts) rest[c] = remainder_mfma(minus_one, part[c][s], rest[c]);
+    }
+  }
+}
+
+// Output block mb of a layer into its half of the next operand.
+__device__ __forceinline__ void put_block(u2 minus_one, JetOperand& h, int mb, const f4 (&x)[4]) {
+  u2 part[4][kParts];
+  split_block(minus_one, x, part);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+#pragma unroll
+    for (int s = 0; s < kParts; ++s) {
+      h.part[mb >> 1][c][s][2 * (mb & 1)] = part[c][s][0];
+      h.part[mb >> 1][c][s][2 * (mb & 1) + 1] = part[c][s][1];
+    }
+  }
+}
+
+// The weights' A operands of one output block: [half][part].
+struct WeightOperand {
+  u4 part[2][kParts];
+};
+
+// The products of a block in the order they accumulate: the five small ones of the contraction's
+// half 0, those of half 1, then hi hi of both. The matrix cores truncate as they accumulate, so
+// an accumulator should take its large terms last and few of them.
+template <int t>
+__device__ __forceinline__ void small_products(const WeightOperand& w, const JetOperand& h, f4 (&z)[4]) {
+#pragma unroll
+  for (int k = 0; k < kProducts - 1; ++k) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) z[c] = mfma_bf16(w.part[t][part_a(k)], h.part[t][c][part_b(k)], z[c]);
+  }
+}
+
+__device__ __forceinline__ void large_products(const WeightOperand& w, const JetOperand& h, f4 (&z)[4]) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) z[c] = mfma_bf16(w.part[t][0], h.part[t][c][0], z[c]);
+  }
+}
+
+// One output block: z[c] = W[16 mb + ., :] h_c, plus the bias for the value component.
+__device__ __forceinline__ void block_product(const WeightOperand& w, const JetOperand& h,
+                                              const f4 bias, f4 (&z)[4]) {
+  z[0] = bias;
+#pragma unroll
+  for (int c = 1; c < 4; ++c) z[c] = f4{0.f, 0.f, 0.f, 0.f};
+  small_products<0>(w, h, z);
+  small_products<1>(w, h, z);
+  large_products(w, h, z);
+}
 
 // tanh in the scaled jet, four values at a time. Input zv = c z_v; outputs v = (c / 4) tanh(z_v)
 // and s = (1 - tanh^2 z_v) / 4. With t = exp(-2 z_v) = exp2(zv) and u = 1 / (1 + t):
@@ -117,18 +243,14 @@ __device__ __forceinline__ f4 lds4(const float* p) { return *reinterpret_cast<co
 // (v_exp_f32, v_rcp_f32) per value. t overflows to +inf for z_v < -44 (u = 0: tanh = -1,
 // s = 0) and flushes to 0 for z_v > 44 (u = 1: tanh = 1, s = 0). Near tanh = +1, s carries the
 // absolute rounding of u (about 6e-8), as 1 - a^2 does.
-// The four values go in stages: the four exp2, then the four rcp, then the rest, with fences
-// so the scheduler keeps the stages. Each value's chain is serial (exp2 -> add -> rcp -> fma),
-// and left alone the compiler ran the chains one after another; a wave alone on its SIMD (the
-// backward, the forward's last tiles) then waited out every transcendental's latency.
+// The four values go in stages: the four exp2, then the four rcp, then the rest (each value's
+// chain is serial).
 __device__ __forceinline__ void tanh_scaled4(const f4 zv, f4& v, f4& s) {
   f4 u;
 #pragma unroll
   for (int r = 0; r < 4; ++r) u[r] = __builtin_amdgcn_exp2f(zv[r]);
-  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int r = 0; r < 4; ++r) u[r] = __builtin_amdgcn_rcpf(u[r] + 1.0f);
-  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     v[r] = __builtin_fmaf(u[r], 0.5f * kC, -0.25f * kC);
@@ -210,6 +332,22 @@ __device__ __forceinline__ T opaque(T x) {
   return x;
 }
 
+// Keep a value in an accumulation register (AGPR) from here on: for state that a full register
+// file has to hold through phases that do not use it. VALU instructions reach only the 256
+// architectural registers, and left alone the allocator spilled to memory instead.
+__device__ __forceinline__ void park(float& x) { __asm__ volatile("" : "+a"(x)); }
+__device__ __forceinline__ void park_block(f4 (&x)[4]) {
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float y = x[c][r];
+      park(y);
+      x[c][r] = y;
+    }
+  }
+}
+
 // Small-parameter staging shared by all kernels, in the scaled forms listed at kSmallCwx (the
 // factors 2 and 4 are exact), split into its global loads (load_small) and its LDS writes
 // (store_small), so that a kernel can issue these loads together with its other staging loads
@@ -262,101 +400,84 @@ __device__ __forceinline__ void store_small(float* s_small, int tid, SmallLoads 
   if (tid == 0) s_small[kSmallBout] = s.bout;
 }
 
-// Hidden-weight staging: every thread issues all of its global loads before its first LDS
-// write (16-byte loads when the parameter buffer is 16-byte aligned, 4-byte loads otherwise),
-// then scatters the values with put(layer, o, i, value) for W_layer[o][i].
-template <int kThreads, typename Put>
-__device__ __forceinline__ void stage_hidden(const float* __restrict__ params, int tid, Put put) {
-  constexpr int kQuads = 3 * kHidden * kHidden / 4;
-  constexpr int kPerThread = (kQuads + kThreads - 1) / kThreads;
-  if ((reinterpret_cast<uintptr_t>(params) & 15) == 0) {
-    f4 v[kPerThread];
+// Operands in LDS: one operand of a wave is 64 entries of 16 bytes, lane (m, g)'s at operand_entry.
+// The rotation of the 16 entries of each g by 4 g (as an xor) leaves a wave's own reads and writes
+// of its entries free of bank conflicts, and spreads the transposed reads (lds_transposed), whose 16
+// lanes take 8 bytes at 4 m and all four g, over all banks.
+__device__ __forceinline__ int operand_entry(int m, int g) { return 16 * g + (m ^ (4 * g)); }
+
+// LDS layout of the hidden weights, in MFMA operand order and split into bf16 parts: for hidden
+// layer l, output block mb, contraction half t, part s and lane (m, g), the 16 bytes at u4 index
+// (24 l + (2 mb + t) 3 + s) * 64 + operand_entry(m, g) hold part s of 4 W[16 mb + m][32 t +
+// 16 (e / 4) + 4 g + e % 4], e = 0..7 (the scaled jet's weights, in JetOperand's order). The offsets
+// within a layer are immediates. 72 KB.
+constexpr int kBlockU4 = 2 * kParts * kWave;  // u4 entries of one output block
+constexpr int kLayerU4 = 4 * kBlockU4;        // of one layer (24 KB)
+
+// One lane's operand of (layer, mb, t): 8 weights, loaded as two rows of four and split.
+__device__ __forceinline__ void load_weights8(const float* __restrict__ params, bool aligned, int layer,
+                                              int mb, int t, int lane, f4 (&w)[2]) {
+  const float* p = params + kHiddenBase + layer * kHiddenStride + (16 * mb + (lane & 15)) * kHidden +
+                   32 * t + 4 * (lane >> 4);
 #pragma unroll
-    for (int n = 0; n < kPerThread; ++n) {
-      const int q = tid + n * kThreads;
-      if (q < kQuads) {
-        const int layer = q >> 10, o = (q >> 4) & 63, i = (q & 15) << 2;
-        v[n] = *reinterpret_cast<const f4*>(params + kHiddenBase + layer * kHiddenStride +
-                                            (o << 6) + i);
-      }
-    }
+  for (int half = 0; half < 2; ++half) {
+    const float* q = p + 16 * half;
+    w[half] = aligned ? *reinterpret_cast<const f4*>(q) : f4{q[0], q[1], q[2], q[3]};
+  }
+}
+
+__device__ __forceinline__ void split_weights8(const f4 (&w)[2], u4 (&part)[kParts]) {
 #pragma unroll
-    for (int n = 0; n < kPerThread; ++n) {
-      const int q = tid + n * kThreads;
-      if (q < kQuads) {
-        const int layer = q >> 10, o = (q >> 4) & 63, i = (q & 15) << 2;
+  for (int half = 0; half < 2; ++half) {
+    u2 parts[kParts];
+    split4(4.0f * w[half], parts);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) put(layer, o, i + e, v[n][e]);
-      }
-    }
-  } else {
-    for (int k = tid; k < 4 * kQuads; k += kThreads) {
-      const int layer = k >> 12, o = (k >> 6) & 63, i = k & 63;
-      put(layer, o, i, params[kHiddenBase + layer * kHiddenStride + (o << 6) + i]);
+    for (int s = 0; s < kParts; ++s) {
+      part[s][2 * half] = parts[s][0];
+      part[s][2 * half + 1] = parts[s][1];
     }
   }
 }
 
-// Copy the packed parameters into LDS for the backward: the three hidden W, as 4 W (the scaled
-// jet's weights), into pitch-68 planes, the small blocks in the scaled forms listed at
-// kSmallCwx.
+// Staging: work item (l, mb, t, lane). A thread issues the loads of all its items before its
+// first LDS write.
 template <int kThreads>
-__device__ __forceinline__ void stage_parameters(const float* __restrict__ params, float* s_w,
-                                                 float* s_small, int tid) {
-  const SmallLoads small = load_small<kThreads>(params, tid);
-  stage_hidden<kThreads>(params, tid, [&](int layer, int o, int i, float value) {
-    s_w[layer * kPlane + kWRow * o + i] = 4.0f * value;
-  });
-  store_small(s_small, tid, small);
-}
-
-// Forward-only LDS layout of the hidden weights, in MFMA operand order: for hidden layer l,
-// k-step (ob, j) and lane (m, g), the 16 bytes at f4 index (16 l + 4 ob + j) * 64 + lane hold
-// 4 W[16 mb + m][16 ob + 4 g + j] for mb = 0..3 (the scaled jet's weights). One ds_read_b128
-// per k-step feeds the 4 MFMAs of that step; the 64 lanes read 1 KB contiguously (no bank
-// conflicts) and every k-step offset is an instruction immediate.
-constexpr int kOperandLayerF4 = 16 * kWave;  // f4 entries per layer (16 KB)
-
-// Staging: work item (l, ob, lane) loads the 4 x 4 block of W_l with rows m, 16 + m, 32 + m,
-// 48 + m and columns 16 ob + 4 g .. + 3 (four 16-byte global loads) and stores its 4 columns as
-// the 4 k-steps (ob, j) of that lane: 16-byte LDS writes, each wave's 64 of them to 1 KB
-// contiguous, so conflict-free. 768 work items: one per thread of a 12-wave workgroup, two for
-// some threads of an 8-wave one; a thread issues the loads of all its items before its first
-// LDS write.
-template <int kThreads>
-__device__ __forceinline__ void stage_operand_weights(const float* __restrict__ params, float* s_wa,
+__device__ __forceinline__ void stage_operand_weights(const float* __restrict__ params, u4* s_wa,
                                                       int tid) {
-  constexpr int kItems = 3 * 4 * kWave;  // (layer, ob, lane)
+  constexpr int kItems = 3 * 4 * 2 * kWave;  // (layer, mb, t, lane)
   constexpr int kPerThread = (kItems + kThreads - 1) / kThreads;
   const bool aligned = (reinterpret_cast<uintptr_t>(params) & 15) == 0;
-  f4* wa = reinterpret_cast<f4*>(s_wa);
-  f4 rows[kPerThread][4];
+  f4 rows[kPerThread][2];
 #pragma unroll
   for (int n = 0; n < kPerThread; ++n) {
     const int item = tid + n * kThreads;
     if (item < kItems) {
-      const int lane = item & (kWave - 1), ob = (item >> 6) & 3, layer = item >> 8;
-      const float* block = params + kHiddenBase + layer * kHiddenStride + (lane & 15) * kHidden +
-                           16 * ob + 4 * (lane >> 4);
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        const float* p = block + 16 * kHidden * mb;
-        rows[n][mb] = aligned ? *reinterpret_cast<const f4*>(p) : f4{p[0], p[1], p[2], p[3]};
-      }
+      load_weights8(params, aligned, item >> 9, (item >> 7) & 3, (item >> 6) & 1, item & 63, rows[n]);
     }
   }
 #pragma unroll
   for (int n = 0; n < kPerThread; ++n) {
     const int item = tid + n * kThreads;
     if (item < kItems) {
-      const int lane = item & (kWave - 1), ob = (item >> 6) & 3, layer = item >> 8;
+      u4 parts[kParts];
+      split_weights8(rows[n], parts);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        wa[(16 * layer + 4 * ob + j) * kWave + lane] =
-            4.0f * f4{rows[n][0][j], rows[n][1][j], rows[n][2][j], rows[n][3][j]};
+      for (int s = 0; s < kParts; ++s) {
+        s_wa[((item >> 6) * kParts + s) * kWave + operand_entry(item & 15, (item >> 4) & 3)] = parts[s];
       }
     }
   }
+}
+
+// One output block's operands from LDS; w is this lane's entry of the layer's first operand.
+__device__ __forceinline__ WeightOperand lds_weights(const u4* w, int mb) {
+  WeightOperand o;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+#pragma unroll
+    for (int s = 0; s < kParts; ++s) o.part[t][s] = w[mb * kBlockU4 + (t * kParts + s) * kWave];
+  }
+  return o;
 }
 
 // Layer-0 data of the 4 neurons o = 16 mb + 4 g + r (r = 0..3) held by this lane.
@@ -379,61 +500,6 @@ __device__ __forceinline__ Layer0Weights layer0_weights(const float* s_small, in
 
 __device__ __forceinline__ float layer0_zv(const Layer0Weights& w, int r, float x0, float x1) {
   return __builtin_fmaf(w.cwx[r], x0, __builtin_fmaf(w.cwy[r], x1, w.cb[r]));
-}
-
-// Forward hidden product with the operand-native weight layout: wa points at this lane's f4
-// in the layer's block; k-step (ob, j) reads wa[(4 ob + j) * 64]. Each k-step's operand is
-// read one k-step ahead, with a fence on both sides of the step's 16 MFMAs so the read stays
-// there: a wave that runs alone on its SIMD (the last tiles of a launch) then waits for no LDS
-// read; left alone, the compiler issued each read right before its MFMAs. `first` = wa[0],
-// read by the caller before the previous layer's tanh jet.
-__device__ __forceinline__ void hidden_product_native(const f4* wa, const f4 (&h)[4][4],
-                                                      const f4 (&bias)[4], f4 (&acc)[4][4],
-                                                      f4 first) {
-  f4 next = first;
-#pragma unroll
-  for (int ob = 0; ob < 4; ++ob) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int step = 4 * ob + j;
-      const f4 a = next;
-      if (step < 15) next = wa[(step + 1) * kWave];
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const f4 cin = (ob | j) ? acc[mb][c] : (c == 0 ? bias[mb] : f4{0.f, 0.f, 0.f, 0.f});
-          acc[mb][c] = mfma(a[mb], h[ob][c][j], cin);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-}
-
-// Scaled value biases c b of the 4 x 4 neurons 16 mb + 4 g + r held by this lane.
-__device__ __forceinline__ void load_bias(const float* s_small, int layer, int g, f4 (&bias)[4]) {
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) bias[mb] = lds4(s_small + kSmallBh + layer * kHidden + 16 * mb + 4 * g);
-}
-
-// tanh_jet over a layer's 16 values per lane, the tanh four at a time (tanh_scaled4).
-__device__ __forceinline__ void apply_tanh_jet(const f4 (&z)[4][4], f4 (&h)[4][4]) {
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
-    f4 v, sl;
-    tanh_scaled4(z[mb][0], v, sl);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float zj0 = z[mb][1][r], zj1 = z[mb][2][r];
-      const float q = __builtin_fmaf(zj0, zj0, zj1 * zj1);
-      h[mb][0][r] = v[r];
-      h[mb][1][r] = sl[r] * zj0;
-      h[mb][2][r] = sl[r] * zj1;
-      h[mb][3][r] = sl[r] * __builtin_fmaf(v[r], q, z[mb][3][r]);
-    }
-  }
 }
 
 // Layer 0 in closed form: the input jet is (x, I, 0), so z_J = W0 columns and z_L = 0, and
@@ -466,17 +532,6 @@ __device__ __forceinline__ void layer0_forward(const float* s_small, int g, floa
 // the whole kernel. An empty asm statement with a memory clobber at the top of each tile keeps
 // them as per-tile LDS reads.
 __device__ __forceinline__ void keep_lds_reads_in_loop() { __asm__ volatile("" ::: "memory"); }
-
-// A scheduling fence that only SALU instructions cross. Placed between the LDS reads for the
-// next step and the MFMAs of the current one, it keeps the reads issued a step ahead (at full
-// register use the scheduler otherwise sinks each read to just before its first use, and the
-// MFMA then waits out the LDS latency). It also keeps VALU work out of the MFMA runs: FP32
-// MFMA and VALU never execute together on gfx950, and a VALU instruction issued right after an
-// MFMA costs about 8 cycles more than one issued after another VALU instruction (measured with
-// a one-wave probe: 1 MFMA + k independent FMAs take 32.5 + 8 + 4.7 k cycles, 4 MFMAs + 16
-// FMAs no more than their separate times). Letting VALU cross, the scheduler had spread single
-// instructions between MFMAs, about 250 such switches per backward tile; with this fence 57.
-__device__ __forceinline__ void lds_mfma_fence() { __builtin_amdgcn_sched_barrier(0x0004); }
 
 // Value of lane l ^ 32 (permlane32) or l ^ 16 (permlane16) in every lane, with gfx950's
 // v_permlane32_swap / v_permlane16_swap (VALU, no LDS round trip). swap(u, 0) leaves the
@@ -554,45 +609,6 @@ __device__ __forceinline__ float row_reduce_scatter16(const float (&v)[16], int 
 }
 
 // ---------------------------------------------------------------------------------------------
-// Layer outputs saved by the forward for a backward that reads them instead of re-running the
-// forward (fhoad_forward_laplacian_saving, fhoad_forward_laplacian_backward_saved): per
-// 16-point tile t, hidden layer l (0..2 for layers 1..3), row block mb and jet component c, the
-// 64 lanes' f4 in lane order. Lane (m, g)'s f4 holds rows 16 mb + 4 g + r (r = 0..3) at point
-// 16 t + m, the MFMA accumulator layout every kernel here keeps a layer's output in, so each
-// store and load moves 1 KB per wave contiguously. 3,072 f4 (49,152 bytes) per tile.
-constexpr int64_t kSavedF4PerTile = 3 * 16 * kWave;
-__device__ __forceinline__ int64_t saved_index(int64_t tile, int layer, int mb, int c, int lane) {
-  return ((tile * 3 + layer) * 16 + 4 * mb + c) * kWave + lane;
-}
-
-// The forward writes the saved layers as non-temporal stores (about 2 us less per 64K call than
-// plain stores, measured); the backward reads them with plain loads (non-temporal loads
-// measured about 7 us slower per 64K call).
-__device__ __forceinline__ void store_saved(f4* __restrict__ saved, int64_t index, f4 value) {
-  __builtin_nontemporal_store(value, &saved[index]);
-}
-
-// One hidden layer's saved output of a 16-point tile into the accumulator layout (zeros for a
-// tile past the saved ones).
-__device__ __forceinline__ void load_saved_layer(const f4* __restrict__ saved, int64_t tile,
-                                                 int64_t saved_tiles, int layer, int lane,
-                                                 f4 (&h)[4][4]) {
-  if (tile < saved_tiles) {
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) h[mb][c] = saved[saved_index(tile, layer, mb, c, lane)];
-    }
-  } else {
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) h[mb][c] = f4{0.f, 0.f, 0.f, 0.f};
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------------------------
 // Forward kernel (replaces fused_forward_laplacian_tiled_kernel<2>,
 // /root/reference/csrc/fused_residual.cu:157-295). A grid of at most one workgroup per CU
 // stages the weights once, then every wave walks 16-point tiles: tile t < whole goes to
@@ -643,21 +659,79 @@ __device__ __forceinline__ bool quad_sync(unsigned* flag, unsigned target, int s
   return met;
 }
 
-// kSave: also write each tile's hidden-layer outputs to `saved` (saved_index).
-template <int kWaves, bool kSave>
+// Layer 0's output as the first hidden product's operand.
+__device__ __forceinline__ void layer0_operand(const float* s_small, u2 minus_one, int g, float x0,
+                                               float x1, JetOperand& h) {
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb) {
+    f4 x[4];
+    layer0_block(s_small, mb, g, x0, x1, x);
+    put_block(minus_one, h, mb, x);
+  }
+}
+
+// One output block's terms of u = w_out . v + b_out and lap = w_out . L, from the scaled jet.
+// Every path adds the four blocks' terms in block order.
+__device__ __forceinline__ f2 output_terms(const float* s_small, int mb, int g, const f4 (&h)[4]) {
+  const f4 wv = lds4(s_small + kSmallWoutV + 16 * mb + 4 * g);
+  const f4 wl = lds4(s_small + kSmallWoutL + 16 * mb + 4 * g);
+  f2 out{0.0f, 0.0f};
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    out[0] = __builtin_fmaf(wv[r], h[0][r], out[0]);
+    out[1] = __builtin_fmaf(wl[r], h[3][r], out[1]);
+  }
+  return out;
+}
+
+// Exchange of a 16-point tile whose rows are split over four waves: wave q's block of a layer's
+// output goes, split into parts, into its half of the next operand's entries, so that each wave
+// reads the whole operand 16 bytes at a time (1 KB contiguous per wave).
+struct Exchange {
+  u4 part[2][4][kParts][kWave];  // [half t][component][part][operand_entry], 24 KB
+};
+
+__device__ __forceinline__ void put_exchange(Exchange& x, u2 minus_one, int q, int entry,
+                                             const f4 (&mine)[4]) {
+  u2 part[4][kParts];
+  split_block(minus_one, mine, part);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+#pragma unroll
+    for (int s = 0; s < kParts; ++s) {
+      reinterpret_cast<u2*>(&x.part[q >> 1][c][s][entry])[q & 1] = part[c][s];
+    }
+  }
+}
+
+__device__ __forceinline__ void get_exchange(const Exchange& x, int entry, JetOperand& h) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int s = 0; s < kParts; ++s) h.part[t][c][s] = x.part[t][c][s][entry];
+    }
+  }
+}
+
+template <int kWaves>
 __global__ void __launch_bounds__(kWaves * kWave)
 forward_kernel(const float* __restrict__ coordinates, const float* __restrict__ params,
                float* __restrict__ output, float* __restrict__ laplacian, int64_t batch,
-               int64_t whole, int64_t tiles, f4* __restrict__ saved, int spin_limit) {
-  __shared__ __attribute__((aligned(16))) float s_wa[3 * kOperandLayerF4 * 4];
+               int64_t whole, int64_t tiles, int spin_limit) {
+  __shared__ u4 s_wa[3 * kLayerU4];
   __shared__ __attribute__((aligned(16))) float s_small[kSmallFloats];
-  __shared__ f4 s_x[2][4][4][kWave];  // split tiles: [buffer][wave q][component][lane], 32 KB
-  __shared__ unsigned s_quad;         // split tiles: quad_sync counter
+  __shared__ Exchange s_x[2];  // split tiles
+  __shared__ unsigned s_quad;  // split tiles: quad_sync counter
+  __shared__ unsigned s_next;  // the next k to take
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int g = lane >> 4;
   const int m = lane & 15;
-  const int64_t step = static_cast<int64_t>(gridDim.x) * kWaves;
+  // A workgroup's tiles are blockIdx.x + k gridDim.x; its waves take k from a counter in LDS as
+  // they go. A SIMD issues from its older wave first, so with equal shares the younger one of
+  // each pair was left to run the last 40 % of the time alone.
   // Coordinates are read one tile ahead (the first tile's during the staging), so no tile
   // waits for global memory; a wave that runs alone on its SIMD would expose that latency.
   int64_t tile = blockIdx.x + static_cast<int64_t>(wave) * gridDim.x;
@@ -666,24 +740,28 @@ forward_kernel(const float* __restrict__ coordinates, const float* __restrict__ 
     next_x0 = coordinates[2 * (tile * kTile + m)];
     next_x1 = coordinates[2 * (tile * kTile + m) + 1];
   }
-  if (threadIdx.x == 0) s_quad = 0;
+  if (threadIdx.x == 0) {
+    s_quad = 0;
+    s_next = kWaves;
+  }
   const SmallLoads small = load_small<kWaves * kWave>(params, threadIdx.x);
   stage_operand_weights<kWaves * kWave>(params, s_wa, threadIdx.x);
   store_small(s_small, threadIdx.x, small);
   __syncthreads();
   next_x0 = opaque(next_x0);  // delivered before the loop, for the same reason as below
   next_x1 = opaque(next_x1);
+  const int entry = operand_entry(m, g);
+  const u4* wa_lane = s_wa + entry;
+  const u2 minus_one = minus_identity(m, g);
 
   // ---- split tiles first: the last four waves, one 16-point tile at a time, rows split ----
   // (first, so their quarter tiles interleave with the other waves' whole tiles on each SIMD)
   const int q = wave - (kWaves - 4);
   if (q >= 0 && whole < tiles) {
     // Raised wave priority while on split tiles: the four waves of a quad meet three times a
-    // tile, each meeting waits for the slowest of them, and each shares its SIMD with two waves
-    // on whole tiles. (65,537 points: 54.9 -> 53.5 us per call, 70,000: 60.6 -> 57.7 us,
-    // 100,000: 79.8 -> 78.5 us; levels 1 to 3 measured the same.)
+    // tile, each meeting waits for the slowest of them, and each shares its SIMD with waves
+    // on whole tiles.
     __builtin_amdgcn_s_setprio(2);
-    const float* wa_q = s_wa + 4 * lane + q;  // component q of this lane's operand f4s
     unsigned meetings = 0;
     int phase = 0;  // alternates the exchange buffers across layers and tiles
     for (int64_t t = whole + blockIdx.x; t < tiles; t += gridDim.x) {
@@ -695,149 +773,114 @@ forward_kernel(const float* __restrict__ coordinates, const float* __restrict__ 
         x0 = coordinates[2 * point];
         x1 = coordinates[2 * point + 1];
       }
-      f4 h[4][4];
-      layer0_forward(s_small, g, x0, x1, h);
+      JetOperand h;
+      layer0_operand(s_small, minus_one, g, x0, x1, h);
       bool met = true;  // every quad meeting of this tile completed
 #pragma unroll
       for (int layer = 0; layer < 3; ++layer) {
         const f4 bias = lds4(s_small + kSmallBh + layer * kHidden + 16 * q + 4 * g);
-        f4 acc[4];
+        f4 z[4], mine[4];
+        block_product(lds_weights(wa_lane + layer * kLayerU4, q), h, bias, z);
+        tanh_jet4(z, mine);
+        Exchange& buf = s_x[phase];
+        phase ^= 1;
+        meetings += 4;
+        if (layer < 2) {
+          put_exchange(buf, minus_one, q, entry, mine);
+          met = quad_sync(&s_quad, meetings, spin_limit) && met;
+          get_exchange(buf, entry, h);
+        } else {
+          f2* terms = reinterpret_cast<f2*>(&buf);
+          terms[q * kWave + lane] = output_terms(s_small, q, g, mine);
+          met = quad_sync(&s_quad, meetings, spin_limit) && met;
+          if (q == 0) {
+            f2 out = terms[lane];
 #pragma unroll
-        for (int ob = 0; ob < 4; ++ob) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            // 4 W[16 q + m][16 ob + 4 g + j]: component q of k-step (ob, j)'s operand f4
-            const float a = wa_q[4 * ((16 * layer + 4 * ob + j) * kWave)];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              const f4 cin = (ob | j) ? acc[c] : (c == 0 ? bias : f4{0.f, 0.f, 0.f, 0.f});
-              acc[c] = mfma(a, h[ob][c][j], cin);
+            for (int mb = 1; mb < 4; ++mb) {
+              const f2 more = terms[mb * kWave + lane];
+              out[0] += more[0];
+              out[1] += more[1];
+            }
+            const float u = sum_lane_groups(out[0]), lap = sum_lane_groups(out[1]);
+            if (g == 0 && active) {
+              // A tile whose meetings gave up read stale rows: its outputs are NaN (and the
+              // device status word says why).
+              output[point] = met ? u + s_small[kSmallBout] : __builtin_nanf("");
+              laplacian[point] = met ? lap : __builtin_nanf("");
             }
           }
-        }
-        f4 mine[4];
-        tanh_jet4(acc, mine);
-        if (kSave) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) store_saved(saved, saved_index(t, layer, q, c, lane), mine[c]);
-        }
-        f4 (*buf)[4][kWave] = s_x[phase];
-        phase ^= 1;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) buf[q][c][lane] = mine[c];
-        meetings += 4;
-        met = quad_sync(&s_quad, meetings, spin_limit) && met;
-        if (layer < 2 || q == 0) {  // after the last layer only wave q = 0 (the output) reads
-#pragma unroll
-          for (int ob = 0; ob < 4; ++ob) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) h[ob][c] = buf[ob][c][lane];
-          }
-        }
-      }
-      if (q == 0) {
-        float u = 0.0f, lap = 0.0f;
-#pragma unroll
-        for (int mb = 0; mb < 4; ++mb) {
-          const f4 wv = lds4(s_small + kSmallWoutV + 16 * mb + 4 * g);
-          const f4 wl = lds4(s_small + kSmallWoutL + 16 * mb + 4 * g);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            u = __builtin_fmaf(wv[r], h[mb][0][r], u);
-            lap = __builtin_fmaf(wl[r], h[mb][3][r], lap);
-          }
-        }
-        u = sum_lane_groups(u);
-        lap = sum_lane_groups(lap);
-        if (g == 0 && active) {
-          // A tile whose meetings gave up read stale rows: its outputs are NaN (and the device
-          // status word says why).
-          output[point] = met ? u + s_small[kSmallBout] : __builtin_nanf("");
-          laplacian[point] = met ? lap : __builtin_nanf("");
         }
       }
     }
   }
 
   __builtin_amdgcn_s_setprio(0);
-  const f4* wa_lane = reinterpret_cast<const f4*>(s_wa) + lane;
-  for (; tile < whole; tile += step) {
+  while (tile < whole) {
     keep_lds_reads_in_loop();
     const int64_t point = tile * kTile + m;
     const bool active = point < batch;
     const float x0 = next_x0, x1 = next_x1;
-    const int64_t next_point = (tile + step) * kTile + m;
-    if (tile + step < whole && next_point < batch) {
+    unsigned k = 0;
+    if (lane == 0) k = __hip_atomic_fetch_add(&s_next, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    k = __builtin_amdgcn_readfirstlane(k);
+    tile = blockIdx.x + static_cast<int64_t>(k) * gridDim.x;
+    const int64_t next_point = tile * kTile + m;
+    if (tile < whole && next_point < batch) {
       next_x0 = coordinates[2 * next_point];
       next_x1 = coordinates[2 * next_point + 1];
     }
-    f4 first = wa_lane[0];
-    f4 h[4][4];
-    layer0_forward(s_small, g, x0, x1, h);
+    JetOperand h;
+    layer0_operand(s_small, minus_one, g, x0, x1, h);
+    f2 out{0.0f, 0.0f};
+#pragma unroll
     for (int layer = 0; layer < 3; ++layer) {
-      f4 bias[4];
-      load_bias(s_small, layer, g, bias);
-      f4 acc[4][4];
-      hidden_product_native(wa_lane + layer * kOperandLayerF4, h, bias, acc, first);
-      if (layer < 2) first = wa_lane[(layer + 1) * kOperandLayerF4];
-      apply_tanh_jet(acc, h);
-      if (kSave) {
+      JetOperand next;
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) store_saved(saved, saved_index(tile, layer, mb, c, lane), h[mb][c]);
+      for (int mb = 0; mb < 4; ++mb) {
+        f4 z[4], mine[4];
+        block_product(lds_weights(wa_lane + layer * kLayerU4, mb), h,
+                      lds4(s_small + kSmallBh + layer * kHidden + 16 * mb + 4 * g), z);
+        tanh_jet4(z, mine);
+        if (layer < 2) {
+          put_block(minus_one, next, mb, mine);
+        } else {
+          const f2 terms = output_terms(s_small, mb, g, mine);
+          out[0] = mb ? out[0] + terms[0] : terms[0];
+          out[1] = mb ? out[1] + terms[1] : terms[1];
         }
       }
+      if (layer < 2) h = next;
     }
     // Take delivery of the next coordinates here, before this tile's stores: a wait at the
     // top of the next tile would also wait for those stores (they sit behind a branch, so the
     // compiler cannot count them), and a store takes far longer than a tile's head.
     next_x0 = opaque(next_x0);
     next_x1 = opaque(next_x1);
-    // u = w_out . v + b_out and lap = w_out . L, from the scaled jet.
-    float u = 0.0f, lap = 0.0f;
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
-      const f4 wv = lds4(s_small + kSmallWoutV + 16 * mb + 4 * g);
-      const f4 wl = lds4(s_small + kSmallWoutL + 16 * mb + 4 * g);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        u = __builtin_fmaf(wv[r], h[mb][0][r], u);
-        lap = __builtin_fmaf(wl[r], h[mb][3][r], lap);
-      }
-    }
-    u = sum_lane_groups(u);
-    lap = sum_lane_groups(lap);
+    const float u = sum_lane_groups(out[0]), lap = sum_lane_groups(out[1]);
     if (g == 0 && active) {
       output[point] = u + s_small[kSmallBout];
       laplacian[point] = lap;
     }
   }
-
 }
 
 // ---------------------------------------------------------------------------------------------
 // Small-batch forward. With fewer tiles than SIMDs, forward_kernel's call time is one tile's
-// latency: 768 dependent MFMAs on one wave. Here a workgroup of 4 waves (one per SIMD) runs one
-// 16-point tile at a time, and wave w computes output rows 16 w .. 16 w + 15 of every layer
-// (64 MFMAs per layer instead of 256). The tanh-jet outputs go through LDS to the other waves,
-// which need all 64 rows as the next layer's B operand. In forward_kernel's register layout the
-// B operand of k-step (ob, j) is register j of accumulator (ob, c) of the same lane, so the
-// exchange is lane to lane: each wave stores its 4 f4 per lane and reads the other waves' f4
-// at the same lane index (1 KB contiguous per wave access, no bank conflicts). Two LDS buffers
-// alternate, so one barrier per layer suffices.
+// latency. Here a workgroup of 4 waves (one per SIMD) runs one 16-point tile at a time, and wave
+// w computes output rows 16 w .. 16 w + 15 of every layer (a quarter of the MFMAs). The tanh-jet
+// outputs go through LDS to the other waves, which need all 64 rows as the next layer's operand
+// (Exchange). Two LDS buffers alternate, so one barrier per layer suffices.
 //
 // Wave w's chains are forward_kernel's accumulators (mb = w, c) with the same operands in the
-// same order, layer 0 is the same closed form, and wave 0 forms u and lap in forward_kernel's
-// order, so both kernels give bitwise the same results.
+// same order, layer 0 is the same closed form, and wave 0 adds the blocks' output terms in
+// forward_kernel's order, so both kernels give bitwise the same results.
 constexpr int kSplitWaves = 4;
 
-template <bool kSave>
 __global__ void __launch_bounds__(kSplitWaves * kWave)
 forward_split_kernel(const float* __restrict__ coordinates, const float* __restrict__ params,
                      float* __restrict__ output, float* __restrict__ laplacian, int64_t batch,
-                     int64_t tiles, f4* __restrict__ saved) {
-  __shared__ f4 s_h[2][kSplitWaves][4][kWave];  // [buffer][wave][component][lane], 32 KB
+                     int64_t tiles) {
+  __shared__ Exchange s_x[2];
   __shared__ __attribute__((aligned(16))) float s_small[kSmallFloats];
   const int lane = threadIdx.x & (kWave - 1);
   const int w = threadIdx.x / kWave;
@@ -847,24 +890,27 @@ forward_split_kernel(const float* __restrict__ coordinates, const float* __restr
   // only after the barrier and the first tile's coordinates): issued together, the operand loads
   // were waited for before the barrier and a 1K-point call took 0.4 us longer.
   store_small(s_small, threadIdx.x, load_small<kSplitWaves * kWave>(params, threadIdx.x));
-  // A operands of this wave's rows: wa[l][ob][j] = 4 W_l[16 w + m][16 ob + 4 g + j] (the
-  // scaled jet's weights), loaded once (global memory, L2-resident) instead of staging
-  // the whole matrix in LDS.
-  f4 wa[3][4];
+  // This wave's operands (output block w of every layer), loaded once (global memory,
+  // L2-resident) instead of staging the whole matrix in LDS.
+  WeightOperand wa[3];
   {
-    const float* row = params + kHiddenBase + (16 * w + m) * kHidden + 4 * g;
     const bool aligned = (reinterpret_cast<uintptr_t>(params) & 15) == 0;
+    f4 rows[3][2][2];
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
 #pragma unroll
-      for (int ob = 0; ob < 4; ++ob) {
-        const float* p = row + l * kHiddenStride + 16 * ob;
-        wa[l][ob] = 4.0f * (aligned ? *reinterpret_cast<const f4*>(p) : f4{p[0], p[1], p[2], p[3]});
-      }
+      for (int t = 0; t < 2; ++t) load_weights8(params, aligned, l, w, t, lane, rows[l][t]);
+    }
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) split_weights8(rows[l][t], wa[l].part[t]);
     }
   }
   __syncthreads();  // s_small
 
+  const u2 minus_one = minus_identity(m, g);
+  const int entry = operand_entry(m, g);
   int phase = 0;  // alternates the exchange buffers across layers and tiles
   for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
     keep_lds_reads_in_loop();
@@ -875,70 +921,38 @@ forward_split_kernel(const float* __restrict__ coordinates, const float* __restr
       x0 = coordinates[2 * point];
       x1 = coordinates[2 * point + 1];
     }
-    f4 h[4][4];
-    layer0_forward(s_small, g, x0, x1, h);
+    JetOperand h;
+    layer0_operand(s_small, minus_one, g, x0, x1, h);
 #pragma unroll
     for (int layer = 0; layer < 3; ++layer) {
       const f4 bias = lds4(s_small + kSmallBh + layer * kHidden + 16 * w + 4 * g);
-      f4 acc[4];
+      f4 z[4], mine[4];
+      block_product(wa[layer], h, bias, z);
+      tanh_jet4(z, mine);
+      Exchange& buf = s_x[phase];
+      phase ^= 1;
+      if (layer < 2) {
+        put_exchange(buf, minus_one, w, entry, mine);
+        __syncthreads();
+        get_exchange(buf, entry, h);
+      } else {
+        f2* terms = reinterpret_cast<f2*>(&buf);
+        terms[w * kWave + lane] = output_terms(s_small, w, g, mine);
+        __syncthreads();
+        if (w == 0) {
+          f2 out = terms[lane];
 #pragma unroll
-      for (int ob = 0; ob < 4; ++ob) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            const f4 cin = (ob | j) ? acc[c] : (c == 0 ? bias : f4{0.f, 0.f, 0.f, 0.f});
-            acc[c] = mfma(wa[layer][ob][j], h[ob][c][j], cin);
+          for (int mb = 1; mb < 4; ++mb) {
+            const f2 more = terms[mb * kWave + lane];
+            out[0] += more[0];
+            out[1] += more[1];
+          }
+          const float u = sum_lane_groups(out[0]), lap = sum_lane_groups(out[1]);
+          if (g == 0 && active) {
+            output[point] = u + s_small[kSmallBout];
+            laplacian[point] = lap;
           }
         }
-      }
-      f4 mine[4];
-      {
-        f4 v, sl;
-        tanh_scaled4(acc[0], v, sl);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float q = __builtin_fmaf(acc[1][r], acc[1][r], acc[2][r] * acc[2][r]);
-          mine[0][r] = v[r];
-          mine[1][r] = sl[r] * acc[1][r];
-          mine[2][r] = sl[r] * acc[2][r];
-          mine[3][r] = sl[r] * __builtin_fmaf(v[r], q, acc[3][r]);
-        }
-      }
-      if (kSave) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) store_saved(saved, saved_index(tile, layer, w, c, lane), mine[c]);
-      }
-      f4 (*buf)[4][kWave] = s_h[phase];
-      phase ^= 1;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) buf[w][c][lane] = mine[c];
-      __syncthreads();
-      if (layer < 2 || w == 0) {  // after the last layer only wave 0 (the output) reads
-#pragma unroll
-        for (int ob = 0; ob < 4; ++ob) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) h[ob][c] = ob == w ? mine[c] : buf[ob][c][lane];
-        }
-      }
-    }
-    if (w == 0) {
-      float u = 0.0f, lap = 0.0f;
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        const f4 wv = lds4(s_small + kSmallWoutV + 16 * mb + 4 * g);
-        const f4 wl = lds4(s_small + kSmallWoutL + 16 * mb + 4 * g);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          u = __builtin_fmaf(wv[r], h[mb][0][r], u);
-          lap = __builtin_fmaf(wl[r], h[mb][3][r], lap);
-        }
-      }
-      u = sum_lane_groups(u);
-      lap = sum_lane_groups(lap);
-      if (g == 0 && active) {
-        output[point] = u + s_small[kSmallBout];
-        laplacian[point] = lap;
       }
     }
   }
@@ -952,16 +966,15 @@ forward_split_kernel(const float* __restrict__ coordinates, const float* __restr
 // tiles (16 points per wave). Per tile:
 //   1. every wave re-runs the forward for its 16 points, keeping each hidden layer's tanh-jet
 //      output h in registers;
-//   2. the adjoint is seeded from the linear output layer and walked back through layers 3..1:
-//      tanh-jet adjoint from h in registers (tanh_jet_adjoint_h, no tanh re-evaluated),
-//      dW += zbar h_prev^T, hbar = W^T zbar one input block at a time (registers), and
-//      finally layer 0 in closed form;
-//   3. dW contracts over the points of all 4 waves: zbar and h_prev are staged in LDS (three
-//      jet components written behind the MFMAs of the phase before, the fourth behind the first
-//      components' dW MFMAs; see staged_dw) and wave w owns output rows 16 w .. 16 w + 15 of
-//      every dW; the hidden bias gradients fall out of the same LDS reads. W0, b0 and w_out gradients are
-//      summed over each wave's points in registers (row_reduce_scatter16) and over the 4 waves once
-//      per slot.
+//   2. the adjoint is seeded from the linear output layer and walked back through layers 3..1
+//      (backward_layer): hbar = W^T zbar one 16-row input block at a time, each block's hbar
+//      feeding that block's tanh-jet adjoint at once (tanh_jet_adjoint_h, from h, no tanh
+//      re-evaluated), and dW += zbar h_prev^T; finally layer 0 in closed form;
+//   3. dW contracts over the points of all 4 waves: zbar and h_prev go through LDS one jet
+//      component at a time, split into bf16 parts, and wave w owns the 32 x 32 block
+//      (w >> 1, w & 1) of every dW. Bias, W0, b0 and w_out gradients are summed over each wave's
+//      points in registers (row_reduce_scatter16) and over the 4 waves once per slot.
+// Every hidden product runs on the bf16 matrix cores with split operands (see split_pair).
 // Weight gradients accumulate in registers across the tiles of a "slot": slot s takes the
 // workgroup tiles s, s + slots, s + 2 slots, ... in that order and writes one partial row.
 // A second kernel sums the rows in a fixed tree. The slot count depends only on the batch,
@@ -973,100 +986,100 @@ constexpr int kRowStride = 12800;            // floats per partial row (>= 12737
 constexpr int kReduceGroups = 16;            // fixed reduction tree: 16 groups of 16 slots
 static_assert(kMaxSlots % kReduceGroups == 0, "reduction tree must tile the slots");
 
+typedef float f16 __attribute__((ext_vector_type(16)));
+
 __device__ __forceinline__ f4 zero4() { return f4{0.f, 0.f, 0.f, 0.f}; }
 
-// Staging bases of one lane, formed where each phase starts (from opaque copies of the lane
-// offsets, see backward_kernel): writes of zbar (planes 0..2) and h_prev (planes 3..5) at rows
-// 4 g + r of a block and point 16 w + m; reads of the A operand (this wave's rows 16 w + m, zbar
-// planes) and of the B operands (rows 16 n + m, h_prev planes) at points 4 g .. 4 g + 3 of a
-// 16-point block. Every other offset is an instruction immediate (planes 0..2 from a base stay
-// within a DS offset's 64 KB reach, hence the second base for planes 3..5).
-struct StageBases {
-  float* wz;
-  float* wh;
-  const float* ra;
-  const float* rb;
-};
-
-// Staging write i (0..23) of block mb: the three early components of zbar (x, planes 0..2) and
-// of h_prev (y, planes 3..5), alternating, for this lane's rows 16 mb + 4 g + r.
-__device__ __forceinline__ void stage_early_write(const StageBases& sb, int mb, const f4 (&x)[4],
-                                                  const f4 (&y)[4], int i) {
-  const int e = i >> 3, r = (i >> 1) & 3;
-  float* base = (i & 1) ? sb.wh : sb.wz;
-  base[e * kPlane + kWRow * (16 * mb + r)] = (i & 1) ? y[early_component(e)][r] : x[early_component(e)][r];
+// Transposed read of bf16 values in LDS (ds_read_b64_tr_b16): within each 16 lanes, lanes
+// 4 j .. 4 j + 3 point at the 16 values of row j, 8 bytes each, and lane l gets column l of the
+// four rows.
+__device__ __forceinline__ u2 lds_transposed(const u2* p) {
+  typedef short s4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s4 lds_s4;
+  return __builtin_bit_cast(u2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)p));
 }
 
-// Staging write i (0..31) of the late component: zbar (xl[mb], plane 0) and h_prev (yl[mb],
-// plane 3), alternating, rows 16 mb + 4 g + r.
-__device__ __forceinline__ void stage_late_write(const StageBases& sb, const f4 (&xl)[4],
-                                                 const f4 (&yl)[4], int i) {
-  const int mb = i >> 3, r = (i >> 1) & 3;
-  float* base = (i & 1) ? sb.wh : sb.wz;
-  base[kWRow * (16 * mb + r)] = (i & 1) ? yl[mb][r] : xl[mb][r];
-}
+// W^T operands from the same LDS copy as the forward's (stage_operand_weights): for hbar of input
+// block ib, lane (m, g) supplies W[32 t + 16 (e / 4) + 4 g + e % 4][16 ib + m], e = 0..7: two
+// transposed reads of rows 4 g .. 4 g + 3 of output blocks 2 t and 2 t + 1. w is this lane's entry
+// (transposed_entry) of the layer.
+__device__ __forceinline__ int transposed_entry(int m, int g) { return operand_entry(4 * g + (m >> 2), m & 3); }
 
-// The five 16-byte operands of one dW step: the A operand zbar[16 w + m][p] and the B operands
-// h_prev[16 n + m][p], n = 0..3, for p = 16 s + 4 g + k, k = 0..3, of the component staged in
-// plane pair (plane, 3 + plane).
-struct DwOperands {
-  f4 a, b[4];
-};
-
-__device__ __forceinline__ DwOperands dw_read(const StageBases& sb, int plane, int s) {
-  DwOperands o;
-  o.a = lds4(sb.ra + plane * kPlane + 16 * s);
+__device__ __forceinline__ void lds_transposed_half(const u4* w, int ib, int t, u4 (&part)[kParts]) {
 #pragma unroll
-  for (int n = 0; n < 4; ++n) o.b[n] = lds4(sb.rb + plane * kPlane + 16 * kWRow * n + 16 * s);
+  for (int s = 0; s < kParts; ++s) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const u4* entry = w + (2 * t + i) * kBlockU4 + ((ib >> 1) * kParts + s) * kWave;
+      const u2 v = lds_transposed(reinterpret_cast<const u2*>(entry) + (ib & 1));
+      part[s][2 * i] = v[0];
+      part[s][2 * i + 1] = v[1];
+    }
+  }
+}
+
+__device__ __forceinline__ WeightOperand lds_transposed_weights(const u4* w, int ib) {
+  WeightOperand o;
+  lds_transposed_half(w, ib, 0, o.part[0]);
+  lds_transposed_half(w, ib, 1, o.part[1]);
   return o;
 }
 
-// dW[16 w + ., 16 n + .] += sum over the 64 tile points of zbar_c h_prev_c^T for the components
-// staged in plane pairs (kFirst + i, kFirst + 3 + i), i < kN: four steps (point blocks) per
-// component, 16 MFMAs each contracting over the step's points; every lane supplies the same
-// points at each step. `ops` holds the first step's operands on entry and each step reads the
-// next step's; with kNext >= 0 the last step reads the first operands of plane pair kNext into
-// `ops`. emit(step, k) issues staging writes after the MFMAs of point k: they follow the next
-// step's reads, so waiting for those reads never waits for them, and they drain behind the
-// MFMAs. With kBias, returns the sum of this lane's reads of the first component (the hidden bias
-// gradient's partial for row 16 w + m when it is zbar_v).
-template <int kFirst, int kN, bool kBias, int kNext, typename Emit>
-__device__ __forceinline__ float dw_pass(const StageBases& sb, DwOperands& ops, f4 (&dw)[4],
-                                         Emit emit) {
-  float bias = 0.0f;
-#pragma unroll
-  for (int step = 0; step < 4 * kN; ++step) {
-    const DwOperands cur = ops;
-    if (kBias && step < 4) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) bias += cur.a[k];
-    }
-    if (step + 1 < 4 * kN) {
-      ops = dw_read(sb, kFirst + ((step + 1) >> 2), (step + 1) & 3);
-    } else if (kNext >= 0) {
-      ops = dw_read(sb, kNext, 0);
-    }
-    lds_mfma_fence();
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-#pragma unroll
-      for (int n = 0; n < 4; ++n) dw[n] = mfma(cur.a[k], cur.b[n][k], dw[n]);
-      if (emit(step, k)) __builtin_amdgcn_sched_barrier(0);
-    }
-    lds_mfma_fence();
-  }
-  return bias;
+// dW operands. A 16-point set's values of one tensor and component, split, lie in LDS as they are
+// the hidden products' B operand: entry (t, s, lane (m, g)) holds part s of rows 32 t + 16 (e / 4) +
+// 4 g + e % 4 at point m. For v_mfma_f32_32x32x16_bf16 (A or B: lane (n, h) = (lane % 32, lane / 32)
+// supplies row n at points 8 h .. 8 h + 7), two transposed reads give 4 points each of row n of
+// half t, points 8 h .. 8 h + 3 from `lo` and 8 h + 4 .. 8 h + 7 from `hi` (this lane's 8 bytes of
+// part 0: dw_lane_offset, and half t's entries).
+struct DwOperand {
+  u4 part[kParts];
+};
+struct DwPointers {
+  const u2 *lo, *hi;
+};
+
+__device__ __forceinline__ int dw_lane_offset(int m, int g, int i) {  // in u2 (8 bytes)
+  return 2 * operand_entry(8 * (g >> 1) + 4 * i + (m >> 2), m & 3) + (g & 1);
 }
 
-// emit() that issues nothing.
-struct NoEmit {
-  __device__ __forceinline__ bool operator()(int, int) const { return false; }
-};
+__device__ __forceinline__ DwPointers dw_pointers(const u4* entries, int m, int g) {
+  const u2* p = reinterpret_cast<const u2*>(entries);
+  return {p + dw_lane_offset(m, g, 0), p + dw_lane_offset(m, g, 1)};
+}
 
-// after() that does nothing.
-struct NoAfter {
-  __device__ __forceinline__ void operator()(int) const {}
-};
+// `at`: u4 offset of the set from the pointers'.
+__device__ __forceinline__ DwOperand lds_dw_operand(const DwPointers& p, int at) {
+  DwOperand o;
+#pragma unroll
+  for (int s = 0; s < kParts; ++s) {
+    const u2 lo = lds_transposed(p.lo + 2 * (at + s * kWave)), hi = lds_transposed(p.hi + 2 * (at + s * kWave));
+    o.part[s] = u4{lo[0], lo[1], hi[0], hi[1]};
+  }
+  return o;
+}
+
+__device__ __forceinline__ f16 mfma_dw(u4 a, u4 b, f16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), c, 0, 0, 0);
+}
+
+// sum += A B^T over the operands' 16 points, the products smallest first.
+//
+// The matrix cores truncate as they accumulate, towards minus infinity, so the errors of many
+// additions have the same sign and do not cancel: adjoints and weight-gradient sums formed there
+// without more care were up to 4 times further from float64 than with float32 products (gradients
+// of 262,144 points whose contributions cancel). So every other tile of a slot, and every other
+// slot's first, runs its whole walk back on the negated upstream gradients (walk_sign) and its
+// sums are subtracted: the truncations of both halves cancel. And an accumulator holds one
+// component of one tile (64 points); the slot's sums are formed in float32, rounded to nearest.
+__device__ __forceinline__ f16 add_products(const DwOperand& a, const DwOperand& b, f16 sum) {
+#pragma unroll
+  for (int k = 0; k < kProducts; ++k) sum = mfma_dw(a.part[part_a(k)], b.part[part_b(k)], sum);
+  return sum;
+}
+
+__device__ __forceinline__ float walk_sign(int slot, int round) { return ((slot ^ round) & 1) ? -1.0f : 1.0f; }
+
+__device__ __forceinline__ f16 zero16() { return f16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}; }
 
 // Per-neuron sums over a wave's 16 points without LDS: lane (m, g) holds x for neuron
 // 16 mb + 4 g + r at point m, so summing value k = 4 mb + r over the 16 lanes of row g gives
@@ -1074,31 +1087,6 @@ struct NoAfter {
 // thus keeps the total of neuron owned_neuron(m, g) = 16 (m >> 2) + 4 g + (m & 3): the 64 lanes
 // own the 64 neurons once each.
 __device__ __forceinline__ int owned_neuron(int m, int g) { return 16 * (m >> 2) + 4 * g + (m & 3); }
-
-// dW += zbar h_prev^T over the workgroup tile from the staged planes, once the early components
-// of zbar and h_prev are written (planes 0..2, 3..5) and the late ones are in registers (xl: zbar,
-// yl: h_prev, per block):
-//   barrier; component e = 0 (zbar_v: the bias sum); barrier (every wave is done with planes 0
-//   and 3); components e = 1, 2, with the late component's writes into planes 0 and 3 between
-//   their MFMAs; barrier; the late component.
-// Adds sum_p zbar_v' of row 16 w + m (all lane groups) to g_bias. The products accumulate in the
-// component order v, L, J0, J1 and point order of each, as two passes of (v, L), (J0, J1) did.
-__device__ __forceinline__ void staged_dw(const StageBases& sb, const f4 (&xl)[4], const f4 (&yl)[4],
-                                          f4 (&dw)[4], float& g_bias) {
-  __syncthreads();  // the early components are written
-  DwOperands ops = dw_read(sb, 0, 0);
-  // The first pass's last step reads the second pass's first operands (planes 1 and 4 were
-  // complete at the first barrier), so the second pass does not start by waiting for LDS.
-  g_bias += sum_lane_groups(dw_pass<0, 1, true, 1>(sb, ops, dw, NoEmit{}));
-  __syncthreads();  // every wave is done with planes 0 and 3
-  dw_pass<1, 2, false, -1>(sb, ops, dw, [&](int step, int k) {
-    stage_late_write(sb, xl, yl, 4 * step + k);
-    return true;
-  });
-  __syncthreads();  // the late component is written
-  ops = dw_read(sb, 0, 0);
-  dw_pass<0, 1, false, -1>(sb, ops, dw, NoEmit{});
-}
 
 // ---- the interior tiles of backward_kernel: the walk back from each layer's tanh-jet output ----
 //
@@ -1150,128 +1138,265 @@ __device__ __forceinline__ void tanh_jet_adjoint_h_seed(float v, float hj0, floa
   bl = s * bl;
 }
 
-// One hidden layer of the forward re-run, one output block at a time: z = W[16 mb + ., :] h_in
-// + b (the first k-step takes the bias as its C operand), then the block's tanh jet into
-// h_out[mb]. Each accumulator takes its k-steps (ob, j) in order (as in forward_kernel's
-// hidden_product_native); a block's tanh jet (VALU) and the next block's 64 MFMAs are independent,
-// so either can fill the other's latencies. The next block's four A operands (16-byte LDS
-// reads) are issued before this block's MFMAs, so no block waits for LDS. w_rows is this
-// lane's row base (68 m + 4 g). emit(mb, k) may issue LDS writes after k-step k (0..15) of
-// block mb's MFMAs (returning whether it did), behind the next block's reads; after(mb) runs once
-// block mb's output is complete (VALU work of the caller that the next block's MFMAs follow).
-template <typename Emit = NoEmit, typename After = NoAfter>
-__device__ __forceinline__ void forward_layer(const float* s_small, const float* w_rows, int layer,
-                                              int g, const f4 (&hin)[4][4], f4 (&hout)[4][4],
-                                              Emit emit = Emit{}, After after = After{}) {
-  f4 bias[4];
-  load_bias(s_small, layer, g, bias);
-  const float* w = w_rows + layer * kPlane;
-  f4 next[4];
+// A wave of backward_kernel is alone on its SIMD, so its MFMAs and VALU work must alternate in its
+// own instruction stream: an MFMA takes 16 clocks (32 for the 32 x 32 form) of which its issue
+// takes 8.5, and the VALU can work in the rest. The tile is cut into scheduling regions
+// (region_end), each holding the MFMAs of one block and independent VALU work of the block before,
+// and interleave<n, k>() asks for n groups of one MFMA and k VALU instructions in the region.
+__device__ __forceinline__ void region_end() { __builtin_amdgcn_sched_barrier(0); }
+
+template <int kMfmas, int kValu>
+__device__ __forceinline__ void interleave() {
 #pragma unroll
-  for (int ob = 0; ob < 4; ++ob) next[ob] = lds4(w + 16 * ob);
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
-    f4 a[4];
-#pragma unroll
-    for (int ob = 0; ob < 4; ++ob) a[ob] = next[ob];
-    if (mb < 3) {
-#pragma unroll
-      for (int ob = 0; ob < 4; ++ob) next[ob] = lds4(w + 1088 * (mb + 1) + 16 * ob);
-    }
-    lds_mfma_fence();
-    f4 z[4];
-#pragma unroll
-    for (int ob = 0; ob < 4; ++ob) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const f4 cin = (ob | j) ? z[c] : (c == 0 ? bias[mb] : zero4());
-          z[c] = mfma(a[ob][j], hin[ob][c][j], cin);
-        }
-        if (emit(mb, 4 * ob + j)) __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    lds_mfma_fence();  // the next block's reads stay ahead of this block's MFMAs
-    tanh_jet4(z, hout[mb]);
-    after(mb);
+  for (int i = 0; i < kMfmas; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
   }
 }
 
-// A operands of transposed_block for input block ib: W[16 ob + 4 g + j][16 ib + m] for the 16
-// k-steps (ob, j), 4-byte LDS reads from this lane's column base w (272 g + m) in the layer's
-// pitch-68 plane.
-__device__ __forceinline__ void transposed_operands(const float* w, int ib, float (&a)[16]) {
+// Step j (0..11) of a block's product: one product of the four components, in block_product's
+// order (half 0's small products, half 1's, then hi hi of both).
+__device__ __forceinline__ void product_step(int j, const WeightOperand& w, const JetOperand& h, f4 (&z)[4]) {
+  const int t = j < 5 ? 0 : j < 10 ? 1 : j - 10, k = j < 5 ? j : j < 10 ? j - 5 : kProducts - 1;
 #pragma unroll
-  for (int step = 0; step < 16; ++step) a[step] = w[1088 * (step >> 2) + kWRow * (step & 3) + 16 * ib];
+  for (int c = 0; c < 4; ++c) z[c] = mfma_bf16(w.part[t][part_a(k)], h.part[t][c][part_b(k)], z[c]);
 }
 
-// hb[c] = sum_o W[o][16 ib + .] zb[o][c][.] for one input block ib: 64 MFMAs over the k-steps
-// (ob, j) in order, from the operands a of
-// transposed_operands.
-__device__ __forceinline__ void transposed_block(const float (&a)[16], const f4 (&zb)[4][4],
-                                                 f4 (&hb)[4]) {
+// The same for hbar, in the order S0, hi hi 0, S1, hi hi 1: half 0's operands are free after six.
+__device__ __forceinline__ void hbar_step(int j, const WeightOperand& w, const JetOperand& h, f4 (&z)[4]) {
+  const int t = j / kProducts, k = j % kProducts;
 #pragma unroll
-  for (int step = 0; step < 16; ++step) {
+  for (int c = 0; c < 4; ++c) z[c] = mfma_bf16(w.part[t][part_a(k)], h.part[t][c][part_b(k)], z[c]);
+}
+
+// The work on an output block after its product, in twelve stages to run one per step of the next
+// block's: the tanh jet (tanh_jet4) and, with kOperand, the split into the next operand
+// (split_block), whose remainders have a step or two to come out of the matrix cores.
+template <bool kOperand>
+struct BlockWork {
+  f4 z[4], v, s, q;
+  u2 part[4][kParts];
+  __device__ __forceinline__ void stage(int j, u2 minus_one, f4 (&out)[4]) {
+    if (j == 0) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v[r] = __builtin_amdgcn_exp2f(z[0][r]);
+        q[r] = __builtin_fmaf(z[1][r], z[1][r], z[2][r] * z[2][r]);
+      }
+    } else if (j == 1) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = __builtin_amdgcn_rcpf(v[r] + 1.0f);
+    } else if (j == 2) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        s[r] = __builtin_fmaf(-v[r], v[r], v[r]);
+        out[0][r] = __builtin_fmaf(v[r], 0.5f * kC, -0.25f * kC);
+      }
+    } else if (j == 3) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        out[1][r] = s[r] * z[1][r];
+        out[2][r] = s[r] * z[2][r];
+      }
+    } else if (j == 4) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) out[3][r] = s[r] * __builtin_fmaf(out[0][r], q[r], z[3][r]);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) z[c] = out[c];
+    } else if (kOperand && (j == 5 || j == 8 || j == 11)) {
+      const int p = (j - 5) / 3;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) part[c][p] = u2{bf16_pair(z[c][0], z[c][1]), bf16_pair(z[c][2], z[c][3])};
+    } else if (kOperand && (j == 6 || j == 9)) {
+      const int p = (j - 6) / 3;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) z[c] = remainder_mfma(minus_one, part[c][p], z[c]);
+    }
+  }
+  __device__ __forceinline__ void put(JetOperand& h, int mb) const {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      hb[c] = mfma(a[step], zb[step >> 2][c][step & 3], step ? hb[c] : zero4());
+#pragma unroll
+      for (int p = 0; p < kParts; ++p) {
+        h.part[mb >> 1][c][p][2 * (mb & 1)] = part[c][p][0];
+        h.part[mb >> 1][c][p][2 * (mb & 1) + 1] = part[c][p][1];
+      }
+    }
+  }
+};
+
+// One hidden layer of the forward re-run (forward_kernel's chains): h_out in registers and, with
+// kOperand, as the next product's operand. Each block's work runs between the MFMAs of the next
+// block, block 3's between the next layer's first ones: before(j), j = 0..4, does the previous
+// layer's, and `work` leaves this layer's block 3. w holds block 0's operands on entry and those of
+// `w_after` on exit.
+template <bool kOperand, typename Before>
+__device__ __forceinline__ void forward_layer(const float* s_small, const u4* w_layer, const u4* w_after,
+                                              u2 minus_one, int layer, int g, const JetOperand& in,
+                                              f4 (&hout)[4][4], JetOperand& next, WeightOperand& w,
+                                              BlockWork<kOperand>& work, Before before) {
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb) {
+    const WeightOperand cur = w;
+    f4 z[4];
+    z[0] = lds4(s_small + kSmallBh + layer * kHidden + 16 * mb + 4 * g);
+#pragma unroll
+    for (int c = 1; c < 4; ++c) z[c] = zero4();
+    w = lds_weights(mb < 3 ? w_layer : w_after, (mb + 1) & 3);
+    region_end();
+#pragma unroll
+    for (int j = 0; j < 12; ++j) {
+      product_step(j, cur, in, z);
+      if (mb == 0 && j < 5) before(j);
+      if (mb > 0) work.stage(j, minus_one, hout[mb - 1]);
+      interleave<4, 2>();
+      region_end();
+    }
+    if (mb > 0 && kOperand) {
+      work.put(next, mb - 1);
+      park_block(hout[mb - 1]);
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) work.z[c] = z[c];
+  }
+}
+
+// dW staging of a 64-point tile: one jet component of zbar and of h_prev, each wave's 16 points
+// as a set of entries (see DwOperand): 24 KB each.
+constexpr int kSetU4 = 2 * kParts * kWave;
+struct DwStage {
+  u4 z[kBwdWaves][kSetU4];
+  u4 h[kBwdWaves][kSetU4];
+};
+
+// One lane's pointers into the staging: its entries of its wave's sets, and its wave's operands
+// (half w >> 1 of zbar, half w & 1 of h_prev) in wave 0's set.
+struct StagePointers {
+  u4 *wz, *wh;
+  DwPointers ra, rb;
+};
+
+// The parts of half t of one component of a layer's output: blocks 2 t and 2 t + 1 (VALU only: it
+// runs between the 32 x 32 MFMAs, which leave the VALU 24 of their 32 clocks).
+__device__ __forceinline__ void split_half(const f4 (&h)[4][4], int c, int t, u4 (&part)[kParts]) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    u2 p[kParts];
+    split4(h[2 * t + i][c], p);
+#pragma unroll
+    for (int s = 0; s < kParts; ++s) {
+      part[s][2 * i] = p[s][0];
+      part[s][2 * i + 1] = p[s][1];
     }
   }
 }
 
-// The adjoint through one hidden layer's weights and the tanh jet below it, one input block at
-// a time: hbar = W^T zbar for block ib, then the tanh-jet adjoint of that block of the layer
-// below, from its output hp, which replaces hp[ib] by the layer below's zbar. Only one block of
-// hbar is live at a time. after(ib) runs once block ib's adjoint is done (VALU work of the caller
-// for that block); emit(ib, step) may issue LDS writes of block ib after k-step `step` of block
-// ib + 1's MFMAs (returning whether it did), behind block ib + 2's operand reads, and block 3's
-// writes follow its adjoint.
-template <typename After, typename Emit>
-__device__ __forceinline__ void adjoint_through(const float* w, const f4 (&zb)[4][4],
-                                                f4 (&hp)[4][4], After after, Emit emit) {
-  float next[16];
-  transposed_operands(w, 0, next);
+// One hidden layer of the walk back: dW += zbar h^T, and hbar = W^T zbar given to
+// adjoint(ib, r, hb) per input block and register. The two are interleaved, one component of dW
+// with one block of hbar, so that hbar's MFMAs cover the staging's writes, barriers and first
+// reads: stage component c; block c's products, with the adjoint of block c - 1 between them and
+// the barrier and dW's first reads halfway; dW over the four waves' points, each set's operands
+// read behind the previous set's MFMAs, with the next component's split between them; the second
+// barrier (every wave has read component c) before the last set's MFMAs. w holds block 0's operands
+// on entry and w_after's on exit.
+template <typename Adjoint>
+__device__ __forceinline__ void backward_layer(const u4* w_t, const u4* w_after, const StagePointers& sp,
+                                               const JetOperand& zb, const f4 (&h)[4][4], float sign, f16& dw,
+                                               WeightOperand& w, Adjoint adjoint) {
+  f16 sum = zero16();
+  u4 part[2][kParts];
+  split_half(h, 0, 0, part[0]);
+  split_half(h, 0, 1, part[1]);
+  f4 done[4];  // the previous block's hbar
 #pragma unroll
-  for (int ib = 0; ib < 4; ++ib) {
-    float a[16];
+  for (int c = 0; c < 4; ++c) {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) a[k] = next[k];
-    if (ib < 3) transposed_operands(w, ib + 1, next);
-    lds_mfma_fence();
-    f4 hb[4];
+    for (int t = 0; t < 2; ++t) {
 #pragma unroll
-    for (int step = 0; step < 16; ++step) {
+      for (int s = 0; s < kParts; ++s) {
+        sp.wz[(t * kParts + s) * kWave] = zb.part[t][c][s];
+        sp.wh[(t * kParts + s) * kWave] = part[t][s];
+      }
+    }
+    region_end();
+    f4 hb[4] = {zero4(), zero4(), zero4(), zero4()};
+    DwOperand a, b;
+    u4 next0[kParts];  // half 0 of the next block's weights
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (i == 2) {
+        __syncthreads();  // component c is staged
+        a = lds_dw_operand(sp.ra, 0);
+        b = lds_dw_operand(sp.rb, 0);
+        lds_transposed_half(c < 3 ? w_t : w_after, (c + 1) & 3, 0, next0);
+        region_end();
+      }
+#pragma unroll
+      for (int j = 0; j < 3; ++j) hbar_step(3 * i + j, w, zb, hb);
+      if (c > 0) {
+        adjoint(c - 1, i, done);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) dw[4 * i + r] = __builtin_fmaf(sign, sum[4 * i + r], dw[4 * i + r]);
+      }
+      interleave<12, 2>();
+      region_end();
+    }
+    sum = zero16();
+#pragma unroll
+    for (int set = 0; set < kBwdWaves; ++set) {
+      const DwOperand ca = a, cb = b;
+      if (set + 1 < kBwdWaves) {
+        a = lds_dw_operand(sp.ra, (set + 1) * kSetU4);
+        b = lds_dw_operand(sp.rb, (set + 1) * kSetU4);
+      } else {
+        __syncthreads();  // every wave has read component c
+        lds_transposed_half(c < 3 ? w_t : w_after, (c + 1) & 3, 1, w.part[1]);
+      }
+      region_end();
+      sum = add_products(ca, cb, sum);
+      if (c < 3) {
+        u2 p[kParts];
+        split4(h[set][c + 1], p);
+#pragma unroll
+        for (int s = 0; s < kParts; ++s) {
+          part[set >> 1][s][2 * (set & 1)] = p[s][0];
+          part[set >> 1][s][2 * (set & 1) + 1] = p[s][1];
+        }
+      }
+      interleave<6, 4>();
+      region_end();
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) done[i] = hb[i];
+#pragma unroll
+    for (int s = 0; s < kParts; ++s) w.part[0][s] = next0[s];
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) adjoint(3, i, done);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    float x = __builtin_fmaf(sign, sum[r], dw[r]);
+    park(x);
+    dw[r] = x;
+  }
+}
+
+// All blocks of a layer's adjoint into an operand, 16 independent chains of conversions and
+// remainders (split_block of one block would wait for each of its MFMAs).
+__device__ __forceinline__ void put_all(u2 minus_one, JetOperand& h, f4 (&x)[4][4]) {
+#pragma unroll
+  for (int s = 0; s < kParts; ++s) {
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        hb[c] = mfma(a[step], zb[step >> 2][c][step & 3], step ? hb[c] : zero4());
+        const u2 part = {bf16_pair(x[mb][c][0], x[mb][c][1]), bf16_pair(x[mb][c][2], x[mb][c][3])};
+        h.part[mb >> 1][c][s][2 * (mb & 1)] = part[0];
+        h.part[mb >> 1][c][s][2 * (mb & 1) + 1] = part[1];
+        if (s + 1 < kParts) x[mb][c] = remainder_mfma(minus_one, part, x[mb][c]);
       }
-      if (ib > 0 && emit(ib - 1, step)) __builtin_amdgcn_sched_barrier(0);
     }
-    lds_mfma_fence();
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float bv = hb[0][r], bj0 = hb[1][r], bj1 = hb[2][r], bl = hb[3][r];
-      tanh_jet_adjoint_h(hp[ib][0][r], hp[ib][1][r], hp[ib][2][r], hp[ib][3][r], bv, bj0, bj1, bl);
-      hp[ib][0][r] = bv;
-      hp[ib][1][r] = bj0;
-      hp[ib][2][r] = bj1;
-      hp[ib][3][r] = bl;
-    }
-    after(ib);
   }
-#pragma unroll
-  for (int step = 0; step < 16; ++step) emit(3, step);
-}
-
-// Staging writes of a block's early components spread over the 16 k-steps of a block of MFMAs:
-// writes 2 step and 2 step + 1 of stage_early_write after k-step `step` < 12.
-__device__ __forceinline__ bool emit_early_pair(const StageBases& sb, int mb, const f4 (&x)[4],
-                                                const f4 (&y)[4], int step) {
-  if (step >= 12) return false;
-  stage_early_write(sb, mb, x, y, 2 * step);
-  stage_early_write(sb, mb, x, y, 2 * step + 1);
-  return true;
 }
 
 // Seed of the fused Poisson training step (kLoss). The loss is the PINN loss
@@ -1282,7 +1407,7 @@ __device__ __forceinline__ bool emit_early_pair(const StageBases& sb, int mb, co
 //   interior points: grad_u = 0, grad_lap = fl(1 / B) (2 r) with r = lap - f;
 //   boundary points: grad_u = fl(w / B_b) (2 u), grad_lap = 0.
 // Tiles [0, interior_tiles) hold interior points and the rest boundary points, 16 per tile in
-// both gradient kernels (boundary_tile, backward_split_kernel). sum r^2 and
+// both gradient kernels (split_tile<1>). sum r^2 and
 // sum u^2 go into columns kLossColumn and kLossColumn + 1 of the slot's partial row. `step` is
 // the Adam step counter, advanced here (one lane of workgroup 0) so that the update kernel that
 // follows reads a settled value.
@@ -1298,191 +1423,6 @@ struct LossSeed {
 
 constexpr int kLossColumn = kParameterCount;  // partial-row columns of sum r^2, sum u_b^2
 static_assert(kLossColumn + 1 < kRowStride, "the loss columns must fit in a partial row");
-
-// Per-slot gradient sums of one wave (see backward_kernel).
-struct WaveSums {
-  f4 dw[3][4];         // hidden dW, rows 16 w + ., in MFMA accumulator layout
-  float bh[3];         // hidden bias sums of c^-1 zbar_v (row 16 w + m, see dw_pass)
-  float w0x, w0y, b0;  // layer-0 sums, lane = owned neuron
-  float wout, bout;    // output-layer sums
-  float loss, bloss;   // kLoss: sums of r^2 and u_b^2
-};
-
-// A boundary tile of the fused step. Boundary points enter the loss through u alone
-// (grad_lap = 0), so the output seed is (vbar', Jbar', Lbar') = (4 gu w_out / c, 0, 0), and the
-// tanh-jet adjoint maps (vbar', 0, 0, 0) to (s' vbar', 0, 0, 0): every adjoint component but
-// the value one is exactly zero at every layer. The weight-gradient terms reduce to
-// zbar_v h_v^T, and the forward's J and L components feed nothing. A boundary tile therefore
-// runs the value channel only; the terms it skips are exact zeros.
-//
-// A boundary tile holds 16 points, shared by the workgroup's 4 waves: wave w owns rows
-// 16 w .. 16 w + 15 of every layer, so the forward, dW and W^T zbar products of a layer are 16
-// MFMAs each per wave (a 16-point value-channel tile on one wave would be 64 each). Layer
-// outputs and adjoints go to the other waves lane to lane through LDS (the register layout of
-// forward_split_kernel: register r of block ob holds row 16 ob + 4 g + r at point m), for the
-// next product's B operand. dW contracts over the tile's points, which sit on the lane axis, so
-// each layer's h_v and the wave's zbar_v are also stored transposed: row R, point 4 s + g at
-// column 4 g + s of a 20-float row, so one 16-byte read gives a lane the points of its 4 k-steps.
-// Scratch inside the dW staging buffer (floats):
-constexpr int kBndPitch = 20;                                   // transposed row, 16 points + pad
-constexpr int kBndExchange = 0;                                 // [2][4 waves][64 lanes] f4
-constexpr int kBndH = kBndExchange + 2 * kBwdWaves * kWave * 4;  // [3 layers][64 rows][pitch]
-constexpr int kBndZ = kBndH + 3 * kHidden * kBndPitch;          // [2][4 waves][16 rows][pitch]
-static_assert(kBndZ + 2 * kBwdWaves * 16 * kBndPitch <= kStagePlanes * kPlane,
-              "the boundary tile's scratch must fit the dW staging buffer");
-
-// Store this lane's 4 rows row0 + 4 g + r (value at point m) into a transposed buffer.
-__device__ __forceinline__ void store_point_columns(float* t, int row0, int g, int m, f4 x) {
-  const int col = 4 * (m & 3) + (m >> 2);
-#pragma unroll
-  for (int r = 0; r < 4; ++r) t[(row0 + 4 * g + r) * kBndPitch + col] = x[r];
-}
-
-// Per-neuron point sums of this wave's rows: t[r] is the total of row 16 w + 4 g + r (the same
-// in all 16 lanes of row g). Lane (m, g) owns neuron owned_neuron(m, g) =
-// 16 (m >> 2) + 4 g + (m & 3) in the slot sums, so it takes t[m & 3] when m >> 2 == w and adds
-// nothing otherwise (the other waves own those neurons' rows).
-__device__ __forceinline__ float own_row_total(const f4 t, int m, int w) {
-  const float lo = (m & 1) ? t[1] : t[0];
-  const float hi = (m & 1) ? t[3] : t[2];
-  const float v = (m & 2) ? hi : lo;
-  return (m >> 2) == w ? v : 0.0f;
-}
-
-__device__ __forceinline__ f4 row_totals(const f4 x) {
-  f4 t;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) t[r] = sum_row16(x[r]);
-  return t;
-}
-
-__device__ __forceinline__ void boundary_tile(const float* s_w, const float* s_small,
-                                              float* s_stage, int rows_off, int cols_off, int w,
-                                              int g, int m, float x0, float x1, bool active,
-                                              float boundary_scale, WaveSums& acc) {
-  __syncthreads();  // the previous tile's readers of the staging buffer are done
-  f4* xch = reinterpret_cast<f4*>(s_stage + kBndExchange);
-  float* ht = s_stage + kBndH;
-  float* zt = s_stage + kBndZ;
-  const int lane = 16 * g + m;
-  int phase = 0;  // alternates the exchange and zbar buffers
-
-  // ---- forward, value channel: layer 0 whole, then this wave's rows of hidden layers 1..3 ----
-  f4 h[4];      // v' of all 64 rows of the current layer output
-  f4 s_own[3];  // s' of this wave's rows of layer 0 and hidden layers 1, 2
-  f4 v_top, s_top;  // hidden layer 3, this wave's rows
-#pragma unroll
-  for (int ob = 0; ob < 4; ++ob) {
-    const Layer0Weights w0 = layer0_weights(s_small, ob, g);
-    f4 zv, unused;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) zv[r] = layer0_zv(w0, r, x0, x1);
-    tanh_scaled4(zv, h[ob], unused);
-  }
-  {
-    // this wave's block again (h[w] would need a dynamic register index)
-    const Layer0Weights w0 = layer0_weights(s_small, w, g);
-    f4 zv, v;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) zv[r] = layer0_zv(w0, r, x0, x1);
-    tanh_scaled4(zv, v, s_own[0]);
-    store_point_columns(ht, 16 * w, g, m, v);
-  }
-#pragma unroll
-  for (int l = 0; l < 3; ++l) {
-    const f4 b = lds4(s_small + kSmallBh + l * kHidden + 16 * w + 4 * g);
-    const float* wrow = s_w + l * kPlane + opaque(rows_off) + 1088 * w;  // W[16 w + m][.]
-    f4 z;
-#pragma unroll
-    for (int ob = 0; ob < 4; ++ob) {
-      const f4 a = lds4(wrow + 16 * ob);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) z = mfma(a[j], h[ob][j], (ob | j) ? z : b);
-    }
-    f4 v, sl;
-    tanh_scaled4(z, v, sl);
-    if (l < 2) {
-      s_own[l + 1] = sl;
-      store_point_columns(ht + (l + 1) * kHidden * kBndPitch, 16 * w, g, m, v);
-    } else {
-      v_top = v;
-      s_top = sl;
-    }
-    xch[(phase * kBwdWaves + w) * kWave + lane] = v;
-    __syncthreads();
-#pragma unroll
-    for (int ob = 0; ob < 4; ++ob) h[ob] = xch[(phase * kBwdWaves + ob) * kWave + lane];
-    phase ^= 1;
-  }
-
-  // ---- u = w_out . v + b_out over all 64 rows, the seed gu = fl(w / B_b) (2 u) ----
-  float out = 0.0f;
-#pragma unroll
-  for (int ob = 0; ob < 4; ++ob) {
-    const f4 wo = lds4(s_small + kSmallWoutV + 16 * ob + 4 * g);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) out = __builtin_fmaf(wo[r], h[ob][r], out);
-  }
-  out = sum_lane_groups(out);
-  const float u = active ? out + s_small[kSmallBout] : 0.0f;
-  const float gu = boundary_scale * (2.0f * u);
-  if (w == 0) {  // the 4 waves share the tile's points: one of them adds the point sums
-    acc.bloss += sum_row16(u * u);
-    acc.bout += sum_row16(gu);
-  }
-  const float gu_c = gu * (4.0f / kC);
-  acc.wout += own_row_total(row_totals(gu_c * v_top), m, w);
-  const f4 wv = lds4(s_small + kSmallWoutV + 16 * w + 4 * g);
-  f4 zb = s_top * (gu * wv);  // hidden layer 3's zbar_v' = s' vbar', this wave's rows
-
-  // ---- hidden layers 3, 2, 1: dW, the bias sum, hbar = W^T zbar, the next zbar ----
-#pragma unroll
-  for (int l = 2; l >= 0; --l) {
-    float* ztw = zt + (phase * kBwdWaves + w) * 16 * kBndPitch;
-    store_point_columns(ztw, 0, g, m, zb);
-    xch[(phase * kBwdWaves + w) * kWave + lane] = zb;
-    __syncthreads();
-    {
-      // dW[16 w + ., 16 nb + .] += sum over the 16 points of zbar h_prev^T: A = zbar of row
-      // 16 w + m, B = h_prev of row 16 nb + m, k-step s = points 4 s + g.
-      const f4 a = lds4(ztw + m * kBndPitch + 4 * g);
-      const float* hrow = ht + l * kHidden * kBndPitch + m * kBndPitch + 4 * g;
-      f4 bt[4];
-#pragma unroll
-      for (int nb = 0; nb < 4; ++nb) bt[nb] = lds4(hrow + 16 * nb * kBndPitch);
-      float bsum = 0.0f;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        bsum += a[k];
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) acc.dw[l][nb] = mfma(a[k], bt[nb][k], acc.dw[l][nb]);
-      }
-      acc.bh[l] += sum_lane_groups(bsum);
-    }
-    f4 hb;
-    {
-      // hbar of this wave's rows of the layer below: sum over the 64 rows o of
-      // W[o][16 w + m] zbar[o].
-      const float* wt = s_w + l * kPlane + opaque(cols_off) + 16 * w;
-#pragma unroll
-      for (int ob = 0; ob < 4; ++ob) {
-        const f4 zo = xch[(phase * kBwdWaves + ob) * kWave + lane];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          hb = mfma(wt[1088 * ob + kWRow * j], zo[j], (ob | j) ? hb : zero4());
-        }
-      }
-    }
-    phase ^= 1;
-    zb = s_own[l] * hb;  // zbar_v' of the layer below (l = 0: layer 0's bv)
-  }
-
-  // ---- layer 0: dW0[o][d] = 2 sum_p bv (c x_d / 2) (the row takes the 2), db0 = c sum_p bv ----
-  const float cx0 = kHalfC * x0, cx1 = kHalfC * x1;
-  acc.w0x += own_row_total(row_totals(zb * cx0), m, w);
-  acc.w0y += own_row_total(row_totals(zb * cx1), m, w);
-  acc.b0 += own_row_total(row_totals(zb), m, w);
-}
 
 // Per-point inputs of one gradient-kernel tile for this lane: coordinates and, for interior
 // points, the upstream gradients (gu, gl) or, with kLoss, the source f (in a). Boundary tiles
@@ -1532,119 +1472,176 @@ __device__ __forceinline__ void deliver(TileInputs& in) {
 }
 
 constexpr int kSplitBwdMaxTiles = 768;  // backward_split_kernel up to 768 16-point tiles
-constexpr int kTPlane = 64 * kWRow;     // floats of one transposed 64-row layer (h)
-constexpr int kTWave = 16 * kWRow;      // floats of one wave's transposed zbar
 
-// Store this lane's 4 rows (rows0 + 4 g + r) x 4 components at point m into a transposed
-// buffer t[row][68]: component c of point p = 4 s + g' at t[row * 68 + 16 c + 4 g' + s].
-__device__ __forceinline__ void store_transposed(float* t, int rows0, int g, int m,
-                                                 const f4 (&x)[4]) {
-  const int col = 4 * (m & 3) + (m >> 2);
+// Scratch of one 16-point tile whose rows are split over the workgroup's 4 waves: the layer
+// outputs h1, h2 and the adjoint as operands of all 64 rows (Exchange, 24 KB each; dW reads
+// them transposed), and the partial coordinate gradients.
+struct SplitScratch {
+  Exchange h1, h2, z;
+  float gx[kSplitWaves][2][kTile];
+};
+
+// Per-lane point sums of split_tile, of row 16 w + 4 g + (m & 3) (bh, w0x, w0y, b0, wout), or the
+// same in every lane of a wave (bout, loss, bloss).
+struct SplitSums {
+  float bh[3], w0x, w0y, b0, wout, bout, loss, bloss;
+};
+
+// This lane's share of the point sums of rows 16 w + 4 g + r: sum over the 16 lanes of row g of
+// x[r], r = m & 3.
+__device__ __forceinline__ float row_total(const f4 x, int m) {
+  f4 t;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
+  for (int r = 0; r < 4; ++r) t[r] = sum_row16(x[r]);
+  const float lo = (m & 1) ? t[1] : t[0];
+  const float hi = (m & 1) ? t[3] : t[2];
+  return (m & 2) ? hi : lo;
+}
+
+// The operand entries of the components in use: JetOperand's and Exchange's first C.
+template <int C>
+__device__ __forceinline__ void get_components(const Exchange& x, int entry, JetOperand& h) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) t[(rows0 + 4 * g + r) * kWRow + 16 * c + col] = x[c][r];
+  for (int t = 0; t < 2; ++t) {
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+#pragma unroll
+      for (int s = 0; s < kParts; ++s) h.part[t][c][s] = x.part[t][c][s][entry];
+    }
   }
 }
 
-// Scratch of one 16-point tile whose rows are split over the workgroup's 4 waves.
-struct SplitScratch {
-  float* ht;                       // [3][kTPlane]: h of layers 0..2, transposed
-  f4 (*x)[kSplitWaves][4][kWave];  // [2 buffers]: lane-major exchange
-  float (*zt)[kTWave];             // [4 waves]: this wave's zbar, transposed
-  float (*gx)[2][kTile];           // [4 waves]: partial coordinate gradients
-};
-constexpr int kSplitScratchFloats = 3 * kTPlane + 2 * kSplitWaves * 4 * kWave * 4 +
-                                    kSplitWaves * kTWave + kSplitWaves * 2 * kTile;
-
-// Per-lane point sums of split_tile: bias sums go to the caller's array (row 16 w + m, as in
-// dw_pass); these are of row 16 w + 4 g + (m & 3) (w0x, w0y, b0, wout), or the same in every
-// lane of a wave (bout, loss, bloss).
-struct SplitSums {
-  float w0x, w0y, b0, wout, bout, loss, bloss;
-};
-
-// One 16-point tile, all 4 waves: wave w owns rows 16 w .. 16 w + 15 of every layer (64 MFMAs
-// per layer for the forward re-run, dW and W^T zbar). Layer outputs and adjoints go to the
-// other waves lane to lane through LDS (`sc.x`, the register layout of forward_split_kernel),
-// and each layer's h (all 64 rows) and the wave's zbar are also stored transposed,
-// [row][c][4 g + s] for point 4 s + g at pitch 68, so dW contracts over the tile's points with
-// 16-byte reads. dW and the bias sums accumulate into `dw` / `bias` (the layout of
-// backward_kernel's); grad_coordinates of interior points are written here. `rows_off` and
-// `cols_off` are this wave's lane offsets W[16 w + m][.] and W[.][16 w + m]; t_read = 68 m + 4 g.
-template <bool kLoss>
-__device__ __forceinline__ void split_tile(const float* s_w, const float* s_small,
-                                           const SplitScratch& sc, int& phase, int w, int g, int m,
-                                           int rows_off, int cols_off, int t_read, float x0,
-                                           float x1, float gu, float gl, float f, bool active,
-                                           bool on_boundary, int64_t point,
+// One 16-point tile, all 4 waves: wave w owns rows 16 w .. 16 w + 15 of every layer for the
+// forward re-run and W^T zbar (48 MFMAs per layer each with 4 components) and the 32 x 32 block
+// (w >> 1, w & 1) of every dW. Layer outputs and adjoints go to the other waves through LDS
+// (Exchange), where dW also reads them, transposed, so dW contracts over the tile's points one
+// component at a time. dW accumulates into `dw` (the layout of backward_kernel's);
+// grad_coordinates of interior points are written here. w_lane and w_t are this lane's entries of
+// the staged weights (forward and transposed).
+//
+// kComponents = 1: a boundary tile of the fused step. Boundary points enter the loss through u
+// alone (grad_lap = 0), so the output seed is (vbar', Jbar', Lbar') = (4 gu w_out / c, 0, 0), and
+// the tanh-jet adjoint maps (vbar', 0, 0, 0) to (s' vbar', 0, 0, 0): every adjoint component but
+// the value one is exactly zero at every layer. The weight-gradient terms reduce to
+// zbar_v h_v^T, and the forward's J and L components feed nothing. A boundary tile therefore
+// runs the value channel only; the terms it skips are exact zeros.
+template <int kComponents, bool kLoss>
+__device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, const float* s_small,
+                                           SplitScratch& sc, u2 minus_one, int w, int g, int m,
+                                           float x0, float x1, float gu, float gl, float f,
+                                           bool active, float sign, int64_t point,
                                            float* __restrict__ grad_coordinates,
-                                           const LossSeed& seed, f4 (&dw)[3][4], float (&bias)[3],
-                                           SplitSums& sums) {
+                                           const LossSeed& seed, f16 (&dw)[3], SplitSums& sums) {
+  constexpr int C = kComponents;
+  constexpr bool kBoundary = C == 1;
   const int lane = 16 * g + m;
-  // ---- forward re-run: all 64 rows of layer 0, then this wave's rows of layers 1..3 ----
-  f4 h[4][4];
-  layer0_forward(s_small, g, x0, x1, h);
-  {
-    f4 own[4];  // this wave's block again (h[w] would need a dynamic register index)
-    layer0_block(s_small, w, g, x0, x1, own);
-    store_transposed(sc.ht, 16 * w, g, m, own);
-  }
-  f4 z[3][4];  // this wave's pre-activations of hidden layers 1..3
-  f4 mine[4];  // this wave's rows of the current layer output
+  const int entry = operand_entry(m, g);
+  auto tanh_rows = [&](const f4 (&z)[4], f4 (&out)[4]) {
+    if (kBoundary) {
+      f4 unused;
+      tanh_scaled4(z[0], out[0], unused);
+    } else {
+      tanh_jet4(z, out);
+    }
+  };
+  auto split_rows = [&](const f4 (&x)[4], u2 (&part)[4][kParts]) {
+    f4 rest[4];
 #pragma unroll
-  for (int layer = 0; layer < 3; ++layer) {
-    const f4 b = lds4(s_small + kSmallBh + layer * kHidden + 16 * w + 4 * g);
-    const float* wrow = s_w + layer * kPlane + opaque(rows_off);
+    for (int c = 0; c < C; ++c) rest[c] = x[c];
 #pragma unroll
-    for (int ob = 0; ob < 4; ++ob) {
-      const f4 a = lds4(wrow + 16 * ob);
+    for (int s = 0; s < kParts; ++s) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const f4 cin = (ob | j) ? z[layer][c] : (c == 0 ? b : zero4());
-          z[layer][c] = mfma(a[j], h[ob][c][j], cin);
-        }
+      for (int c = 0; c < C; ++c) {
+        part[c][s] = u2{bf16_pair(rest[c][0], rest[c][1]), bf16_pair(rest[c][2], rest[c][3])};
+        if (s + 1 < kParts) rest[c] = remainder_mfma(minus_one, part[c][s], rest[c]);
       }
     }
-    tanh_jet4(z[layer], mine);
-    f4 (*xb)[4][kWave] = sc.x[phase];
-    phase ^= 1;
+  };
+  auto put_rows = [&](Exchange& x, const f4 (&mine)[4]) {
+    u2 part[4][kParts];
+    split_rows(mine, part);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) xb[w][c][lane] = mine[c];
-    if (layer < 2) store_transposed(sc.ht + (layer + 1) * kTPlane, 16 * w, g, m, mine);
-    __syncthreads();
+    for (int c = 0; c < C; ++c) {
 #pragma unroll
-    for (int ob = 0; ob < 4; ++ob) {
+      for (int s = 0; s < kParts; ++s) {
+        reinterpret_cast<u2*>(&x.part[w >> 1][c][s][entry])[w & 1] = part[c][s];
+      }
+    }
+  };
+  auto product = [&](const WeightOperand& a, const JetOperand& b, const f4 start, f4 (&z)[4]) {
+    z[0] = start;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) h[ob][c] = xb[ob][c][lane];  // this wave's block included
+    for (int c = 1; c < C; ++c) z[c] = zero4();
+#pragma unroll
+    for (int i = 0; i < 2 * kProducts; ++i) {  // the order of block_product
+      const int t = i < 2 * (kProducts - 1) ? i / (kProducts - 1) : i - 2 * (kProducts - 1);
+      const int k = i < 2 * (kProducts - 1) ? i % (kProducts - 1) : kProducts - 1;
+#pragma unroll
+      for (int c = 0; c < C; ++c) z[c] = mfma_bf16(a.part[t][part_a(k)], b.part[t][c][part_b(k)], z[c]);
+    }
+  };
+
+  // ---- forward re-run: all 64 rows of layer 0, then this wave's rows of layers 1..3 ----
+  JetOperand op;
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb) {
+    f4 x[4];
+    layer0_block(s_small, mb, g, x0, x1, x);
+    u2 part[4][kParts];
+    split_rows(x, part);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+#pragma unroll
+      for (int s = 0; s < kParts; ++s) {
+        op.part[mb >> 1][c][s][2 * (mb & 1)] = part[c][s][0];
+        op.part[mb >> 1][c][s][2 * (mb & 1) + 1] = part[c][s][1];
+      }
+    }
+  }
+  f4 h[3][4];  // this wave's rows of the hidden layers' outputs
+#pragma unroll
+  for (int layer = 0; layer < 3; ++layer) {
+    const f4 bias = lds4(s_small + kSmallBh + layer * kHidden + 16 * w + 4 * g);
+    f4 z[4];
+    product(lds_weights(w_lane + layer * kLayerU4, w), op, bias, z);
+    tanh_rows(z, h[layer]);
+    if (layer < 2) {
+      Exchange& x = layer ? sc.h2 : sc.h1;
+      put_rows(x, h[layer]);
+      __syncthreads();
+      get_components<C>(x, entry, op);
     }
   }
 
   if (kLoss) {
-    // u (boundary) or lap (interior) over all 64 rows, in backward_kernel's order.
-    float out = 0.0f;
+    // u (boundary) or lap (interior) over all 64 rows, in forward_kernel's order.
+    float* terms = reinterpret_cast<float*>(&sc.z);
+    {
+      const f4 wo = lds4(s_small + (kBoundary ? kSmallWoutV : kSmallWoutL) + 16 * w + 4 * g);
+      float t = 0.0f;
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb) {
-      const f4 wo = lds4(s_small + (on_boundary ? kSmallWoutV : kSmallWoutL) + 16 * mb + 4 * g);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        out = __builtin_fmaf(wo[r], on_boundary ? h[mb][0][r] : h[mb][3][r], out);
-      }
+      for (int r = 0; r < 4; ++r) t = __builtin_fmaf(wo[r], h[2][kBoundary ? 0 : 3][r], t);
+      terms[w * kWave + lane] = t;
     }
+    __syncthreads();
+    float out = terms[lane];
+#pragma unroll
+    for (int mb = 1; mb < 4; ++mb) out += terms[mb * kWave + lane];
     out = sum_lane_groups(out);
-    // u (boundary) or the residual lap - f (interior); both sums are updated with a select, so
-    // that `sums` stays in registers (a branch per field made the compiler address it).
-    const float e = active ? (on_boundary ? out + s_small[kSmallBout] : out - f) : 0.0f;
-    if (on_boundary) {
-      gu = seed.boundary_scale * (2.0f * e);
-    } else {
-      gl = seed.inv_batch * (2.0f * e);
-    }
+    __syncthreads();  // sc.z is free again
+    // u (boundary) or the residual lap - f (interior).
+    const float e = active ? (kBoundary ? out + s_small[kSmallBout] : out - f) : 0.0f;
     const float sq = sum_row16(e * e);
-    sums.bloss += on_boundary ? sq : 0.0f;
-    sums.loss += on_boundary ? 0.0f : sq;
+    if (kBoundary) {
+      gu = sign * (seed.boundary_scale * (2.0f * e));
+      sums.bloss += sq;
+    } else {
+      gl = sign * (seed.inv_batch * (2.0f * e));
+      sums.loss += sq;
+    }
+  } else {
+    gu *= sign;
+    gl *= sign;
   }
 
   // ---- output layer: this wave's rows of the seed and of dw_out ----
@@ -1654,16 +1651,19 @@ __device__ __forceinline__ void split_tile(const float* s_w, const float* s_smal
     const float gl_l = gl * (4.0f / kLambda);
     const f4 wv = lds4(s_small + kSmallWoutV + 16 * w + 4 * g);
     const f4 wl = lds4(s_small + kSmallWoutL + 16 * w + 4 * g);
+    f4 terms;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const float total = sum_row16(__builtin_fmaf(gu_c, mine[0][r], gl_l * mine[3][r]));
-      sums.wout = (m & 3) == r ? sums.wout + total : sums.wout;
+      terms[r] = kBoundary ? gu_c * h[2][0][r] : __builtin_fmaf(gu_c, h[2][0][r], gl_l * h[2][3][r]);
       hb[0][r] = gu * wv[r];
-      hb[1][r] = 0.0f;
-      hb[2][r] = 0.0f;
-      hb[3][r] = gl * wl[r];
+      if (!kBoundary) {
+        hb[1][r] = 0.0f;
+        hb[2][r] = 0.0f;
+        hb[3][r] = gl * wl[r];
+      }
     }
-    sums.bout += sum_row16(gu);
+    sums.wout += sign * row_total(terms, m);
+    sums.bout += sign * sum_row16(gu);
   }
 
   // ---- hidden layers 3, 2, 1 ----
@@ -1671,64 +1671,59 @@ __device__ __forceinline__ void split_tile(const float* s_w, const float* s_smal
   for (int layer = 2; layer >= 0; --layer) {
     // zbar of this wave's rows (tanh-jet adjoint, lane-local)
     f4 zb[4];
-    f4 v4, s4;
-    tanh_scaled4(z[layer][0], v4, s4);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const float v = v4[r], s = s4[r];
-      float bv = hb[0][r], bj0 = hb[1][r], bj1 = hb[2][r], bl = hb[3][r];
-      tanh_jet_adjoint_vs(v, s, z[layer][1][r], z[layer][2][r], z[layer][3][r], bv, bj0, bj1,
-                          bl);
-      zb[0][r] = bv;
-      zb[1][r] = bj0;
-      zb[2][r] = bj1;
-      zb[3][r] = bl;
+      const float v = h[layer][0][r];
+      if (kBoundary) {
+        zb[0][r] = __builtin_fmaf(kHalfKappa * v, v, 0.25f) * hb[0][r];
+      } else {
+        float bv = hb[0][r], bj0 = hb[1][r], bj1 = hb[2][r], bl = hb[3][r];
+        tanh_jet_adjoint_h(v, h[layer][1][r], h[layer][2][r], h[layer][3][r], bv, bj0, bj1, bl);
+        zb[0][r] = bv;
+        zb[1][r] = bj0;
+        zb[2][r] = bj1;
+        zb[3][r] = bl;
+      }
     }
-    f4 (*xb)[4][kWave] = sc.x[phase];
-    phase ^= 1;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) xb[w][c][lane] = zb[c];
-    float* zt = sc.zt[w];
-    store_transposed(zt, 0, g, m, zb);
+    sums.bh[layer] += sign * row_total(zb[0], m);
+    if (layer < 2) __syncthreads();  // every wave has read the layer above's adjoint and h
+    put_rows(sc.z, zb);
+    if (layer == 0) {  // layer 0's output, this wave's rows, in place of h2
+      f4 own[4];
+      layer0_block(s_small, w, g, x0, x1, own);
+      put_rows(sc.h2, own);
+    }
     __syncthreads();
-    // dW[16 w + ., 16 nb + .] += sum over (c, points) of zbar h_prev^T; the A reads of
-    // component 0 also give the bias sum of row 16 w + m.
+    // dW += sum over (c, points) of zbar h_prev^T.
     {
-      const float* ht = sc.ht + layer * kTPlane + opaque(t_read);
-      const float* za = zt + opaque(t_read);
-      float bsum = 0.0f;
+      const Exchange& hx = layer == 1 ? sc.h1 : sc.h2;
+      const DwPointers a = dw_pointers(&sc.z.part[w >> 1][0][0][0], m, g);
+      const DwPointers b = dw_pointers(&hx.part[w & 1][0][0][0], m, g);
+      f16 sum = zero16();
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const f4 a = lds4(za + 16 * c);
-        f4 bt[4];
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) bt[nb] = lds4(ht + 16 * kWRow * nb + 16 * c);
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          if (c == 0) bsum += a[s];
-#pragma unroll
-          for (int nb = 0; nb < 4; ++nb) dw[layer][nb] = mfma(a[s], bt[nb][s], dw[layer][nb]);
-        }
+      for (int c = 0; c < C; ++c) {
+        sum = add_products(lds_dw_operand(a, c * kParts * kWave), lds_dw_operand(b, c * kParts * kWave), sum);
       }
-      bias[layer] += sum_lane_groups(bsum);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dw[layer][r] = __builtin_fmaf(sign, sum[r], dw[layer][r]);
     }
-    // hbar of this wave's rows of the layer below: sum over all 64 rows o of
-    // W[o][16 w + .] zbar[o].
-    {
-      const float* wt = s_w + layer * kPlane + opaque(cols_off);
+    // hbar of this wave's rows of the layer below.
+    get_components<C>(sc.z, entry, op);
+    const u4* wt = w_t + layer * kLayerU4 + (w >> 1) * kParts * kWave;
+    WeightOperand a;
 #pragma unroll
-      for (int ob = 0; ob < 4; ++ob) {
-        f4 zo[4];  // zbar of rows 16 ob .. 16 ob + 15 (this wave's block included)
+    for (int t = 0; t < 2; ++t) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) zo[c] = xb[ob][c][lane];
+      for (int s = 0; s < kParts; ++s) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float a = wt[1088 * ob + kWRow * j];
-#pragma unroll
-          for (int c = 0; c < 4; ++c) hb[c] = mfma(a, zo[c][j], (ob | j) ? hb[c] : zero4());
+        for (int i = 0; i < 2; ++i) {
+          const u2 v = lds_transposed(reinterpret_cast<const u2*>(wt + (2 * t + i) * kBlockU4 + s * kWave) + (w & 1));
+          a.part[t][s][2 * i] = v[0];
+          a.part[t][s][2 * i + 1] = v[1];
         }
       }
     }
+    product(a, op, zero4(), hb);
   }
 
   // ---- layer 0 for this wave's rows: dW0, db0 and this wave's part of grad_x ----
@@ -1736,34 +1731,59 @@ __device__ __forceinline__ void split_tile(const float* s_w, const float* s_smal
     const Layer0Weights w0 = layer0_weights(s_small, w, g);
     const float cx0 = kHalfC * x0, cx1 = kHalfC * x1;
     float gx0 = 0.f, gx1 = 0.f;
-    f4 zv4, v4, s4;
+    f4 zv4, v4, s4, tx, ty, tb;
 #pragma unroll
     for (int r = 0; r < 4; ++r) zv4[r] = layer0_zv(w0, r, x0, x1);
     tanh_scaled4(zv4, v4, s4);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const float v = v4[r], s = s4[r];
-      float bv = hb[0][r], bj0 = hb[1][r], bj1 = hb[2][r], bl = hb[3][r];
-      tanh_jet_adjoint_vs(v, s, w0.wx[r], w0.wy[r], 0.0f, bv, bj0, bj1, bl);
-      gx0 = __builtin_fmaf(w0.cwx[r], bv, gx0);
-      gx1 = __builtin_fmaf(w0.cwy[r], bv, gx1);
-      const float t0 = sum_row16(__builtin_fmaf(bv, cx0, bj0));
-      const float t1 = sum_row16(__builtin_fmaf(bv, cx1, bj1));
-      const float tb = sum_row16(bv);
-      sums.w0x = (m & 3) == r ? sums.w0x + t0 : sums.w0x;
-      sums.w0y = (m & 3) == r ? sums.w0y + t1 : sums.w0y;
-      sums.b0 = (m & 3) == r ? sums.b0 + tb : sums.b0;
+      float bv = hb[0][r];
+      if (kBoundary) {
+        bv *= s4[r];
+        tx[r] = bv * cx0;
+        ty[r] = bv * cx1;
+      } else {
+        float bj0 = hb[1][r], bj1 = hb[2][r], bl = hb[3][r];
+        tanh_jet_adjoint_layer0(v4[r], s4[r], w0.wx[r], w0.wy[r], w0.q[r], bv, bj0, bj1, bl);
+        gx0 = __builtin_fmaf(w0.cwx[r], bv, gx0);
+        gx1 = __builtin_fmaf(w0.cwy[r], bv, gx1);
+        tx[r] = __builtin_fmaf(bv, cx0, bj0);
+        ty[r] = __builtin_fmaf(bv, cx1, bj1);
+      }
+      tb[r] = bv;
     }
-    gx0 = sum_lane_groups(gx0);
-    gx1 = sum_lane_groups(gx1);
-    if (g == 0) {
-      sc.gx[w][0][m] = gx0;
-      sc.gx[w][1][m] = gx1;
+    sums.w0x += sign * row_total(tx, m);
+    sums.w0y += sign * row_total(ty, m);
+    sums.b0 += sign * row_total(tb, m);
+    if (!kBoundary) {
+      gx0 = sum_lane_groups(gx0);
+      gx1 = sum_lane_groups(gx1);
+      if (g == 0) {
+        sc.gx[w][0][m] = gx0;
+        sc.gx[w][1][m] = gx1;
+      }
     }
-    __syncthreads();
-    if (w == 0 && g == 0 && active && grad_coordinates != nullptr && !on_boundary) {
-      grad_coordinates[2 * point] = ((sc.gx[0][0][m] + sc.gx[1][0][m]) + sc.gx[2][0][m]) + sc.gx[3][0][m];
-      grad_coordinates[2 * point + 1] = ((sc.gx[0][1][m] + sc.gx[1][1][m]) + sc.gx[2][1][m]) + sc.gx[3][1][m];
+    __syncthreads();  // also: every wave is done with the exchanges
+    if (!kBoundary && w == 0 && g == 0 && active && grad_coordinates != nullptr) {
+      grad_coordinates[2 * point] = sign * (((sc.gx[0][0][m] + sc.gx[1][0][m]) + sc.gx[2][0][m]) + sc.gx[3][0][m]);
+      grad_coordinates[2 * point + 1] = sign * (((sc.gx[0][1][m] + sc.gx[1][1][m]) + sc.gx[2][1][m]) + sc.gx[3][1][m]);
+    }
+  }
+}
+
+// A wave's 32 x 32 block (w >> 1, w & 1) of each hidden dW into the partial row: register r of
+// lane (n, h) holds row 8 (r / 4) + 4 h + r % 4, column n of the block. The sums are of d/d(4 W).
+// Non-temporal stores: the row is read once, by the reduction kernel, so it is streamed out
+// at once instead of waiting dirty in L2 for the write-back at the kernel's end (with every
+// workgroup's row dirty there, that write-back took about 3 us of a short call's tail).
+__device__ __forceinline__ void store_dw(float* row, int w, int lane, const f16 (&dw)[3]) {
+  const int at = opaque((32 * (w >> 1) + 4 * (lane >> 5)) * kHidden + 32 * (w & 1) + (lane & 31));
+#pragma unroll
+  for (int l = 0; l < 3; ++l) {
+    float* block = row + kHiddenBase + l * kHiddenStride;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      __builtin_nontemporal_store(4.0f * dw[l][r], &block[at + (8 * (r >> 2) + (r & 3)) * kHidden]);
     }
   }
 }
@@ -1776,14 +1796,11 @@ __device__ __forceinline__ void split_tile(const float* s_w, const float* s_smal
 // somewhat slower than the library's.
 enum ClockField : int {
   kClockStage,          // kernel start to the end of the parameter staging
-  kClockForward,        // a tile's start: layer 0 and hidden layers 1, 2 (the forward re-run)
-  kClockLayer3,         // hidden layer 3's forward, the loss and output seed, zbar3's staging
-  kClockDw3,            // dW3 (three staged passes)
-  kClockAdjoint3,       // W3^T zbar3 into layer 2's adjoint
-  kClockDw2,            // dW2
-  kClockAdjoint2,       // W2^T zbar2 into layer 1's adjoint, layer 0 rebuilt
-  kClockDw1,            // dW1
-  kClockLayer0,         // W1^T zbar1, layer 0's adjoint, coordinate gradients
+  kClockForward,        // a tile's start: layer 0 and hidden layers 1..3 (the forward re-run)
+  kClockSeed,           // the loss and output seed, zbar3 split
+  kClockLayer3,         // dW3 and W3^T zbar3 into layer 2's adjoint
+  kClockLayer2,         // dW2 and W2^T zbar2 into layer 1's adjoint
+  kClockLayer1,         // layer 0 rebuilt, dW1, W1^T zbar1, layer 0's adjoint, coordinate gradients
   kClockRest,           // 16-point split tiles past the last whole round
   kClockBoundary,       // boundary tiles of the fused step
   kClockPartials,       // the slot's partial row
@@ -1828,31 +1845,26 @@ struct PhaseClock {
 };
 #endif
 
-// The outputs h1, h2, h3 of the hidden layers stay in registers through the walk back (each
-// layer's zbar replaces its h in place, and hbar is live one 16-row block at a time), so no
-// layer is parked in memory.
+// The outputs h1, h2, h3 of the hidden layers stay in registers through the walk back (a layer's
+// zbar replaces h3, then is built beside the h that dW still reads).
 //
 // kLoss: grad_output and grad_laplacian are unused and the seed comes from `seed` (above);
 // grad_coordinates may be null.
-// kSaved (backward call only): interior tiles read h1, h2, h3 from `saved`, written by the
-// saving forward (saved_index; saved_tiles 16-point tiles), instead of re-running the forward.
-// A wave whose 16-point tile lies past the batch takes zeros: its upstream gradients are zero,
-// so every product with its h is zero either way. Split tiles past the last whole round still
-// re-run the forward.
-template <bool kLoss, bool kRest, bool kSaved>
+template <bool kLoss, bool kRest>
 __global__ void __launch_bounds__(kBwdWaves * kWave, 1)
 backward_kernel(const float* __restrict__ coordinates, const float* __restrict__ params,
                 const float* __restrict__ grad_output, const float* __restrict__ grad_laplacian,
                 float* __restrict__ grad_coordinates, float* __restrict__ partials,
-                int64_t batch, int64_t whole, int64_t tiles, int slots, LossSeed seed,
-                const f4* __restrict__ saved, int64_t saved_tiles) {
-  static_assert(!(kLoss && kSaved), "the fused step computes its forward once; nothing to read");
-  constexpr int kStageFloats = kRest && kSplitScratchFloats > kStagePlanes * kPlane
-                                   ? kSplitScratchFloats
-                                   : kStagePlanes * kPlane;
-  __shared__ __attribute__((aligned(16))) float s_w[3 * kPlane];
+                int64_t batch, int64_t whole, int64_t tiles, int slots, LossSeed seed) {
+  constexpr int kCombined = 7;  // point sums combined over the waves: w0x, w0y, b0, wout, bh[3]
+  union Scratch {
+    DwStage stage;
+    SplitScratch split;
+    float comb[kCombined][kBwdWaves][kHidden];
+  };
+  __shared__ u4 s_w[3 * kLayerU4];
   __shared__ __attribute__((aligned(16))) float s_small[kSmallFloats];
-  __shared__ __attribute__((aligned(16))) float s_stage[kStageFloats];
+  __shared__ Scratch s_x;
   __shared__ float s_red[3][kBwdWaves];
   const int lane = threadIdx.x & (kWave - 1);
   const int w = threadIdx.x / kWave;
@@ -1868,32 +1880,33 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
   // kLoss: the Adam step count is read with the staging loads and advanced after the barrier
   // (an increment in place waited for its load before wave 0 issued any staging load).
   const float step_count = kLoss ? seed.step[0] : 0.0f;
-  stage_parameters<kBwdWaves * kWave>(params, s_w, s_small, threadIdx.x);
+  const SmallLoads small = load_small<kBwdWaves * kWave>(params, threadIdx.x);
+  stage_operand_weights<kBwdWaves * kWave>(params, s_w, threadIdx.x);
+  store_small(s_small, threadIdx.x, small);
   __syncthreads();
   if (kLoss && blockIdx.x == 0 && threadIdx.x == 0) seed.step[0] = step_count + 1.0f;
   clock.mark(kClockStage);
 
-  // Lane offsets into the LDS arrays. Each use forms its base from an opaque copy: the arrays
-  // span more than the 64 KB reach of a DS offset, and hoisted bases would be spilled.
-  const int rows_off = lane_rows(m, g);
-  const int cols_off = lane_cols(m, g);
-  const int stage_write_off = cols_off + 16 * w;    // staging writes: point 16 w + m
-  const int stage_a_off = rows_off + 16 * kWRow * w;  // A operand reads: this wave's rows
-  auto stage_bases = [&]() {
-    const int wo = opaque(stage_write_off), ao = opaque(stage_a_off), ro = opaque(rows_off);
-    return StageBases{s_stage + wo, s_stage + 3 * kPlane + wo, s_stage + ao,
-                      s_stage + 3 * kPlane + ro};
-  };
+  const u2 minus_one = minus_identity(m, g);
+  const int entry = operand_entry(m, g);
+  const u4* w_lane = s_w + entry;
+  const u4* w_t = s_w + transposed_entry(m, g);
+  StagePointers sp;
+  sp.wz = s_x.stage.z[w] + entry;
+  sp.wh = s_x.stage.h[w] + entry;
+  sp.ra = dw_pointers(s_x.stage.z[0] + (w >> 1) * kParts * kWave, m, g);
+  sp.rb = dw_pointers(s_x.stage.h[0] + (w & 1) * kParts * kWave, m, g);
 
   for (int slot = blockIdx.x; slot < slots; slot += gridDim.x) {
-    WaveSums acc;
+    f16 dw[3];
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) acc.dw[l][nb] = zero4();
-      acc.bh[l] = 0.f;
+      for (int r = 0; r < 16; ++r) dw[l][r] = 0.0f;
     }
-    acc.w0x = acc.w0y = acc.b0 = acc.wout = acc.bout = acc.loss = acc.bloss = 0.f;
+    // Point sums of this wave (lane = owned neuron), and of r^2 and u_b^2 (kLoss).
+    float sum[kCombined] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float sum_bout = 0.f, sum_loss = 0.f, sum_bloss = 0.f;
 
     // Per-point inputs are read one tile ahead and delivered mid-tile (deliver), so no tile
     // starts with a wait on global memory: with one wave per SIMD nothing would hide it. The
@@ -1908,25 +1921,11 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
     // the same order as one would. One loop with both kinds of tile cost about 100 register
     // copies a tile, where the two paths' accumulators met at the loop's back edge.
     int64_t tile = slot;
+    int round = 0;  // tiles of this slot so far (walk_sign)
     const int64_t interior_end = kLoss ? std::min<int64_t>(tiles, seed.interior_tiles) : tiles;
     const int64_t loop_end = kRest ? whole : interior_end;
-    // Hidden-layer outputs of the current tile. With kSaved each layer of the next tile is read
-    // where this tile's copy dies in the walk back (layer 3 after W3^T zbar3, layer 2 after
-    // W2^T zbar2, layer 1 at the end), so the reads spread over the tile: read at each tile's
-    // start, the waves of all CUs asked for their 48 KB at once and waited out that burst.
-    // (Reading a slot's first tile before the weight staging measured no faster.)
-    f4 h1[4][4], h2[4][4], h3[4][4];
-    if constexpr (kSaved) {
-      if (tile < loop_end) {
-        const int64_t saved_tile = kBwdWaves * tile + w;
-        load_saved_layer(saved, saved_tile, saved_tiles, 2, lane, h3);
-        load_saved_layer(saved, saved_tile, saved_tiles, 1, lane, h2);
-        load_saved_layer(saved, saved_tile, saved_tiles, 0, lane, h1);
-      }
-    }
-    for (; tile < loop_end; tile += slots) {
-      const bool has_next = tile + slots < loop_end;
-      const int64_t next_saved_tile = kBwdWaves * (tile + slots) + w;
+    f4 h1[4][4], h2[4][4], h3[4][4];  // hidden-layer outputs of the current tile
+    for (; tile < loop_end; tile += slots, ++round) {
       keep_lds_reads_in_loop();
       const int m_pick = opaque(m);  // row_reduce_scatter16's lane masks stay inside the tile
       const TileInputs in = next;
@@ -1937,234 +1936,195 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
       const float x0 = in.x0, x1 = in.x1;
       const int64_t point = tile * kBwdTile + kTile * w + m;
       const bool active = point < batch;
-      float gu = kLoss ? 0.f : in.a, gl = kLoss ? 0.f : in.b;
-      const float f = kLoss ? in.a : 0.f;
+      const float sign = walk_sign(slot, round);
+      const float gu = kLoss ? 0.f : sign * in.a;
+      float gl = kLoss ? 0.f : sign * in.b;
 
-      // ---- 1. forward recompute (kSaved: read ahead, above and in the walk back) ----
-      // h2 is dW3's h_prev: its early components go to the staging planes between hidden layer
-      // 3's MFMAs, once every wave is done with the previous tile's planes.
-      if constexpr (!kSaved) {
-        {
-          f4 h0[4][4];
-          layer0_forward(s_small, g, x0, x1, h0);
-          forward_layer(s_small, s_w + opaque(rows_off), 0, g, h0, h1);
-        }
-        forward_layer(s_small, s_w + opaque(rows_off), 1, g, h1, h2);
+      // ---- 1. forward re-run ----
+      {
+        JetOperand a, b;
+        WeightOperand wf = lds_weights(w_lane, 0);
+        layer0_operand(s_small, minus_one, g, x0, x1, a);
+        BlockWork<true> work;
+        BlockWork<false> last;
+        // The previous layer's block 3 in the five steps before its operand is needed.
+        auto finish = [&](int j, f4 (&out)[4], JetOperand& op) {
+          const int from = j == 0 ? 0 : 2 * j + 2, to = j == 0 ? 4 : 2 * j + 4;
+#pragma unroll
+          for (int i = 0; i < 12; ++i) {
+            if (i >= from && i < to) work.stage(i, minus_one, out);
+          }
+          if (j == 4) {
+            work.put(op, 3);
+            park_block(out);
+          }
+        };
+        forward_layer<true>(s_small, w_lane, w_lane + kLayerU4, minus_one, 0, g, a, h1, b, wf, work,
+                            [](int) {});
+        forward_layer<true>(s_small, w_lane + kLayerU4, w_lane + 2 * kLayerU4, minus_one, 1, g, b, h2, a, wf,
+                            work, [&](int j) { finish(j, h1[3], b); });
+        forward_layer<false>(s_small, w_lane + 2 * kLayerU4, w_lane, minus_one, 2, g, a, h3, b, wf, last,
+                             [&](int j) { finish(j, h2[3], a); });
+#pragma unroll
+        for (int j = 0; j < 5; ++j) last.stage(j, minus_one, h3[3]);
+        region_end();
       }
       clock.mark(kClockForward);
-      __syncthreads();  // the previous tile's readers of the staging planes are done
-      const StageBases sb3 = stage_bases();
-      auto stage_h2 = [&](int mb, int step) {
-        if (step >= 12) return false;
-        const int e = step >> 2, r = step & 3;
-        sb3.wh[e * kPlane + kWRow * (16 * mb + r)] = h2[mb][early_component(e)][r];
-        return true;
-      };
-      auto stage_zbar3 = [&](int mb, int i) {  // write i < 12 of zbar3's early components
-        sb3.wz[(i >> 2) * kPlane + kWRow * (16 * mb + (i & 3))] = h3[mb][early_component(i >> 2)][i & 3];
-      };
 
       // ---- 2. output layer: w_out / b_out gradients, and hidden layer 3's adjoint ----
       // In the scaled jet u = (4 w_out / c) . v' + b_out and lap = (4 w_out / lambda) . L', so
       // dw_out = sum_p (4 gu / c) v' + (4 gl / lambda) L' and the seeds are
       // vbar' = 4 gu w_out / c, Lbar' = 4 gl w_out / lambda, Jbar' = 0. The point sums stay in
       // registers (row_reduce_scatter16). With kLoss, gu = 0 on interior points: the value seed
-      // and the u terms are dropped (their products with zero). h3 becomes zbar3 in place, block
-      // by block: in the backward call, whose upstream gradients are inputs, as soon as hidden
-      // layer 3's block is done (its staging writes then drain behind the next block's MFMAs);
-      // in the fused step after the loss, which needs all of h3.
-      float wout_terms[16];
-      auto seed_block = [&](int mb) {
-        const float gu_c = gu * (4.0f / kC);
-        const float gl_l = gl * (4.0f / kLambda);
-        const f4 wv = lds4(s_small + kSmallWoutV + 16 * mb + 4 * g);
-        const f4 wl = lds4(s_small + kSmallWoutL + 16 * mb + 4 * g);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          wout_terms[4 * mb + r] = kLoss ? gl_l * h3[mb][3][r]
-                                         : __builtin_fmaf(gu_c, h3[mb][0][r], gl_l * h3[mb][3][r]);
-          float bv = kLoss ? 0.0f : gu * wv[r], bj0, bj1, bl = gl * wl[r];
-          tanh_jet_adjoint_h_seed<kLoss>(h3[mb][0][r], h3[mb][1][r], h3[mb][2][r], h3[mb][3][r],
-                                         bv, bj0, bj1, bl);
-          h3[mb][0][r] = bv;
-          h3[mb][1][r] = bj0;
-          h3[mb][2][r] = bj1;
-          h3[mb][3][r] = bl;
-        }
-      };
-      constexpr bool kSeedInLayer3 = !kLoss && !kSaved;
-      if constexpr (kSeedInLayer3) {
-        forward_layer(
-            s_small, s_w + opaque(rows_off), 2, g, h2, h3,
-            [&](int mb, int step) {
-              const bool wrote = stage_h2(mb, step);
-              if (mb > 0 && step < 12) stage_zbar3(mb - 1, step);
-              return wrote || (mb > 0 && step < 12);
-            },
-            seed_block);
-#pragma unroll
-        for (int i = 0; i < 12; ++i) stage_zbar3(3, i);
-      } else {
-        if constexpr (!kSaved) {
-          forward_layer(s_small, s_w + opaque(rows_off), 2, g, h2, h3, stage_h2);
-        } else {
-#pragma unroll
-          for (int mb = 0; mb < 4; ++mb) {
-#pragma unroll
-            for (int step = 0; step < 12; ++step) stage_h2(mb, step);
-          }
-        }
-        if (kLoss) {
-          // lap = w_out . L in the forward kernel's order, then the seed.
-          float out = 0.0f;
-#pragma unroll
-          for (int mb = 0; mb < 4; ++mb) {
-            const f4 wo = lds4(s_small + kSmallWoutL + 16 * mb + 4 * g);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) out = __builtin_fmaf(wo[r], h3[mb][3][r], out);
-          }
-          out = sum_lane_groups(out);
-          const float res = active ? out - f : 0.0f;
-          gl = seed.inv_batch * (2.0f * res);
-          acc.loss += sum_row16(res * res);
-        }
+      // and the u terms are dropped (their products with zero).
+      if (kLoss) {
+        // lap = w_out . L in the forward kernel's order, then the seed.
+        float out = 0.0f;
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb) {
-          seed_block(mb);
+          const f4 wo = lds4(s_small + kSmallWoutL + 16 * mb + 4 * g);
+          float t = 0.0f;
 #pragma unroll
-          for (int i = 0; i < 12; ++i) stage_zbar3(mb, i);
+          for (int r = 0; r < 4; ++r) t = __builtin_fmaf(wo[r], h3[mb][3][r], t);
+          out = mb ? out + t : t;
         }
+        out = sum_lane_groups(out);
+        const float res = active ? out - in.a : 0.0f;
+        gl = sign * (seed.inv_batch * (2.0f * res));
+        sum_loss += sum_row16(res * res);
       }
-      acc.wout += row_reduce_scatter16(wout_terms, m_pick);
-      if (!kLoss) acc.bout += sum_row16(gu);
+      JetOperand zb;
+      {
+        const float gu_c = gu * (4.0f / kC);
+        const float gl_l = gl * (4.0f / kLambda);
+        float wout_terms[16], bias_terms[16];
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb) {
+          const f4 wv = lds4(s_small + kSmallWoutV + 16 * mb + 4 * g);
+          const f4 wl = lds4(s_small + kSmallWoutL + 16 * mb + 4 * g);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            wout_terms[4 * mb + r] = kLoss ? gl_l * h3[mb][3][r]
+                                           : __builtin_fmaf(gu_c, h3[mb][0][r], gl_l * h3[mb][3][r]);
+            float bv = kLoss ? 0.0f : gu * wv[r], bj0, bj1, bl = gl * wl[r];
+            tanh_jet_adjoint_h_seed<kLoss>(h3[mb][0][r], h3[mb][1][r], h3[mb][2][r], h3[mb][3][r],
+                                           bv, bj0, bj1, bl);
+            h3[mb][0][r] = bv;
+            h3[mb][1][r] = bj0;
+            h3[mb][2][r] = bj1;
+            h3[mb][3][r] = bl;
+            bias_terms[4 * mb + r] = bv;
+          }
+        }
+        put_all(minus_one, zb, h3);
+        sum[3] += sign * row_reduce_scatter16(wout_terms, m_pick);
+        sum[6] += sign * row_reduce_scatter16(bias_terms, m_pick);
+        if (!kLoss) sum_bout += sign * sum_row16(gu);
+      }
+      clock.mark(kClockSeed);
+
+      // ---- 3. hidden layers 3 and 2: dW from (zbar, h_prev), W^T zbar into the adjoint of the
+      // layer below, which is the next zbar ----
+      WeightOperand wt = lds_transposed_weights(w_t + 2 * kLayerU4, 0);
+      auto walk = [&](int layer, const f4 (&h)[4][4], float& bias) {
+        f4 z[4][4];
+        backward_layer(w_t + layer * kLayerU4, w_t + (layer - 1) * kLayerU4, sp, zb, h, sign, dw[layer], wt,
+                       [&](int ib, int r, const f4 (&hb)[4]) {
+                         float bv = hb[0][r], bj0 = hb[1][r], bj1 = hb[2][r], bl = hb[3][r];
+                         tanh_jet_adjoint_h(h[ib][0][r], h[ib][1][r], h[ib][2][r], h[ib][3][r], bv, bj0,
+                                            bj1, bl);
+                         z[ib][0][r] = bv;
+                         z[ib][1][r] = bj0;
+                         z[ib][2][r] = bj1;
+                         z[ib][3][r] = bl;
+                       });
+        float terms[16];
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) terms[4 * mb + r] = z[mb][0][r];
+        }
+        put_all(minus_one, zb, z);
+        bias += sign * row_reduce_scatter16(terms, m_pick);
+      };
+      walk(2, h2, sum[5]);
       clock.mark(kClockLayer3);
+      walk(1, h1, sum[4]);
+      clock.mark(kClockLayer2);
+      deliver(next);  // the next tile's inputs, before this tile's stores
 
-      // ---- 3. hidden layer 3: dW3 from (zbar3, h2), then W3^T zbar3 into layer 2's adjoint ----
-      // The adjoint's blocks of zbar2 and h1 (dW2's operands) are staged behind the MFMAs of the
-      // next block.
-      staged_dw(sb3, {h3[0][kLateComponent], h3[1][kLateComponent], h3[2][kLateComponent], h3[3][kLateComponent]},
-                {h2[0][kLateComponent], h2[1][kLateComponent], h2[2][kLateComponent], h2[3][kLateComponent]},
-                acc.dw[2], acc.bh[2]);
-      clock.mark(kClockDw3);
-      __syncthreads();  // every wave is done with the staged planes
-      {
-        const StageBases sb = stage_bases();
-        adjoint_through(s_w + opaque(cols_off) + 2 * kPlane, h3, h2, [](int) {},
-                        [&](int ib, int step) { return emit_early_pair(sb, ib, h2[ib], h1[ib], step); });
-      }
-      if constexpr (kSaved) {
-        if (has_next) load_saved_layer(saved, next_saved_tile, saved_tiles, 2, lane, h3);
-      }
-      clock.mark(kClockAdjoint3);
-
-      // ---- 4. hidden layer 2: dW2 from (zbar2, h1), then W2^T zbar2 into layer 1's adjoint ----
-      // Layer 0's output h0 (dW1's h_prev) is rebuilt block by block from its closed form
-      // z' = (c (W0 x + b0), 2 W0[:,0], 2 W0[:,1], 0), keeping its (v', s') for layer 0's own
-      // adjoint; the blocks of zbar1 and h0 are staged behind the next block's MFMAs.
-      f4 v0[4], s0[4], h0[4][4];
-      {
-        const StageBases sb = stage_bases();
-        staged_dw(sb, {h2[0][kLateComponent], h2[1][kLateComponent], h2[2][kLateComponent], h2[3][kLateComponent]},
-                  {h1[0][kLateComponent], h1[1][kLateComponent], h1[2][kLateComponent], h1[3][kLateComponent]},
-                  acc.dw[1], acc.bh[1]);
-        clock.mark(kClockDw2);
-        deliver(next);  // the next tile's inputs, before this tile's stores
-        __syncthreads();  // every wave is done with the staged planes
-        adjoint_through(
-            s_w + opaque(cols_off) + kPlane, h2, h1,
-            [&](int ib) {
-              const Layer0Weights w0 = layer0_weights(s_small, ib, g);
-              f4 zv;
-#pragma unroll
-              for (int r = 0; r < 4; ++r) zv[r] = layer0_zv(w0, r, x0, x1);
-              tanh_scaled4(zv, v0[ib], s0[ib]);
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                h0[ib][0][r] = v0[ib][r];
-                h0[ib][1][r] = s0[ib][r] * w0.wx[r];
-                h0[ib][2][r] = s0[ib][r] * w0.wy[r];
-                h0[ib][3][r] = s0[ib][r] * (v0[ib][r] * w0.q[r]);
-              }
-            },
-            [&](int ib, int step) { return emit_early_pair(sb, ib, h1[ib], h0[ib], step); });
-      }
-      if constexpr (kSaved) {
-        if (has_next) load_saved_layer(saved, next_saved_tile, saved_tiles, 1, lane, h2);
-      }
-      clock.mark(kClockAdjoint2);
-
-      // ---- 5. hidden layer 1: dW1 from (zbar1, h0) ----
-      staged_dw(stage_bases(),
-                {h1[0][kLateComponent], h1[1][kLateComponent], h1[2][kLateComponent], h1[3][kLateComponent]},
-                {h0[0][kLateComponent], h0[1][kLateComponent], h0[2][kLateComponent], h0[3][kLateComponent]},
-                acc.dw[0], acc.bh[0]);
-      clock.mark(kClockDw1);
-
-      // ---- 6. W1^T zbar1, one block at a time, into layer 0 in closed form ----
+      // ---- 4. hidden layer 1, whose h_prev is layer 0's output, rebuilt from its closed form
+      // z' = (c (W0 x + b0), 2 W0[:,0], 2 W0[:,1], 0), and layer 0 in closed form ----
       // bv is the adjoint of z'_v = c z_v and bj_d that of z'_Jd = 2 W0[:, d], so
       // grad_x = (c W0)^T bv, dW0[o][d] = sum_p bv (c x_d) + 2 bj_d = 2 sum_p (bv (c x_d / 2) + bj_d)
       // (the row takes the 2), db0 = c sum_p bv.
       {
-        float gx0 = 0.f, gx1 = 0.f, tx[16], ty[16], tb[16];
-        const float cx0 = kHalfC * x0, cx1 = kHalfC * x1;
-        const float* w_t = s_w + opaque(cols_off);
-        float next_a[16];
-        transposed_operands(w_t, 0, next_a);
+        f4 h0[4][4], s0[4];
 #pragma unroll
-        for (int ib = 0; ib < 4; ++ib) {
-          float a[16];
+        for (int mb = 0; mb < 4; ++mb) {
+          const Layer0Weights w0 = layer0_weights(s_small, mb, g);
+          f4 zv;
 #pragma unroll
-          for (int k = 0; k < 16; ++k) a[k] = next_a[k];
-          if (ib < 3) transposed_operands(w_t, ib + 1, next_a);
-          lds_mfma_fence();
-          f4 hb[4];
-          transposed_block(a, h1, hb);
-          lds_mfma_fence();
-          const Layer0Weights w0 = layer0_weights(s_small, ib, g);
+          for (int r = 0; r < 4; ++r) zv[r] = layer0_zv(w0, r, x0, x1);
+          tanh_scaled4(zv, h0[mb][0], s0[mb]);
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            float bv = hb[0][r], bj0 = hb[1][r], bj1 = hb[2][r], bl = hb[3][r];
-            tanh_jet_adjoint_layer0(v0[ib][r], s0[ib][r], w0.wx[r], w0.wy[r], w0.q[r], bv, bj0,
-                                    bj1, bl);
-            gx0 = __builtin_fmaf(w0.cwx[r], bv, gx0);
-            gx1 = __builtin_fmaf(w0.cwy[r], bv, gx1);
-            tx[4 * ib + r] = __builtin_fmaf(bv, cx0, bj0);  // dW0[o][0] / 2
-            ty[4 * ib + r] = __builtin_fmaf(bv, cx1, bj1);  // dW0[o][1] / 2
-            tb[4 * ib + r] = bv;                            // db0[o] / c
+            h0[mb][1][r] = s0[mb][r] * w0.wx[r];
+            h0[mb][2][r] = s0[mb][r] * w0.wy[r];
+            h0[mb][3][r] = s0[mb][r] * (h0[mb][0][r] * w0.q[r]);
           }
         }
-        acc.w0x += row_reduce_scatter16(tx, m_pick);
-        acc.w0y += row_reduce_scatter16(ty, m_pick);
-        acc.b0 += row_reduce_scatter16(tb, m_pick);
-        if constexpr (kSaved) {
-          if (has_next) load_saved_layer(saved, next_saved_tile, saved_tiles, 0, lane, h1);
-        }
+        float gx0 = 0.f, gx1 = 0.f, tx[16], ty[16], tb[16];
+        const float cx0 = kHalfC * x0, cx1 = kHalfC * x1;
+        backward_layer(w_t, w_t, sp, zb, h0, sign, dw[0], wt, [&](int ib, int r, const f4 (&hb)[4]) {
+          const float* w0 = s_small + 16 * ib + 4 * g + r;
+          float bv = hb[0][r], bj0 = hb[1][r], bj1 = hb[2][r], bl = hb[3][r];
+          tanh_jet_adjoint_layer0(h0[ib][0][r], s0[ib][r], w0[kSmallWx], w0[kSmallWy], w0[kSmallQ0], bv, bj0,
+                                  bj1, bl);
+          gx0 = __builtin_fmaf(w0[kSmallCwx], bv, gx0);
+          gx1 = __builtin_fmaf(w0[kSmallCwy], bv, gx1);
+          tx[4 * ib + r] = __builtin_fmaf(bv, cx0, bj0);  // dW0[o][0] / 2
+          ty[4 * ib + r] = __builtin_fmaf(bv, cx1, bj1);  // dW0[o][1] / 2
+          tb[4 * ib + r] = bv;                            // db0[o] / c
+        });
+        sum[0] += sign * row_reduce_scatter16(tx, m_pick);
+        sum[1] += sign * row_reduce_scatter16(ty, m_pick);
+        sum[2] += sign * row_reduce_scatter16(tb, m_pick);
         gx0 = sum_lane_groups(gx0);
         gx1 = sum_lane_groups(gx1);
         if (g == 0 && active && grad_coordinates != nullptr) {
-          grad_coordinates[2 * point] = gx0;
-          grad_coordinates[2 * point + 1] = gx1;
+          grad_coordinates[2 * point] = sign * gx0;
+          grad_coordinates[2 * point + 1] = sign * gx1;
         }
       }
-      clock.mark(kClockLayer0);
+      clock.mark(kClockLayer1);
       clock.count(kClockTiles);
     }
+    // A split tile's point sums into this wave's owned-neuron lanes (owned_neuron): the wave's rows
+    // only; the point sums shared by the 4 waves from wave 0 alone.
+    auto add_split = [&](const SplitSums& s, int m_pick) {
+      const bool own = (m_pick >> 2) == w;
+      sum[0] += own ? s.w0x : 0.f;
+      sum[1] += own ? s.w0y : 0.f;
+      sum[2] += own ? s.b0 : 0.f;
+      sum[3] += own ? s.wout : 0.f;
+#pragma unroll
+      for (int l = 0; l < 3; ++l) sum[4 + l] += own ? s.bh[l] : 0.f;
+      if (w == 0) {
+        sum_bout += s.bout;
+        sum_loss += s.loss;
+        sum_bloss += s.bloss;
+      }
+    };
     // kRest: interior points past the last whole round of 64-point tiles, as 16-point tiles
     // whose rows are split over the 4 waves (split_tile), so a round that is not whole costs a
     // quarter tile on the slots that have one instead of a whole tile on some. The scratch
     // overlays the dW staging buffer: the barrier waits for the last 64-point tile's readers.
     // (A separate instantiation: with this loop in the kernel the compiler schedules the
-    // 64-point loop differently, about 0.5 % slower, so whole rounds run without it.)
+    // 64-point loop differently, so whole rounds run without it.)
     if (kRest && tile < interior_end) {  // uniform per workgroup
       __syncthreads();
-      const SplitScratch scratch{
-          s_stage, reinterpret_cast<f4 (*)[kSplitWaves][4][kWave]>(s_stage + 3 * kTPlane),
-          reinterpret_cast<float (*)[kTWave]>(s_stage + 3 * kTPlane + 2 * kSplitWaves * 4 * kWave * 4),
-          reinterpret_cast<float (*)[2][kTile]>(s_stage + 3 * kTPlane +
-                                                2 * kSplitWaves * 4 * kWave * 4 +
-                                                kSplitWaves * kTWave)};
-      int phase = 0;
-      for (; tile < interior_end; tile += slots) {
+      for (; tile < interior_end; tile += slots, ++round) {
         keep_lds_reads_in_loop();
         const int m_pick = opaque(m);
         const TileInputs in = next;
@@ -2173,29 +2133,18 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
                                          seed, tile + slots, w, m);
         }
         const int64_t point = whole * kBwdTile + (tile - whole) * kTile + m;
-        SplitSums sums{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        split_tile<kLoss>(s_w, s_small, scratch, phase, w, g, m_pick,
-                          opaque(rows_off) + 1088 * w, opaque(cols_off) + 16 * w,
-                          m_pick * kWRow + 4 * g, in.x0, in.x1, kLoss ? 0.f : in.a,
-                          kLoss ? 0.f : in.b, kLoss ? in.a : 0.f, point < batch, false, point,
-                          grad_coordinates, seed, acc.dw, acc.bh, sums);
-        // Into this wave's owned-neuron lanes (owned_neuron): the wave's rows only; the point
-        // sums shared by the 4 waves from wave 0 alone.
-        const bool own = (m_pick >> 2) == w;
-        acc.w0x += own ? sums.w0x : 0.f;
-        acc.w0y += own ? sums.w0y : 0.f;
-        acc.b0 += own ? sums.b0 : 0.f;
-        acc.wout += own ? sums.wout : 0.f;
-        if (w == 0) {
-          acc.bout += sums.bout;
-          acc.loss += sums.loss;
-        }
+        SplitSums s{};
+        split_tile<4, kLoss>(w_lane, w_t, s_small, s_x.split, minus_one, w, g, m_pick, in.x0, in.x1,
+                             kLoss ? 0.f : in.a, kLoss ? 0.f : in.b, kLoss ? in.a : 0.f,
+                             point < batch, walk_sign(slot, round), point, grad_coordinates, seed, dw, s);
+        add_split(s, m_pick);
         deliver(next);
       }
       clock.mark(kClockRest);
     }
-    if (kLoss) {
-      for (; tile < tiles; tile += slots) {  // boundary tiles (uniform per workgroup)
+    if (kLoss && tile < tiles) {  // boundary tiles (uniform per workgroup)
+      __syncthreads();
+      for (; tile < tiles; tile += slots, ++round) {
         keep_lds_reads_in_loop();
         const int m_pick = opaque(m);
         const TileInputs in = next;
@@ -2204,9 +2153,10 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
                                          tile + slots, w, m);
         }
         const int64_t point = (tile - seed.interior_tiles) * kTile + m;
-        const bool active = point < seed.boundary_count;
-        boundary_tile(s_w, s_small, s_stage, rows_off, cols_off, w, g, m_pick, in.x0, in.x1,
-                      active, seed.boundary_scale, acc);
+        SplitSums s{};
+        split_tile<1, kLoss>(w_lane, w_t, s_small, s_x.split, minus_one, w, g, m_pick, in.x0, in.x1, 0.f,
+                             0.f, 0.f, point < seed.boundary_count, walk_sign(slot, round), point, nullptr, seed, dw, s);
+        add_split(s, m_pick);
         deliver(next);
         clock.mark(kClockBoundary);
         clock.count(kClockBoundaryTiles);
@@ -2214,45 +2164,34 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
     }
 
     // ---- this slot's partial row: every entry written by exactly one lane ----
-    // Non-temporal stores: the row is read once, by the reduction kernel, so it is streamed out
-    // at once instead of waiting dirty in L2 for the write-back at the kernel's end (with every
-    // workgroup's row dirty there, that write-back took about 3 us of a short call's tail).
     float* row = partials + static_cast<int64_t>(slot) * kRowStride;
-    const int dw_lane = opaque((16 * w + 4 * g) * kHidden + m);
-#pragma unroll
-    for (int l = 0; l < 3; ++l) {
-      float* wrow = row + kHiddenBase + l * kHiddenStride;
-#pragma unroll
-      for (int nb = 0; nb < 4; ++nb) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          __builtin_nontemporal_store(4.0f * acc.dw[l][nb][r], &wrow[dw_lane + r * kHidden + 16 * nb]);
-        }
-      }
-      // dW: the sums are of d/d(4 W); bias sums are of zbar_v' = c^-1 zbar_v.
-      if (g == 0) __builtin_nontemporal_store(kC * acc.bh[l], &wrow[kHidden * kHidden + 16 * w + m]);
-    }
+    store_dw(row, w, lane, dw);
     // Per-wave sums (lane = owned neuron) combined over the 4 waves in a fixed order.
     __syncthreads();  // every wave is done with the staging buffer
     {
-      float* comb = s_stage;  // [quantity][wave][neuron]
       const int o = owned_neuron(m, g);
-      comb[(0 * kBwdWaves + w) * kHidden + o] = acc.w0x;
-      comb[(1 * kBwdWaves + w) * kHidden + o] = acc.w0y;
-      comb[(2 * kBwdWaves + w) * kHidden + o] = acc.b0;
-      comb[(3 * kBwdWaves + w) * kHidden + o] = acc.wout;
+#pragma unroll
+      for (int q = 0; q < kCombined; ++q) s_x.comb[q][w][o] = sum[q];
       if (lane == 0) {
-        s_red[0][w] = acc.bout;
-        s_red[1][w] = acc.loss;
-        s_red[2][w] = acc.bloss;
+        s_red[0][w] = sum_bout;
+        s_red[1][w] = sum_loss;
+        s_red[2][w] = sum_bloss;
       }
       __syncthreads();
-      const int q = threadIdx.x >> 6, n = threadIdx.x & 63;  // quantity (0..3), neuron
-      const float* c4 = comb + q * kBwdWaves * kHidden + n;
-      const float total = ((c4[0] + c4[kHidden]) + c4[2 * kHidden]) + c4[3 * kHidden];
-      const int dst = q == 0 ? kInputs * n : q == 1 ? kInputs * n + 1 : q == 2 ? kLayer0Bias + n : kOutputBase + n;
-      // dW0 / 2, db0 / c, dw_out
-      __builtin_nontemporal_store((q == 2 ? kC : q == 3 ? 1.0f : 2.0f) * total, &row[dst]);
+      const int n = lane;  // neuron; this wave stores quantities w and w + 4
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int q = w + 4 * i;
+        if (q < kCombined) {
+          const float total = ((s_x.comb[q][0][n] + s_x.comb[q][1][n]) + s_x.comb[q][2][n]) + s_x.comb[q][3][n];
+          // dW0 / 2, db0 / c, dw_out, hidden db / c
+          const int dst = q < 2 ? kInputs * n + q
+                          : q == 2 ? kLayer0Bias + n
+                          : q == 3 ? kOutputBase + n
+                                   : kHiddenBase + (q - 4) * kHiddenStride + kHidden * kHidden + n;
+          __builtin_nontemporal_store((q < 2 ? 2.0f : q == 3 ? 1.0f : kC) * total, &row[dst]);
+        }
+      }
       if (threadIdx.x < (kLoss ? 3 : 1)) {
         const float* red = s_red[threadIdx.x];
         const int col = threadIdx.x == 0 ? kOutputBase + kHidden : kLossColumn + threadIdx.x - 1;
@@ -2266,18 +2205,12 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
 }
 
 // ---------------------------------------------------------------------------------------------
-// Small-batch backward. backward_kernel carries 16 points per wave through the whole walk:
-// 2,304 dependent MFMAs per 64-point workgroup tile, so a batch with at most one workgroup
-// tile per CU costs that latency whatever its size. Here a workgroup of 4 waves runs one
-// 16-point tile at a time and wave w owns rows 16 w .. 16 w + 15 of every layer: 64 MFMAs per
-// layer for the forward re-run, 64 for dW and 64 for W^T zbar (576 per tile and wave).
-//   * Layer outputs h and adjoints zbar go to the other waves lane to lane through LDS
-//     (s_x, the register layout of forward_split_kernel), for the next product's B operand.
-//   * dW contracts over the tile's points, which sit on the lane axis: h (all 64 rows, per
-//     layer) and this wave's zbar are also stored transposed, [row][c][4 g + s] for point
-//     4 s + g at pitch 68, so one 16-byte read gives a lane 4 points of one (row, c).
-//   * Each wave owns distinct entries of the slot's partial row (its rows of every block), so
-//     the partial row needs no combine across waves.
+// Small-batch backward. backward_kernel carries 16 points per wave through the whole walk, so a
+// batch with at most one workgroup tile per CU costs that latency whatever its size. Here a
+// workgroup of 4 waves runs one 16-point tile at a time with rows split over the waves
+// (split_tile; boundary tiles with the value channel alone).
+//   * Each wave owns distinct entries of the slot's partial row (its rows of the vectors, its
+//     block of every dW), so the partial row needs no combine across waves.
 // Slots and the fixed-order reduction are those of backward_kernel with 16-point tiles. The
 // choice between the two kernels depends only on the batch, so results do not depend on the
 // device. The tanh-jet, adjoint and loss arithmetic is backward_kernel's; the sums over points
@@ -2289,12 +2222,9 @@ backward_split_kernel(const float* __restrict__ coordinates, const float* __rest
                       const float* __restrict__ grad_laplacian,
                       float* __restrict__ grad_coordinates, float* __restrict__ partials,
                       int64_t batch, int64_t tiles, int slots, LossSeed seed) {
-  __shared__ __attribute__((aligned(16))) float s_w[3 * kPlane];
+  __shared__ u4 s_w[3 * kLayerU4];
   __shared__ __attribute__((aligned(16))) float s_small[kSmallFloats];
-  __shared__ __attribute__((aligned(16))) float s_ht[3 * kTPlane];  // h0, h1, h2 transposed
-  __shared__ f4 s_x[2][kSplitWaves][4][kWave];                       // lane-major exchange
-  __shared__ __attribute__((aligned(16))) float s_zt[kSplitWaves][kTWave];
-  __shared__ float s_gx[kSplitWaves][2][kTile];
+  __shared__ SplitScratch s_x;
   const int lane = threadIdx.x & (kWave - 1);
   const int w = threadIdx.x / kWave;
   const int m = lane & 15;
@@ -2308,84 +2238,80 @@ backward_split_kernel(const float* __restrict__ coordinates, const float* __rest
                                          blockIdx.x, w, m);
   }
   const float step_count = kLoss ? seed.step[0] : 0.0f;  // advanced below, as in backward_kernel
-  stage_parameters<kSplitWaves * kWave>(params, s_w, s_small, threadIdx.x);
+  const SmallLoads small = load_small<kSplitWaves * kWave>(params, threadIdx.x);
+  stage_operand_weights<kSplitWaves * kWave>(params, s_w, threadIdx.x);
+  store_small(s_small, threadIdx.x, small);
   __syncthreads();
   if (kLoss && blockIdx.x == 0 && threadIdx.x == 0) seed.step[0] = step_count + 1.0f;
 
-  const int rows_off = lane_rows(m, g) + 1088 * w;  // W[16 w + m][.] (forward operand)
-  const int cols_off = lane_cols(m, g) + 16 * w;    // W[.][16 w + m] (transposed operand)
-  const int t_read = m * kWRow + 4 * g;             // transposed reads: row m, points 4 s + g
-
-  const SplitScratch scratch{s_ht, s_x, s_zt, s_gx};
-  int phase = 0;  // alternates the s_x buffers
+  const u2 minus_one = minus_identity(m, g);
+  const int entry = operand_entry(m, g);
+  const u4* w_lane = s_w + entry;
+  const u4* w_t = s_w + transposed_entry(m, g);
   for (int slot = blockIdx.x; slot < slots; slot += gridDim.x) {
-    f4 dw[3][4];
+    f16 dw[3];
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) dw[l][nb] = zero4();
+      for (int r = 0; r < 16; ++r) dw[l][r] = 0.0f;
     }
-    // Per-lane sums: bias[l] of row 16 w + m (all lane groups), the others of row
-    // 16 w + 4 g + (m & 3).
-    float bias[3] = {0.f, 0.f, 0.f};
-    float g_w0x = 0.f, g_w0y = 0.f, g_b0 = 0.f, g_wout = 0.f, g_bout = 0.f;
-    float g_loss = 0.f, g_bloss = 0.f;
-
+    SplitSums sums{};
     if (slot != static_cast<int>(blockIdx.x)) {
       next = load_tile_inputs<kLoss, true>(coordinates, grad_output, grad_laplacian, batch, 0,
                                            seed, slot, w, m);
     }
-    for (int64_t tile = slot; tile < tiles; tile += slots) {
+    // Interior tiles, then (kLoss) boundary tiles.
+    const int64_t interior_end = kLoss ? std::min<int64_t>(tiles, seed.interior_tiles) : tiles;
+    int64_t tile = slot;
+    int round = 0;  // tiles of this slot so far (walk_sign)
+    for (; tile < interior_end; tile += slots, ++round) {
       keep_lds_reads_in_loop();
       const TileInputs in = next;
       if (tile + slots < tiles) {
         next = load_tile_inputs<kLoss, true>(coordinates, grad_output, grad_laplacian, batch, 0,
                                              seed, tile + slots, w, m);
       }
-      const bool on_boundary = kLoss && tile >= seed.interior_tiles;  // uniform per workgroup
-      const int64_t point = (on_boundary ? tile - seed.interior_tiles : tile) * kTile + m;
-      const bool active = point < (on_boundary ? seed.boundary_count : batch);
-      const float gu = kLoss ? 0.f : in.a, gl = kLoss ? 0.f : in.b, f = kLoss ? in.a : 0.f;
-
-      SplitSums sums{g_w0x, g_w0y, g_b0, g_wout, g_bout, g_loss, g_bloss};
-      split_tile<kLoss>(s_w, s_small, scratch, phase, w, g, m, rows_off, cols_off, t_read, in.x0,
-                        in.x1, gu, gl, f, active, on_boundary, point, grad_coordinates, seed, dw,
-                        bias, sums);
-      g_w0x = sums.w0x;
-      g_w0y = sums.w0y;
-      g_b0 = sums.b0;
-      g_wout = sums.wout;
-      g_bout = sums.bout;
-      g_loss = sums.loss;
-      g_bloss = sums.bloss;
+      const int64_t point = tile * kTile + m;
+      split_tile<4, kLoss>(w_lane, w_t, s_small, s_x, minus_one, w, g, m, in.x0, in.x1,
+                           kLoss ? 0.f : in.a, kLoss ? 0.f : in.b, kLoss ? in.a : 0.f, point < batch,
+                           walk_sign(slot, round), point, grad_coordinates, seed, dw, sums);
       deliver(next);
     }
-
-    // ---- this slot's partial row: each wave writes its own rows ----
-    float* row = partials + static_cast<int64_t>(slot) * kRowStride;
-    const int dw_lane = opaque((16 * w + 4 * g) * kHidden + m);
-#pragma unroll
-    for (int l = 0; l < 3; ++l) {
-      float* wrow = row + kHiddenBase + l * kHiddenStride;
-#pragma unroll
-      for (int nb = 0; nb < 4; ++nb) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) wrow[dw_lane + r * kHidden + 16 * nb] = 4.0f * dw[l][nb][r];
+    if (kLoss) {
+      for (; tile < tiles; tile += slots, ++round) {
+        keep_lds_reads_in_loop();
+        const TileInputs in = next;
+        if (tile + slots < tiles) {
+          next = load_tile_inputs<kLoss, true>(coordinates, grad_output, grad_laplacian, batch, 0,
+                                               seed, tile + slots, w, m);
+        }
+        const int64_t point = (tile - seed.interior_tiles) * kTile + m;
+        split_tile<1, kLoss>(w_lane, w_t, s_small, s_x, minus_one, w, g, m, in.x0, in.x1, 0.f, 0.f, 0.f,
+                             point < seed.boundary_count, walk_sign(slot, round), point, nullptr, seed, dw,
+                             sums);
+        deliver(next);
       }
-      if (g == 0) wrow[kHidden * kHidden + 16 * w + m] = kC * bias[l];
     }
+
+    // ---- this slot's partial row: each wave writes its own rows and blocks ----
+    float* row = partials + static_cast<int64_t>(slot) * kRowStride;
+    store_dw(row, w, lane, dw);
     if (m < 4) {
       const int n = 16 * w + 4 * g + m;
-      row[kInputs * n] = 2.0f * g_w0x;
-      row[kInputs * n + 1] = 2.0f * g_w0y;
-      row[kLayer0Bias + n] = kC * g_b0;
-      row[kOutputBase + n] = g_wout;
+      row[kInputs * n] = 2.0f * sums.w0x;
+      row[kInputs * n + 1] = 2.0f * sums.w0y;
+      row[kLayer0Bias + n] = kC * sums.b0;
+      row[kOutputBase + n] = sums.wout;
+#pragma unroll
+      for (int l = 0; l < 3; ++l) {
+        row[kHiddenBase + l * kHiddenStride + kHidden * kHidden + n] = kC * sums.bh[l];
+      }
     }
     if (w == 0 && lane == 0) {
-      row[kOutputBase + kHidden] = g_bout;
+      row[kOutputBase + kHidden] = sums.bout;
       if (kLoss) {
-        row[kLossColumn] = g_loss;
-        row[kLossColumn + 1] = g_bloss;
+        row[kLossColumn] = sums.loss;
+        row[kLossColumn + 1] = sums.bloss;
       }
     }
   }
@@ -2539,11 +2465,7 @@ __global__ void fill_zero_kernel(float* __restrict__ out, int64_t n) {
 // ---------------------------------------------------------------------------------------------
 // Host side.
 
-// Forward workgroup: 12 waves, 3 per SIMD (152 VGPRs each), about 1 % faster than 8 waves at 64K
-// and 256K points; a CU's 16 tiles per 64K still split 4 per SIMD. The saving forward runs 8
-// (launch_forward).
-constexpr int kFwdWaves = 12;
-constexpr int kSaveFwdWaves = 8;
+constexpr int kFwdWaves = 8;  // forward workgroup: 2 waves per SIMD
 constexpr int kSplitTilesPerCu = 2;  // forward_split_kernel up to this many tiles per CU
 
 thread_local char g_last_error[512] = "";
@@ -2725,7 +2647,7 @@ int noalloc_scratch(void** out) {
 // Backward call on a workspace of `workspace_bytes` bytes (checked by the caller).
 int launch_backward(const float* coordinates, const float* parameters, const float* grad_output,
                     const float* grad_laplacian, float* grad_parameters, float* grad_coordinates,
-                    void* workspace, int64_t batch, hipStream_t hs, const void* saved = nullptr);
+                    void* workspace, int64_t batch, hipStream_t hs);
 
 }  // namespace
 }  // namespace fhoad
@@ -2797,35 +2719,25 @@ extern "C" int fhoad_phase_clock_read(unsigned long long* out) {
 namespace fhoad {
 namespace {
 
-// The forward launch shared by fhoad_forward_laplacian and fhoad_forward_laplacian_saving
-// (kSave: the kernels also write the hidden-layer outputs to `saved`). batch > 0.
-template <bool kSave>
+// The forward launch shared by fhoad_forward_laplacian and fhoad_forward_laplacian_saving.
+// batch > 0.
 int launch_forward(const float* coordinates, const float* parameters, float* output,
-                   float* laplacian, void* saved, int64_t batch, hipStream_t hs) {
+                   float* laplacian, int64_t batch, hipStream_t hs) {
   int cus = 0;
   if (int st = current_device_cus(&cus)) return st;
   const int64_t tiles = (batch + kTile - 1) / kTile;
   const int grid = static_cast<int>(std::min<int64_t>(tiles, cus));
-  f4* saved_f4 = static_cast<f4*>(saved);
   // Below kSplitTilesPerCu tiles per CU the split kernel runs each tile on a CU's 4 SIMDs.
   // FUSED_HOAD_FWD_SPLIT=0 / 1 (experiment knob, read per call) forces either kernel.
   const char* split_env = std::getenv("FUSED_HOAD_FWD_SPLIT");
   const bool split = split_env ? std::atoi(split_env) != 0 : tiles <= kSplitTilesPerCu * cus;
   if (split) {
     const int split_grid = static_cast<int>(std::min<int64_t>(tiles, kSplitTilesPerCu * cus));
-    hipLaunchKernelGGL(forward_split_kernel<kSave>, dim3(split_grid), dim3(kSplitWaves * kWave), 0,
-                       hs, coordinates, parameters, output, laplacian, batch, tiles, saved_f4);
+    hipLaunchKernelGGL(forward_split_kernel, dim3(split_grid), dim3(kSplitWaves * kWave), 0, hs,
+                       coordinates, parameters, output, laplacian, batch, tiles);
     return check_launch("forward_split_kernel");
   }
   const int64_t whole = forward_whole_tiles(tiles, grid);
-  // Waves per workgroup: 12 for the forward; 8 for the saving forward, whose 48 KB of stores per
-  // tile slowed the 12-wave form more (64K points: 69 against 60 us; the plain forward 51.1
-  // against 51.6 us). FUSED_HOAD_FWD_WAVES=8 / 12 (experiment knob, read per call) forces either.
-  int waves = kSave ? kSaveFwdWaves : kFwdWaves;
-  if (const char* env = std::getenv("FUSED_HOAD_FWD_WAVES")) {
-    const int forced = std::atoi(env);
-    if (forced == 8 || forced == 12) waves = forced;
-  }
   // Polls per quad meeting before a split tile's wave gives up. FUSED_HOAD_QUAD_SPIN_LIMIT
   // (test knob, read per call) lowers it; 0 makes every meeting give up at once, so the tests can
   // check the timeout path (device status word, NaN outputs) with every kernel exiting normally.
@@ -2833,14 +2745,8 @@ int launch_forward(const float* coordinates, const float* parameters, float* out
   if (const char* env = std::getenv("FUSED_HOAD_QUAD_SPIN_LIMIT")) {
     spin_limit = static_cast<int>(std::min<long>(std::max<long>(std::atol(env), 0), kQuadSpinLimit));
   }
-  if (waves == 8) {
-    hipLaunchKernelGGL((forward_kernel<8, kSave>), dim3(grid), dim3(8 * kWave), 0, hs, coordinates,
-                       parameters, output, laplacian, batch, whole, tiles, saved_f4, spin_limit);
-  } else {
-    hipLaunchKernelGGL((forward_kernel<kFwdWaves, kSave>), dim3(grid), dim3(kFwdWaves * kWave), 0,
-                       hs, coordinates, parameters, output, laplacian, batch, whole, tiles,
-                       saved_f4, spin_limit);
-  }
+  hipLaunchKernelGGL((forward_kernel<kFwdWaves>), dim3(grid), dim3(kFwdWaves * kWave), 0, hs,
+                     coordinates, parameters, output, laplacian, batch, whole, tiles, spin_limit);
   return check_launch("forward_kernel");
 }
 
@@ -2856,9 +2762,13 @@ extern "C" int fhoad_forward_laplacian(const float* coordinates, const float* pa
   if (!coordinates || !parameters || !output || !laplacian) {
     return fail(FHOAD_ERROR_INVALID_VALUE, "null device pointer");
   }
-  return launch_forward<false>(coordinates, parameters, output, laplacian, nullptr, batch,
-                               static_cast<hipStream_t>(stream));
+  return launch_forward(coordinates, parameters, output, laplacian, batch,
+                        static_cast<hipStream_t>(stream));
 }
+
+// The saved-layer pair checks its buffer as it always did and runs the forward and the backward
+// that re-runs it (see fused_hoad.h).
+constexpr int64_t kSavedF4PerTile = 3 * 16 * kWave;  // the buffer: h1..h3 of a 16-point tile
 
 extern "C" size_t fhoad_saved_layers_size(int64_t batch) {
   if (batch <= 0) return 0;
@@ -2886,8 +2796,8 @@ extern "C" int fhoad_forward_laplacian_saving(const float* coordinates, const fl
                 needed);
   }
   if (int st = check_workspace_alignment(saved, "saved-layer buffer")) return st;
-  return launch_forward<true>(coordinates, parameters, output, laplacian, saved, batch,
-                              static_cast<hipStream_t>(stream));
+  return launch_forward(coordinates, parameters, output, laplacian, batch,
+                        static_cast<hipStream_t>(stream));
 }
 
 extern "C" size_t fhoad_backward_workspace_size(int64_t batch) {
@@ -2985,20 +2895,16 @@ extern "C" int fhoad_forward_laplacian_backward_saved(
   }
   if (int st = check_workspace_alignment(workspace)) return st;
   return launch_backward(coordinates, parameters, grad_output, grad_laplacian, grad_parameters,
-                         grad_coordinates, workspace, batch, hs, saved);
+                         grad_coordinates, workspace, batch, hs);
 }
 
 namespace fhoad {
 namespace {
 
-// saved: the saving forward's layer outputs for this batch (fhoad_saved_layers_size bytes), or
-// null to re-run the forward. Batches the small-batch kernel takes re-run it either way.
 int launch_backward(const float* coordinates, const float* parameters, const float* grad_output,
                     const float* grad_laplacian, float* grad_parameters, float* grad_coordinates,
-                    void* workspace, int64_t batch, hipStream_t hs, const void* saved) {
+                    void* workspace, int64_t batch, hipStream_t hs) {
   float* partials = static_cast<float*>(workspace);
-  const f4* saved_f4 = static_cast<const f4*>(saved);
-  const int64_t saved_tiles = (batch + kTile - 1) / kTile;
   int slots = 0, grid = 0;
   if (use_split_backward(batch, 0)) {
     const int64_t tiles = split_tiles(batch);
@@ -3013,26 +2919,14 @@ int launch_backward(const float* coordinates, const float* parameters, const flo
     if (int st = backward_grid(slots, &grid)) return st;
     const InteriorTiles it = interior_tiles_for(batch, slots);
     const dim3 block(kBwdWaves * kWave);
-    if (it.whole != it.total && saved) {
-      hipLaunchKernelGGL((backward_kernel<false, true, true>), dim3(grid), block, 0, hs,
-                         coordinates, parameters, grad_output, grad_laplacian, grad_coordinates,
-                         partials, batch, it.whole, it.total, slots, LossSeed{}, saved_f4,
-                         saved_tiles);
-    } else if (it.whole != it.total) {
-      hipLaunchKernelGGL((backward_kernel<false, true, false>), dim3(grid), block, 0, hs,
-                         coordinates, parameters, grad_output, grad_laplacian, grad_coordinates,
-                         partials, batch, it.whole, it.total, slots, LossSeed{}, nullptr,
-                         int64_t{0});
-    } else if (saved) {
-      hipLaunchKernelGGL((backward_kernel<false, false, true>), dim3(grid), block, 0, hs,
-                         coordinates, parameters, grad_output, grad_laplacian, grad_coordinates,
-                         partials, batch, it.whole, it.total, slots, LossSeed{}, saved_f4,
-                         saved_tiles);
+    if (it.whole != it.total) {
+      hipLaunchKernelGGL((backward_kernel<false, true>), dim3(grid), block, 0, hs, coordinates,
+                         parameters, grad_output, grad_laplacian, grad_coordinates, partials, batch,
+                         it.whole, it.total, slots, LossSeed{});
     } else {
-      hipLaunchKernelGGL((backward_kernel<false, false, false>), dim3(grid), block, 0, hs,
-                         coordinates, parameters, grad_output, grad_laplacian, grad_coordinates,
-                         partials, batch, it.whole, it.total, slots, LossSeed{}, nullptr,
-                         int64_t{0});
+      hipLaunchKernelGGL((backward_kernel<false, false>), dim3(grid), block, 0, hs, coordinates,
+                         parameters, grad_output, grad_laplacian, grad_coordinates, partials, batch,
+                         it.whole, it.total, slots, LossSeed{});
     }
     if (int st = check_launch("backward_kernel")) return st;
   }
@@ -3094,13 +2988,13 @@ extern "C" int fhoad_poisson_adam_step(const float* coordinates, const float* so
     if (int st = check_launch("backward_split_kernel")) return st;
   } else {
     if (it.whole != it.total) {
-      hipLaunchKernelGGL((backward_kernel<true, true, false>), dim3(grid), dim3(kBwdWaves * kWave),
+      hipLaunchKernelGGL((backward_kernel<true, true>), dim3(grid), dim3(kBwdWaves * kWave),
                          0, hs, coordinates, parameters, nullptr, nullptr, grad_coordinates,
-                         partials, batch, it.whole, tiles, slots, seed, nullptr, int64_t{0});
+                         partials, batch, it.whole, tiles, slots, seed);
     } else {
-      hipLaunchKernelGGL((backward_kernel<true, false, false>), dim3(grid), dim3(kBwdWaves * kWave),
+      hipLaunchKernelGGL((backward_kernel<true, false>), dim3(grid), dim3(kBwdWaves * kWave),
                          0, hs, coordinates, parameters, nullptr, nullptr, grad_coordinates,
-                         partials, batch, it.whole, tiles, slots, seed, nullptr, int64_t{0});
+                         partials, batch, it.whole, tiles, slots, seed);
     }
     if (int st = check_launch("backward_kernel")) return st;
   }

@@ -4,8 +4,8 @@ Fixed to the Poisson contract (2 -> 64x4 -> 1 tanh, FP32, on the GPU). The forwa
 kernel; the backward is the fused HIP kernel pair (default) or, when asked for by name, the
 reference's PyTorch recompute-and-differentiate path. Behaviour follows
 /root/reference/src/fused_hoad/backends/fused.py:24-138. One mode the reference does not have,
-``"saved"``, keeps the forward's hidden-layer outputs (3 KB per point) so that the HIP
-backward reads them instead of re-running the forward.
+``"saved"``, used to keep the forward's hidden-layer outputs for the backward; it runs ``"cuda"``
+now, which re-runs the forward in less time than the 3 KB per point take through memory.
 """
 
 from __future__ import annotations
@@ -32,8 +32,8 @@ from fused_hoad.parameters import (
 
 # Backward modes. Every "cuda*" name runs the same fused HIP backward (the reference's kernel
 # versions are kept as names only); "recompute" is the PyTorch reference backward; "saved" is
-# the HIP backward reading the layer outputs the forward kept (bitwise the same gradients as
-# "cuda", with 3 KB per point held from the forward to the backward).
+# another name of "cuda" (always bitwise the same gradients; keeping the layers took longer:
+# 64K points, forward and backward, 206 us with them against 155 us without).
 _CUDA_BACKWARD_VERSIONS = {
     "cuda": 6,
     "cuda_v1": 1,
@@ -44,6 +44,7 @@ _CUDA_BACKWARD_VERSIONS = {
 }
 BACKWARD_MODES = (*_CUDA_BACKWARD_VERSIONS, "recompute")  # the reference's names
 SAVED_MODE = "saved"
+_CUDA_BACKWARD_VERSIONS[SAVED_MODE] = 6
 _ACCEPTED_MODES = (*BACKWARD_MODES, SAVED_MODE)
 
 _cache: dict[str, object] = {}
@@ -59,29 +60,14 @@ class FusedForwardLaplacian(torch.autograd.Function):
     @staticmethod
     def forward(ctx, coordinates: Tensor, parameters: Tensor, version: int, backward: str):
         ctx.backward_mode = backward
-        if backward == SAVED_MODE:
-            output, laplacian, saved = load_extension()._forward_saving(coordinates, parameters, version)
-            ctx.save_for_backward(coordinates, parameters, saved)
-            return output, laplacian
         ctx.save_for_backward(coordinates, parameters)
         return fused_forward_laplacian(coordinates, parameters, version)
 
     @staticmethod
     def backward(ctx, grad_output: Tensor, grad_laplacian: Tensor):
-        coordinates, parameters, *saved = ctx.saved_tensors
+        coordinates, parameters = ctx.saved_tensors
         needs_coordinates, needs_parameters = ctx.needs_input_grad[:2]
         mode = ctx.backward_mode
-        if mode == SAVED_MODE:
-            grad_parameters, grad_coordinates = load_extension()._backward(
-                coordinates,
-                parameters,
-                grad_output.reshape(-1).contiguous(),
-                grad_laplacian.reshape(-1).contiguous(),
-                needs_coordinates,
-                6,
-                saved[0],
-            )
-            return grad_coordinates, grad_parameters if needs_parameters else None, None, None
         if mode in _CUDA_BACKWARD_VERSIONS:
             grad_parameters, grad_coordinates = fused_forward_laplacian_backward(
                 coordinates, parameters, grad_output, grad_laplacian, _CUDA_BACKWARD_VERSIONS[mode]
@@ -204,9 +190,8 @@ def fused_laplacian(
     """``(u, Laplacian u)`` of the fixed Poisson MLP from one gfx950 kernel launch.
 
     ``backward`` selects the gradient path when autograd is active: any ``"cuda*"`` mode runs
-    the fused HIP backward; ``"recompute"`` runs the PyTorch reference backward; ``"saved"``
-    runs the fused HIP backward on the layer outputs the forward kept (3 KB per point until the
-    backward), which spares it the forward re-run and gives bitwise the same gradients.
+    the fused HIP backward, and so does ``"saved"``; ``"recompute"`` runs the PyTorch reference
+    backward.
     """
     if backward not in _ACCEPTED_MODES:
         raise ValueError(f"backward must be one of {_ACCEPTED_MODES}")

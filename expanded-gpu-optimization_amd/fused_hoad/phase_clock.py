@@ -36,20 +36,17 @@ LIBRARY = PACKAGE_DIR / "libfused_hoad_hip.so"
 # Field order of ClockField in csrc/fused_hoad_kernels.hip.
 PHASES = [
     ("stage", "parameter staging (kernel start)"),
-    ("forward", "layer 0, hidden layers 1-2 forward (re-run)"),
-    ("layer3", "hidden layer 3 forward, loss and output seed, zbar3 staged"),
-    ("dw3", "dW3 (three staged passes)"),
-    ("adjoint3", "W3^T zbar3"),
-    ("dw2", "dW2"),
-    ("adjoint2", "W2^T zbar2, layer 0 rebuilt"),
-    ("dw1", "dW1"),
-    ("layer0", "W1^T zbar1, layer 0 adjoint, coordinate gradients"),
+    ("forward", "layer 0, hidden layers 1-3 forward (re-run)"),
+    ("seed", "loss and output seed, zbar3 split"),
+    ("layer3", "dW3, W3^T zbar3"),
+    ("layer2", "dW2, W2^T zbar2"),
+    ("layer1", "layer 0 rebuilt, dW1, W1^T zbar1, layer 0 adjoint, coordinate gradients"),
     ("rest", "16-point split tiles past the last whole round"),
     ("boundary", "boundary tiles"),
     ("partials", "partial row of the slot"),
 ]
-TILES, BOUNDARY_TILES, WALL_START, WALL_END = 12, 13, 14, 15
-FIELDS = 16
+TILES, BOUNDARY_TILES, WALL_START, WALL_END = 9, 10, 11, 12
+FIELDS = 13
 WALL_MHZ = 100.0  # s_memrealtime
 
 
