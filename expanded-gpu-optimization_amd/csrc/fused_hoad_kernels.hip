@@ -1062,19 +1062,25 @@ __device__ __forceinline__ f16 mfma_dw(u4 a, u4 b, f16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), c, 0, 0, 0);
 }
 
-// sum += A B^T over the operands' 16 points, the products smallest first.
+// sum[0] + sum[1] += A B^T over the operands' 16 points, the products smallest first in each. Two
+// accumulators in turn: a 32 x 32 product takes the matrix core 32 clocks but gives its result
+// after 64, so one chain of them runs at half rate (64K points: 123.1 -> 121.1 us per backward call).
 //
 // The matrix cores truncate as they accumulate, towards minus infinity, so the errors of many
 // additions have the same sign and do not cancel: adjoints and weight-gradient sums formed there
 // without more care were up to 4 times further from float64 than with float32 products (gradients
 // of 262,144 points whose contributions cancel). So every other tile of a slot, and every other
 // slot's first, runs its whole walk back on the negated upstream gradients (walk_sign) and its
-// sums are subtracted: the truncations of both halves cancel. And an accumulator holds one
-// component of one tile (64 points); the slot's sums are formed in float32, rounded to nearest.
-__device__ __forceinline__ f16 add_products(const DwOperand& a, const DwOperand& b, f16 sum) {
+// sums are subtracted: the truncations of both halves cancel. And an accumulator holds one tile (64
+// points); the slot's sums are formed in float32, rounded to nearest (add_sums).
+__device__ __forceinline__ void add_products(const DwOperand& a, const DwOperand& b, f16 (&sum)[2]) {
 #pragma unroll
-  for (int k = 0; k < kProducts; ++k) sum = mfma_dw(a.part[part_a(k)], b.part[part_b(k)], sum);
-  return sum;
+  for (int k = 0; k < kProducts; ++k) sum[k & 1] = mfma_dw(a.part[part_a(k)], b.part[part_b(k)], sum[k & 1]);
+}
+
+__device__ __forceinline__ void add_sums(f16& dw, float sign, const f16 (&sum)[2]) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) dw[r] = __builtin_fmaf(sign, sum[0][r] + sum[1][r], dw[r]);
 }
 
 __device__ __forceinline__ float walk_sign(int slot, int round) { return ((slot ^ round) & 1) ? -1.0f : 1.0f; }
@@ -1142,14 +1148,18 @@ __device__ __forceinline__ void tanh_jet_adjoint_h_seed(float v, float hj0, floa
 // own instruction stream: an MFMA takes 16 clocks (32 for the 32 x 32 form) of which its issue
 // takes 8.5, and the VALU can work in the rest. The tile is cut into scheduling regions
 // (region_end), each holding the MFMAs of one block and independent VALU work of the block before,
-// and interleave<n, k>() asks for n groups of one MFMA and k VALU instructions in the region.
+// and interleave<n, v, r, w>() asks for n groups of one MFMA, r LDS reads, w LDS writes and v VALU
+// instructions in the region (issued in one run, LDS instructions stall the wave behind the
+// workgroup's other three: 10 % of the time).
 __device__ __forceinline__ void region_end() { __builtin_amdgcn_sched_barrier(0); }
 
-template <int kMfmas, int kValu>
+template <int kMfmas, int kValu, int kReads = 0, int kWrites = 0>
 __device__ __forceinline__ void interleave() {
 #pragma unroll
   for (int i = 0; i < kMfmas; ++i) {
     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    if (kReads > 0) __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
+    if (kWrites > 0) __builtin_amdgcn_sched_group_barrier(0x200, kWrites, 0);
     __builtin_amdgcn_sched_group_barrier(0x002, kValu, 0);
   }
 }
@@ -1243,13 +1253,16 @@ __device__ __forceinline__ void forward_layer(const float* s_small, const u4* w_
 #pragma unroll
     for (int c = 1; c < 4; ++c) z[c] = zero4();
     w = lds_weights(mb < 3 ? w_layer : w_after, (mb + 1) & 3);
-    region_end();
 #pragma unroll
     for (int j = 0; j < 12; ++j) {
       product_step(j, cur, in, z);
       if (mb == 0 && j < 5) before(j);
       if (mb > 0) work.stage(j, minus_one, hout[mb - 1]);
-      interleave<4, 2>();
+      if (j == 0) {
+        interleave<4, 2, 2>();
+      } else {
+        interleave<4, 2>();
+      }
       region_end();
     }
     if (mb > 0 && kOperand) {
@@ -1264,10 +1277,30 @@ __device__ __forceinline__ void forward_layer(const float* s_small, const u4* w_
 // dW staging of a 64-point tile: one jet component of zbar and of h_prev, each wave's 16 points
 // as a set of entries (see DwOperand): 24 KB each.
 constexpr int kSetU4 = 2 * kParts * kWave;
+//
+// The slot's sums of hidden layers 2 and 3 lie beside it (16 KB each), each lane's 16 in four
+// 16-byte entries; those of layer 1 stay in registers (all three do during split tiles, whose
+// scratch overlays this one). In registers they were 32 of the ones that spilled to memory.
+constexpr int kLdsDw = 2;
 struct DwStage {
   u4 z[kBwdWaves][kSetU4];
   u4 h[kBwdWaves][kSetU4];
+  f4 dw[kLdsDw][4][kBwdWaves * kWave];
 };
+
+__device__ __forceinline__ void load_dw(const f4* p, f16& dw) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f4 x = p[i * kBwdWaves * kWave];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) dw[4 * i + r] = x[r];
+  }
+}
+
+__device__ __forceinline__ void keep_dw(f4* p, const f16& dw) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) p[i * kBwdWaves * kWave] = f4{dw[4 * i], dw[4 * i + 1], dw[4 * i + 2], dw[4 * i + 3]};
+}
 
 // One lane's pointers into the staging: its entries of its wave's sets, and its wave's operands
 // (half w >> 1 of zbar, half w & 1 of h_prev) in wave 0's set.
@@ -1276,18 +1309,12 @@ struct StagePointers {
   DwPointers ra, rb;
 };
 
-// The parts of half t of one component of a layer's output: blocks 2 t and 2 t + 1 (VALU only: it
-// runs between the 32 x 32 MFMAs, which leave the VALU 24 of their 32 clocks).
-__device__ __forceinline__ void split_half(const f4 (&h)[4][4], int c, int t, u4 (&part)[kParts]) {
+// Output block mb's parts of one component into the entries of its half.
+__device__ __forceinline__ void put_component(const u2 (&p)[kParts], int mb, u4 (&part)[2][kParts]) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    u2 p[kParts];
-    split4(h[2 * t + i][c], p);
-#pragma unroll
-    for (int s = 0; s < kParts; ++s) {
-      part[s][2 * i] = p[s][0];
-      part[s][2 * i + 1] = p[s][1];
-    }
+  for (int s = 0; s < kParts; ++s) {
+    part[mb >> 1][s][2 * (mb & 1)] = p[s][0];
+    part[mb >> 1][s][2 * (mb & 1) + 1] = p[s][1];
   }
 }
 
@@ -1300,16 +1327,19 @@ __device__ __forceinline__ void split_half(const f4 (&h)[4][4], int c, int t, u4
 // barrier (every wave has read component c) before the last set's MFMAs. w holds block 0's operands
 // on entry and w_after's on exit.
 template <typename Adjoint>
-__device__ __forceinline__ void backward_layer(const u4* w_t, const u4* w_after, const StagePointers& sp,
-                                               const JetOperand& zb, const f4 (&h)[4][4], float sign, f16& dw,
+__device__ __forceinline__ void backward_layer(const u4* w_t, const u4* w_after, const StagePointers& sp, u2 minus_one,
+                                               const JetOperand& zb, const f4 (&h)[4][4], f16 (&sum)[2],
                                                WeightOperand& w, Adjoint adjoint) {
-  f16 sum = zero16();
-  u4 part[2][kParts];
-  split_half(h, 0, 0, part[0]);
-  split_half(h, 0, 1, part[1]);
-  f4 done[4];  // the previous block's hbar
+  sum[0] = sum[1] = zero16();
+  u4 part[2][kParts];  // of the component to stage next
+  {
+    const f4 x[4] = {h[0][0], h[1][0], h[2][0], h[3][0]};
+    u2 p[4][kParts];
+    split_block(minus_one, x, p);
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
+    for (int mb = 0; mb < 4; ++mb) put_component(p[mb], mb, part);
+  }
+  auto stage = [&](int c) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
@@ -1318,7 +1348,12 @@ __device__ __forceinline__ void backward_layer(const u4* w_t, const u4* w_after,
         sp.wh[(t * kParts + s) * kWave] = part[t][s];
       }
     }
-    region_end();
+  };
+  stage(0);
+  region_end();
+  f4 done[4];  // the previous block's hbar
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
     f4 hb[4] = {zero4(), zero4(), zero4(), zero4()};
     DwOperand a, b;
     u4 next0[kParts];  // half 0 of the next block's weights
@@ -1328,20 +1363,18 @@ __device__ __forceinline__ void backward_layer(const u4* w_t, const u4* w_after,
         __syncthreads();  // component c is staged
         a = lds_dw_operand(sp.ra, 0);
         b = lds_dw_operand(sp.rb, 0);
-        lds_transposed_half(c < 3 ? w_t : w_after, (c + 1) & 3, 0, next0);
-        region_end();
       }
+      if (i == 3) lds_transposed_half(c < 3 ? w_t : w_after, (c + 1) & 3, 0, next0);
 #pragma unroll
       for (int j = 0; j < 3; ++j) hbar_step(3 * i + j, w, zb, hb);
-      if (c > 0) {
-        adjoint(c - 1, i, done);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) dw[4 * i + r] = __builtin_fmaf(sign, sum[4 * i + r], dw[4 * i + r]);
+      if (c > 0) adjoint(c - 1, i, done);
+      if (i < 2) {
+        interleave<12, 2>();
+      } else {
+        interleave<12, 2, 1>();
       }
-      interleave<12, 2>();
       region_end();
     }
-    sum = zero16();
 #pragma unroll
     for (int set = 0; set < kBwdWaves; ++set) {
       const DwOperand ca = a, cb = b;
@@ -1352,32 +1385,32 @@ __device__ __forceinline__ void backward_layer(const u4* w_t, const u4* w_after,
         __syncthreads();  // every wave has read component c
         lds_transposed_half(c < 3 ? w_t : w_after, (c + 1) & 3, 1, w.part[1]);
       }
-      region_end();
-      sum = add_products(ca, cb, sum);
+      add_products(ca, cb, sum);
       if (c < 3) {
-        u2 p[kParts];
-        split4(h[set][c + 1], p);
+        // The next component's split (VALU only: these MFMAs leave it 24 of their 32 clocks) between
+        // the first three sets' MFMAs, its staging behind the last set's.
 #pragma unroll
-        for (int s = 0; s < kParts; ++s) {
-          part[set >> 1][s][2 * (set & 1)] = p[s][0];
-          part[set >> 1][s][2 * (set & 1) + 1] = p[s][1];
+        for (int mb = 0; mb < 4; ++mb) {
+          if ((mb ? mb - 1 : 0) != set) continue;
+          u2 p[kParts];
+          split4(h[mb][c + 1], p);
+          put_component(p, mb, part);
         }
+        if (set == 3) stage(c + 1);
+      } else {
+        adjoint(3, set, hb);
       }
-      interleave<6, 4>();
+      if (set < 3) {
+        interleave<6, 4, 2>();
+      } else {
+        interleave<6, 4, 1, 2>();
+      }
       region_end();
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) done[i] = hb[i];
 #pragma unroll
     for (int s = 0; s < kParts; ++s) w.part[0][s] = next0[s];
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) adjoint(3, i, done);
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    float x = __builtin_fmaf(sign, sum[r], dw[r]);
-    park(x);
-    dw[r] = x;
   }
 }
 
@@ -1699,13 +1732,12 @@ __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, cons
       const Exchange& hx = layer == 1 ? sc.h1 : sc.h2;
       const DwPointers a = dw_pointers(&sc.z.part[w >> 1][0][0][0], m, g);
       const DwPointers b = dw_pointers(&hx.part[w & 1][0][0][0], m, g);
-      f16 sum = zero16();
+      f16 sum[2] = {zero16(), zero16()};
 #pragma unroll
       for (int c = 0; c < C; ++c) {
-        sum = add_products(lds_dw_operand(a, c * kParts * kWave), lds_dw_operand(b, c * kParts * kWave), sum);
+        add_products(lds_dw_operand(a, c * kParts * kWave), lds_dw_operand(b, c * kParts * kWave), sum);
       }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) dw[layer][r] = __builtin_fmaf(sign, sum[r], dw[layer][r]);
+      add_sums(dw[layer], sign, sum);
     }
     // hbar of this wave's rows of the layer below.
     get_components<C>(sc.z, entry, op);
@@ -1897,13 +1929,12 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
   sp.ra = dw_pointers(s_x.stage.z[0] + (w >> 1) * kParts * kWave, m, g);
   sp.rb = dw_pointers(s_x.stage.h[0] + (w & 1) * kParts * kWave, m, g);
 
+  f4* dw_lane = &s_x.stage.dw[0][0][threadIdx.x];  // this lane's sums of layers 2 and 3
+
   for (int slot = blockIdx.x; slot < slots; slot += gridDim.x) {
-    f16 dw[3];
-#pragma unroll
-    for (int l = 0; l < 3; ++l) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) dw[l][r] = 0.0f;
-    }
+    f16 dw[3] = {zero16(), zero16(), zero16()};
+    keep_dw(dw_lane, dw[1]);
+    keep_dw(dw_lane + 4 * kBwdWaves * kWave, dw[2]);
     // Point sums of this wave (lane = owned neuron), and of r^2 and u_b^2 (kLoss).
     float sum[kCombined] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     float sum_bout = 0.f, sum_loss = 0.f, sum_bloss = 0.f;
@@ -2028,7 +2059,8 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
       WeightOperand wt = lds_transposed_weights(w_t + 2 * kLayerU4, 0);
       auto walk = [&](int layer, const f4 (&h)[4][4], float& bias) {
         f4 z[4][4];
-        backward_layer(w_t + layer * kLayerU4, w_t + (layer - 1) * kLayerU4, sp, zb, h, sign, dw[layer], wt,
+        f16 sums[2];
+        backward_layer(w_t + layer * kLayerU4, w_t + (layer - 1) * kLayerU4, sp, minus_one, zb, h, sums, wt,
                        [&](int ib, int r, const f4 (&hb)[4]) {
                          float bv = hb[0][r], bj0 = hb[1][r], bj1 = hb[2][r], bl = hb[3][r];
                          tanh_jet_adjoint_h(h[ib][0][r], h[ib][1][r], h[ib][2][r], h[ib][3][r], bv, bj0,
@@ -2038,6 +2070,10 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
                          z[ib][2][r] = bj1;
                          z[ib][3][r] = bl;
                        });
+        f16 kept;
+        load_dw(dw_lane + (layer - 1) * 4 * kBwdWaves * kWave, kept);
+        add_sums(kept, sign, sums);
+        keep_dw(dw_lane + (layer - 1) * 4 * kBwdWaves * kWave, kept);
         float terms[16];
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb) {
@@ -2076,7 +2112,8 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
         }
         float gx0 = 0.f, gx1 = 0.f, tx[16], ty[16], tb[16];
         const float cx0 = kHalfC * x0, cx1 = kHalfC * x1;
-        backward_layer(w_t, w_t, sp, zb, h0, sign, dw[0], wt, [&](int ib, int r, const f4 (&hb)[4]) {
+        f16 sums[2];
+        backward_layer(w_t, w_t, sp, minus_one, zb, h0, sums, wt, [&](int ib, int r, const f4 (&hb)[4]) {
           const float* w0 = s_small + 16 * ib + 4 * g + r;
           float bv = hb[0][r], bj0 = hb[1][r], bj1 = hb[2][r], bl = hb[3][r];
           tanh_jet_adjoint_layer0(h0[ib][0][r], s0[ib][r], w0[kSmallWx], w0[kSmallWy], w0[kSmallQ0], bv, bj0,
@@ -2087,6 +2124,7 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
           ty[4 * ib + r] = __builtin_fmaf(bv, cx1, bj1);  // dW0[o][1] / 2
           tb[4 * ib + r] = bv;                            // db0[o] / c
         });
+        add_sums(dw[0], sign, sums);
         sum[0] += sign * row_reduce_scatter16(tx, m_pick);
         sum[1] += sign * row_reduce_scatter16(ty, m_pick);
         sum[2] += sign * row_reduce_scatter16(tb, m_pick);
@@ -2100,6 +2138,8 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
       clock.mark(kClockLayer1);
       clock.count(kClockTiles);
     }
+    load_dw(dw_lane, dw[1]);
+    load_dw(dw_lane + 4 * kBwdWaves * kWave, dw[2]);
     // A split tile's point sums into this wave's owned-neuron lanes (owned_neuron): the wave's rows
     // only; the point sums shared by the 4 waves from wave 0 alone.
     auto add_split = [&](const SplitSums& s, int m_pick) {
