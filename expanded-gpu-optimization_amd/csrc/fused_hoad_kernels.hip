@@ -414,15 +414,16 @@ __device__ __forceinline__ int operand_entry(int m, int g) { return 16 * g + (m 
 constexpr int kBlockU4 = 2 * kParts * kWave;  // u4 entries of one output block
 constexpr int kLayerU4 = 4 * kBlockU4;        // of one layer (24 KB)
 
-// One lane's operand of (layer, mb, t): 8 weights, loaded as two rows of four and split.
-__device__ __forceinline__ void load_weights8(const float* __restrict__ params, bool aligned, int layer,
-                                              int mb, int t, int lane, f4 (&w)[2]) {
+// One lane's operand of (layer, mb, t): 8 weights, loaded as two runs of four of a row and split.
+template <bool kAligned>
+__device__ __forceinline__ void load_weights8(const float* __restrict__ params, int layer, int mb, int t,
+                                              int lane, f4 (&w)[2]) {
   const float* p = params + kHiddenBase + layer * kHiddenStride + (16 * mb + (lane & 15)) * kHidden +
                    32 * t + 4 * (lane >> 4);
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
     const float* q = p + 16 * half;
-    w[half] = aligned ? *reinterpret_cast<const f4*>(q) : f4{q[0], q[1], q[2], q[3]};
+    w[half] = kAligned ? *reinterpret_cast<const f4*>(q) : f4{q[0], q[1], q[2], q[3]};
   }
 }
 
@@ -440,31 +441,36 @@ __device__ __forceinline__ void split_weights8(const f4 (&w)[2], u4 (&part)[kPar
 }
 
 // Staging: work item (l, mb, t, lane). A thread issues the loads of all its items before its
-// first LDS write.
+// first LDS write; one branch on the parameters' alignment holds them all (with a branch at each
+// load, each waited for the one before: 2.9 us of a gradient kernel's start).
 template <int kThreads>
 __device__ __forceinline__ void stage_operand_weights(const float* __restrict__ params, u4* s_wa,
                                                       int tid) {
   constexpr int kItems = 3 * 4 * 2 * kWave;  // (layer, mb, t, lane)
   constexpr int kPerThread = (kItems + kThreads - 1) / kThreads;
-  const bool aligned = (reinterpret_cast<uintptr_t>(params) & 15) == 0;
+  static_assert(kItems % kThreads == 0, "whole items per thread");
   f4 rows[kPerThread][2];
+  if ((reinterpret_cast<uintptr_t>(params) & 15) == 0) {
 #pragma unroll
-  for (int n = 0; n < kPerThread; ++n) {
-    const int item = tid + n * kThreads;
-    if (item < kItems) {
-      load_weights8(params, aligned, item >> 9, (item >> 7) & 3, (item >> 6) & 1, item & 63, rows[n]);
+    for (int n = 0; n < kPerThread; ++n) {
+      const int item = tid + n * kThreads;
+      load_weights8<true>(params, item >> 9, (item >> 7) & 3, (item >> 6) & 1, item & 63, rows[n]);
+    }
+  } else {
+#pragma unroll
+    for (int n = 0; n < kPerThread; ++n) {
+      const int item = tid + n * kThreads;
+      load_weights8<false>(params, item >> 9, (item >> 7) & 3, (item >> 6) & 1, item & 63, rows[n]);
     }
   }
 #pragma unroll
   for (int n = 0; n < kPerThread; ++n) {
     const int item = tid + n * kThreads;
-    if (item < kItems) {
-      u4 parts[kParts];
-      split_weights8(rows[n], parts);
+    u4 parts[kParts];
+    split_weights8(rows[n], parts);
 #pragma unroll
-      for (int s = 0; s < kParts; ++s) {
-        s_wa[((item >> 6) * kParts + s) * kWave + operand_entry(item & 15, (item >> 4) & 3)] = parts[s];
-      }
+    for (int s = 0; s < kParts; ++s) {
+      s_wa[((item >> 6) * kParts + s) * kWave + operand_entry(item & 15, (item >> 4) & 3)] = parts[s];
     }
   }
 }
@@ -894,12 +900,19 @@ forward_split_kernel(const float* __restrict__ coordinates, const float* __restr
   // L2-resident) instead of staging the whole matrix in LDS.
   WeightOperand wa[3];
   {
-    const bool aligned = (reinterpret_cast<uintptr_t>(params) & 15) == 0;
     f4 rows[3][2][2];
+    if ((reinterpret_cast<uintptr_t>(params) & 15) == 0) {
 #pragma unroll
-    for (int l = 0; l < 3; ++l) {
+      for (int l = 0; l < 3; ++l) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) load_weights8(params, aligned, l, w, t, lane, rows[l][t]);
+        for (int t = 0; t < 2; ++t) load_weights8<true>(params, l, w, t, lane, rows[l][t]);
+      }
+    } else {
+#pragma unroll
+      for (int l = 0; l < 3; ++l) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) load_weights8<false>(params, l, w, t, lane, rows[l][t]);
+      }
     }
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
@@ -1238,21 +1251,22 @@ struct BlockWork {
 // One hidden layer of the forward re-run (forward_kernel's chains): h_out in registers and, with
 // kOperand, as the next product's operand. Each block's work runs between the MFMAs of the next
 // block, block 3's between the next layer's first ones: before(j), j = 0..4, does the previous
-// layer's, and `work` leaves this layer's block 3. w holds block 0's operands on entry and those of
-// `w_after` on exit.
+// layer's, and `work` leaves this layer's block 3. w and bias hold block 0's operands on entry and
+// the next layer's (w_after) on exit.
 template <bool kOperand, typename Before>
 __device__ __forceinline__ void forward_layer(const float* s_small, const u4* w_layer, const u4* w_after,
                                               u2 minus_one, int layer, int g, const JetOperand& in,
-                                              f4 (&hout)[4][4], JetOperand& next, WeightOperand& w,
+                                              f4 (&hout)[4][4], JetOperand& next, WeightOperand& w, f4& bias,
                                               BlockWork<kOperand>& work, Before before) {
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb) {
     const WeightOperand cur = w;
     f4 z[4];
-    z[0] = lds4(s_small + kSmallBh + layer * kHidden + 16 * mb + 4 * g);
+    z[0] = bias;
 #pragma unroll
     for (int c = 1; c < 4; ++c) z[c] = zero4();
     w = lds_weights(mb < 3 ? w_layer : w_after, (mb + 1) & 3);
+    if (mb < 3 || kOperand) bias = lds4(s_small + kSmallBh + layer * kHidden + 16 * (mb + 1) + 4 * g);
 #pragma unroll
     for (int j = 0; j < 12; ++j) {
       product_step(j, cur, in, z);
@@ -1975,6 +1989,7 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
       {
         JetOperand a, b;
         WeightOperand wf = lds_weights(w_lane, 0);
+        f4 bias = lds4(s_small + kSmallBh + 4 * g);
         layer0_operand(s_small, minus_one, g, x0, x1, a);
         BlockWork<true> work;
         BlockWork<false> last;
@@ -1990,11 +2005,11 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
             park_block(out);
           }
         };
-        forward_layer<true>(s_small, w_lane, w_lane + kLayerU4, minus_one, 0, g, a, h1, b, wf, work,
+        forward_layer<true>(s_small, w_lane, w_lane + kLayerU4, minus_one, 0, g, a, h1, b, wf, bias, work,
                             [](int) {});
         forward_layer<true>(s_small, w_lane + kLayerU4, w_lane + 2 * kLayerU4, minus_one, 1, g, b, h2, a, wf,
-                            work, [&](int j) { finish(j, h1[3], b); });
-        forward_layer<false>(s_small, w_lane + 2 * kLayerU4, w_lane, minus_one, 2, g, a, h3, b, wf, last,
+                            bias, work, [&](int j) { finish(j, h1[3], b); });
+        forward_layer<false>(s_small, w_lane + 2 * kLayerU4, w_lane, minus_one, 2, g, a, h3, b, wf, bias, last,
                              [&](int j) { finish(j, h2[3], a); });
 #pragma unroll
         for (int j = 0; j < 5; ++j) last.stage(j, minus_one, h3[3]);
@@ -2113,16 +2128,16 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
         float gx0 = 0.f, gx1 = 0.f, tx[16], ty[16], tb[16];
         const float cx0 = kHalfC * x0, cx1 = kHalfC * x1;
         f16 sums[2];
+        Layer0Weights lw = layer0_weights(s_small, 0, g);  // of the block at hand, read a block ahead
         backward_layer(w_t, w_t, sp, minus_one, zb, h0, sums, wt, [&](int ib, int r, const f4 (&hb)[4]) {
-          const float* w0 = s_small + 16 * ib + 4 * g + r;
           float bv = hb[0][r], bj0 = hb[1][r], bj1 = hb[2][r], bl = hb[3][r];
-          tanh_jet_adjoint_layer0(h0[ib][0][r], s0[ib][r], w0[kSmallWx], w0[kSmallWy], w0[kSmallQ0], bv, bj0,
-                                  bj1, bl);
-          gx0 = __builtin_fmaf(w0[kSmallCwx], bv, gx0);
-          gx1 = __builtin_fmaf(w0[kSmallCwy], bv, gx1);
+          tanh_jet_adjoint_layer0(h0[ib][0][r], s0[ib][r], lw.wx[r], lw.wy[r], lw.q[r], bv, bj0, bj1, bl);
+          gx0 = __builtin_fmaf(lw.cwx[r], bv, gx0);
+          gx1 = __builtin_fmaf(lw.cwy[r], bv, gx1);
           tx[4 * ib + r] = __builtin_fmaf(bv, cx0, bj0);  // dW0[o][0] / 2
           ty[4 * ib + r] = __builtin_fmaf(bv, cx1, bj1);  // dW0[o][1] / 2
           tb[4 * ib + r] = bv;                            // db0[o] / c
+          if (r == 3 && ib < 3) lw = layer0_weights(s_small, ib + 1, g);
         });
         add_sums(dw[0], sign, sums);
         sum[0] += sign * row_reduce_scatter16(tx, m_pick);
