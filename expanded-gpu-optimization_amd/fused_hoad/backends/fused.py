@@ -211,6 +211,12 @@ def fused_laplacian(
                 return FlattenedFusedLaplacian.apply(coordinates, flat, version, *tensors)
         elif flat is not None:
             return fused_forward_laplacian(coordinates, flat, version)
+    else:
+        # Inference: a flattened model's buffer, without building the list of its parameters that
+        # the pack cache compares (a program that evaluates several models missed it on each call).
+        flat = flattened_poisson_parameters(model)
+        if flat is not None and not flat.requires_grad and not coordinates.requires_grad:
+            return fused_forward_laplacian(coordinates.contiguous(), flat, version)
     parameters = _packed_parameters(model)
     if parameters.requires_grad or coordinates.requires_grad:
         return FusedForwardLaplacian.apply(coordinates.contiguous(), parameters, version, backward)
