@@ -1518,7 +1518,11 @@ __device__ __forceinline__ void deliver(TileInputs& in) {
   in.b = opaque(in.b);
 }
 
-constexpr int kSplitBwdMaxTiles = 768;  // backward_split_kernel up to 768 16-point tiles
+// backward_split_kernel up to this many 16-point tiles, two per CU: its time goes up by a tile's with
+// every 256, backward_kernel's is one 64-point tile's up to 16,384 points. Fused step, split against
+// tiled: 4,096 points 23.9 against 32.7 us, 6,000 32.7 against 33.2, 8,192 34.1 against 33.7, 9,000
+// 41.9 against 34.2, 12,288 44.4 against 35.7.
+constexpr int kSplitBwdMaxTiles = 512;
 
 // Scratch of one 16-point tile whose rows are split over the workgroup's 4 waves: the layer
 // outputs h1, h2 and the adjoint as operands of all 64 rows (Exchange, 24 KB each; dW reads
@@ -1572,7 +1576,7 @@ __device__ __forceinline__ void get_components(const Exchange& x, int entry, Jet
 // the value one is exactly zero at every layer. The weight-gradient terms reduce to
 // zbar_v h_v^T, and the forward's J and L components feed nothing. A boundary tile therefore
 // runs the value channel only; the terms it skips are exact zeros.
-template <int kComponents, bool kLoss>
+template <int kComponents, bool kLoss, bool kHbarFirst>
 __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, const float* s_small,
                                            SplitScratch& sc, u2 minus_one, int w, int g, int m,
                                            float x0, float x1, float gu, float gl, float f,
@@ -1741,19 +1745,10 @@ __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, cons
       put_rows(sc.h2, own);
     }
     __syncthreads();
-    // dW += sum over (c, points) of zbar h_prev^T.
-    {
-      const Exchange& hx = layer == 1 ? sc.h1 : sc.h2;
-      const DwPointers a = dw_pointers(&sc.z.part[w >> 1][0][0][0], m, g);
-      const DwPointers b = dw_pointers(&hx.part[w & 1][0][0][0], m, g);
-      f16 sum[2] = {zero16(), zero16()};
-#pragma unroll
-      for (int c = 0; c < C; ++c) {
-        add_products(lds_dw_operand(a, c * kParts * kWave), lds_dw_operand(b, c * kParts * kWave), sum);
-      }
-      add_sums(dw[layer], sign, sum);
-    }
-    // hbar of this wave's rows of the layer below.
+    // hbar of this wave's rows of the layer below, before dW: the next adjoint waits for it alone, and
+    // its VALU work runs behind dW's MFMAs (kHbarFirst holds the compiler to it: backward call at
+    // 1,000 points 18.2 -> 17.1 us; in backward_kernel<false, true> it made the 64-point tiles spill,
+    // 50,021 points 93.7 -> 96.1 us).
     get_components<C>(sc.z, entry, op);
     const u4* wt = w_t + layer * kLayerU4 + (w >> 1) * kParts * kWave;
     WeightOperand a;
@@ -1770,6 +1765,19 @@ __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, cons
       }
     }
     product(a, op, zero4(), hb);
+    if (kHbarFirst) region_end();
+    // dW += sum over (c, points) of zbar h_prev^T.
+    {
+      const Exchange& hx = layer == 1 ? sc.h1 : sc.h2;
+      const DwPointers a = dw_pointers(&sc.z.part[w >> 1][0][0][0], m, g);
+      const DwPointers b = dw_pointers(&hx.part[w & 1][0][0][0], m, g);
+      f16 sum[2] = {zero16(), zero16()};
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        add_products(lds_dw_operand(a, c * kParts * kWave), lds_dw_operand(b, c * kParts * kWave), sum);
+      }
+      add_sums(dw[layer], sign, sum);
+    }
   }
 
   // ---- layer 0 for this wave's rows: dW0, db0 and this wave's part of grad_x ----
@@ -2189,7 +2197,7 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
         }
         const int64_t point = whole * kBwdTile + (tile - whole) * kTile + m;
         SplitSums s{};
-        split_tile<4, kLoss>(w_lane, w_t, s_small, s_x.split, minus_one, w, g, m_pick, in.x0, in.x1,
+        split_tile<4, kLoss, kLoss>(w_lane, w_t, s_small, s_x.split, minus_one, w, g, m_pick, in.x0, in.x1,
                              kLoss ? 0.f : in.a, kLoss ? 0.f : in.b, kLoss ? in.a : 0.f,
                              point < batch, walk_sign(slot, round), point, grad_coordinates, seed, dw, s);
         add_split(s, m_pick);
@@ -2209,7 +2217,7 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
         }
         const int64_t point = (tile - seed.interior_tiles) * kTile + m;
         SplitSums s{};
-        split_tile<1, kLoss>(w_lane, w_t, s_small, s_x.split, minus_one, w, g, m_pick, in.x0, in.x1, 0.f,
+        split_tile<1, kLoss, kLoss>(w_lane, w_t, s_small, s_x.split, minus_one, w, g, m_pick, in.x0, in.x1, 0.f,
                              0.f, 0.f, point < seed.boundary_count, walk_sign(slot, round), point, nullptr, seed, dw, s);
         add_split(s, m_pick);
         deliver(next);
@@ -2327,7 +2335,7 @@ backward_split_kernel(const float* __restrict__ coordinates, const float* __rest
                                              seed, tile + slots, w, m);
       }
       const int64_t point = tile * kTile + m;
-      split_tile<4, kLoss>(w_lane, w_t, s_small, s_x, minus_one, w, g, m, in.x0, in.x1,
+      split_tile<4, kLoss, true>(w_lane, w_t, s_small, s_x, minus_one, w, g, m, in.x0, in.x1,
                            kLoss ? 0.f : in.a, kLoss ? 0.f : in.b, kLoss ? in.a : 0.f, point < batch,
                            walk_sign(slot, round), point, grad_coordinates, seed, dw, sums);
       deliver(next);
@@ -2341,7 +2349,7 @@ backward_split_kernel(const float* __restrict__ coordinates, const float* __rest
                                                seed, tile + slots, w, m);
         }
         const int64_t point = (tile - seed.interior_tiles) * kTile + m;
-        split_tile<1, kLoss>(w_lane, w_t, s_small, s_x, minus_one, w, g, m, in.x0, in.x1, 0.f, 0.f, 0.f,
+        split_tile<1, kLoss, true>(w_lane, w_t, s_small, s_x, minus_one, w, g, m, in.x0, in.x1, 0.f, 0.f, 0.f,
                              point < seed.boundary_count, walk_sign(slot, round), point, nullptr, seed, dw,
                              sums);
         deliver(next);

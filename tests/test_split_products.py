@@ -24,7 +24,7 @@ BLOCKS = ((0, 128), (128, 192), (192, 4288), (4288, 4352), (4352, 8448), (8448, 
           (12608, 12672), (12672, 12736))
 
 
-@pytest.mark.parametrize("batch", [4096, 12289, 65536, 65537, 70001, 262144])
+@pytest.mark.parametrize("batch", [4096, 8192, 8193, 12289, 65536, 65537, 70001, 262144])
 @pytest.mark.parametrize("scale", [1.0, 1.5])
 def test_cancelling_gradients_are_as_close_as_float32(batch: int, scale: float) -> None:
     announce(f"cancelling gradients against float64, batch={batch}, weights x{scale}")
