@@ -66,7 +66,7 @@ constexpr int kTile = 16;     // points per wave tile (the MFMA N dimension)
 // Scale factors of the carried jet (see the header comment).
 constexpr float kC = -2.8853900817779268f;       // c = -2 log2(e)
 constexpr float kLambda = 1.4426950408889634f;   // lambda = log2(e)
-constexpr float kKappa = -0.96090602783640284f;  // -8 / c^2 (tanh_jet_adjoint_vs)
+constexpr float kKappa = -0.96090602783640284f;  // -8 / c^2 (tanh_jet_adjoint_layer0)
 constexpr float kHalfC = 0.5f * kC;              // c / 2 (layer-0 weight gradients)
 
 // Small parameter blocks in LDS (float offsets inside s_small), each [64] over neurons.
@@ -286,25 +286,9 @@ __device__ __forceinline__ void tanh_jet4(const f4 (&z)[4], f4 (&out)[4]) {
 // place. Evaluated as
 //   zbar_L' = s' Lbar',   zbar_v' = s' [vbar' + kappa v' (Jbar' . z'_J + Lbar' P) + zbar_L' q'],
 //   zbar_Jd' = s' Jbar_d' + 2 zbar_L' v' z'_Jd
-// (17 instructions per value).
-__device__ __forceinline__ void tanh_jet_adjoint_vs(float v, float s, float zj0, float zj1,
-                                                    float zl, float& bv, float& bj0, float& bj1,
-                                                    float& bl) {
-  const float q = __builtin_fmaf(zj0, zj0, zj1 * zj1);
-  const float dot = __builtin_fmaf(bj0, zj0, bj1 * zj1);
-  const float p = __builtin_fmaf(v, q, zl);
-  const float kv = kKappa * v;
-  const float bls = bl * s;
-  const float t = __builtin_fmaf(kv, __builtin_fmaf(bl, p, dot), bv);
-  const float nv = s * __builtin_fmaf(bls, q, t);
-  const float m2 = 2.0f * (bls * v);
-  bj0 = __builtin_fmaf(m2, zj0, s * bj0);
-  bj1 = __builtin_fmaf(m2, zj1, s * bj1);
-  bv = nv;
-  bl = bls;
-}
-
-// tanh_jet_adjoint_vs for layer 0, whose z_J are the W0 columns and z_L = 0: q = |z_J|^2 is
+//
+// Here for layer 0, whose z_J are the W0 columns and z_L = 0 (tanh_jet_adjoint_h is the hidden
+// layers' form): q = |z_J|^2 is
 // the per-neuron constant staged in kSmallQ0 (the same fma), and p = v q.
 __device__ __forceinline__ void tanh_jet_adjoint_layer0(float v, float s, float zj0, float zj1,
                                                         float q, float& bv, float& bj0,
@@ -527,12 +511,6 @@ __device__ __forceinline__ void layer0_block(const float* s_small, int mb, int g
   }
 }
 
-__device__ __forceinline__ void layer0_forward(const float* s_small, int g, float x0, float x1,
-                                               f4 (&h)[4][4]) {
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) layer0_block(s_small, mb, g, x0, x1, h[mb]);
-}
-
 // The small LDS parameters read per tile have loop-invariant addresses; left alone, the
 // compiler hoists those reads out of the tile loop and keeps ~100 values live in registers for
 // the whole kernel. An empty asm statement with a memory clobber at the top of each tile keeps
@@ -617,19 +595,24 @@ __device__ __forceinline__ float row_reduce_scatter16(const float (&v)[16], int 
 // ---------------------------------------------------------------------------------------------
 // Forward kernel (replaces fused_forward_laplacian_tiled_kernel<2>,
 // /root/reference/csrc/fused_residual.cu:157-295). A grid of at most one workgroup per CU
-// stages the weights once, then every wave walks 16-point tiles: tile t < whole goes to
-// workgroup t % grid, wave (t / grid) % kWaves, so small batches still spread over all CUs.
+// stages the weights once, then its 8 waves (two per SIMD, 256 registers each) run 16-point tiles:
+// tiles blockIdx.x + k grid below `whole`, k from a counter in LDS.
 //
-// `whole` is a multiple of 4 x grid (one tile per SIMD per round), so every SIMD runs the same
-// number of whole tiles. The tiles past the last whole round (`split` tiles, fewer than one per
-// SIMD) would each add a whole tile's time to the SIMD that got it; instead, the last four
-// waves of each workgroup (one per SIMD, the ones with the fewest whole tiles) run them with a
+// `whole` is a multiple of 4 x grid (one tile per SIMD per round). The tiles past the last whole
+// round (`split` tiles, fewer than one per SIMD) would each add a whole tile's time to the SIMD that
+// got it; instead, the last four waves of each workgroup (one per SIMD) run them with a
 // 16-point tile's rows split between them, forward_split_kernel's decomposition: wave q
-// computes rows 16 q .. 16 q + 15 of every layer (64 MFMAs per layer instead of 256) and the
-// layer outputs go to the other three through LDS. The four meet at an LDS counter
+// computes rows 16 q .. 16 q + 15 of every layer (a quarter of the MFMAs) and the
+// layer outputs go to the other three through LDS (20,011 points: 15.6 us with whole tiles alone,
+// 12.3 with split ones). The four meet at an LDS counter
 // (quad_sync), not at s_barrier, which would wait for the workgroup's waves still on whole
 // tiles. A split tile's chains are a whole tile's accumulators (mb = q, c) with the same
 // operands in the same order, so both paths give bitwise the same results.
+//
+// A tile is 672 MFMAs (10.8K clocks of the matrix core) and 1,070 VALU instructions; with both
+// waves of a SIMD on tiles it takes about 13.6K clocks, issue-bound, at a shader clock that power
+// holds at 2.1 GHz (zero data runs at 2.4 GHz, 18 % faster). 1,000,003 points 738 -> 400 us against
+// the same kernel on v_mfma_f32_16x16x4f32, 65,536 points 51.0 -> 29.0.
 constexpr int kQuadSpinLimit = 1 << 24;  // about 0.5 s of s_sleep(1); never reached by a whole quad
 
 // Device status word, one per GPU: bit kStatusQuadTimeout is set when a quad meeting gave up
@@ -985,13 +968,19 @@ forward_split_kernel(const float* __restrict__ coordinates, const float* __restr
 //      re-evaluated), and dW += zbar h_prev^T; finally layer 0 in closed form;
 //   3. dW contracts over the points of all 4 waves: zbar and h_prev go through LDS one jet
 //      component at a time, split into bf16 parts, and wave w owns the 32 x 32 block
-//      (w >> 1, w & 1) of every dW. Bias, W0, b0 and w_out gradients are summed over each wave's
+//      (w >> 1, w & 1) of every dW (with it the waves read 96 KB of operands per layer each; a
+//      wave's 16 rows would take 120). Bias, W0, b0 and w_out gradients are summed over each wave's
 //      points in registers (row_reduce_scatter16) and over the 4 waves once per slot.
 // Every hidden product runs on the bf16 matrix cores with split operands (see split_pair).
-// Weight gradients accumulate in registers across the tiles of a "slot": slot s takes the
+// Weight gradients accumulate across the tiles of a "slot": slot s takes the
 // workgroup tiles s, s + slots, s + 2 slots, ... in that order and writes one partial row.
 // A second kernel sums the rows in a fixed tree. The slot count depends only on the batch,
 // so the result does not depend on the grid size. No float atomics anywhere.
+//
+// A tile is 1,656 MFMAs (31K clocks of a SIMD's matrix core) and about 4,700 VALU instructions and
+// takes 55K clocks: one wave per SIMD, bound by its instruction issue and the stalls between
+// dependent instructions. Registers (512, all used) leave no room for a second wave. Backward call
+// at 65,536 points 166.8 -> 107.6 us against v_mfma_f32_16x16x4f32, 262,144 points 638 -> 384.
 constexpr int kBwdWaves = 4;
 constexpr int kBwdTile = kBwdWaves * kTile;  // 64 points
 constexpr int kMaxSlots = 256;
@@ -1109,7 +1098,7 @@ __device__ __forceinline__ int owned_neuron(int m, int g) { return 16 * (m >> 2)
 
 // ---- the interior tiles of backward_kernel: the walk back from each layer's tanh-jet output ----
 //
-// The adjoint of the tanh jet (tanh_jet_adjoint_vs) needs s', z'_J and P = z'_L + v' q' only
+// The adjoint of the tanh jet (tanh_jet_adjoint_layer0) needs s', z'_J and P = z'_L + v' q' only
 // in the products the jet's output already holds: h' = (v', s' z'_J0, s' z'_J1, s' P), so
 // s' z'_J = h'_J, s' P = h'_L and s'^2 q' = |h'_J|^2. With s' from v' alone,
 //   s' = 1/4 + (kappa / 2) v'^2      (v' = (c / 4) tanh z_v, kappa = -8 / c^2: (1 - tanh^2) / 4),
