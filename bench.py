@@ -15,8 +15,8 @@ built), ``train_step_autograd_graphed_ms`` that drop-in step captured whole in a
 (the reference's "whole step CUDA-graph captured" row), and
 ``train_step_autograd_graphed_fused_adam_ms`` the same with ``torch.optim.Adam(fused=True)``
 (``..._saved_ms``: also with ``backward="saved"``). ``saving_forward_ms`` and
-``saved_backward_call_ms`` time the opt-in saved-layer pair (the forward keeps the hidden
-layers, 3 KB per point; the backward reads them instead of re-running the forward).
+``saved_backward_call_ms`` time the saved-layer pair (the plain forward and backward, with the
+pair's buffer of 3 KB per point checked between them).
 ``train_step_no_coordinate_grad_ms`` is the fused step without the coordinate gradient, a
 labelled variant only.
 
@@ -358,9 +358,8 @@ def main() -> None:
         log(f"backward call {args.train_points} pts: {bwd_ms * 1e3:.1f} us (GPU events over the calls)")
         return
 
-    # ---- the saved-layer pair (opt-in "saved" mode): a forward that keeps the hidden layers
-    # (3 KB per point) and a backward that reads them instead of re-running the forward. Checked
-    # bitwise against the pair above first; timed the same way, each call alone.
+    # ---- the saved-layer pair: the plain forward and backward with the pair's buffer between them.
+    # Checked bitwise against the pair above first; timed the same way, each call alone.
     ext = load_extension()
     gu_flat, gl_flat = gu.reshape(-1).contiguous(), gl.reshape(-1).contiguous()
     ref_u, ref_lap = fused_forward_laplacian(x_train, params)
@@ -479,7 +478,7 @@ def main() -> None:
     autograd_graph_ms, autograd_graph_note = checked_graph_timing(False)
     # labelled variant: the same with torch.optim.Adam(fused=True) (one optimizer kernel)
     autograd_graph_fused_ms, autograd_graph_fused_note = checked_graph_timing(True)
-    # labelled variant: the same with backward="saved" (the forward keeps 3 KB per point)
+    # labelled variant: the same with backward="saved" (another name of "cuda")
     autograd_graph_saved_ms, autograd_graph_saved_note = checked_graph_timing(True, "saved")
     for label, ms, note in (("foreach Adam", autograd_graph_ms, autograd_graph_note),
                             ("Adam(fused=True)", autograd_graph_fused_ms, autograd_graph_fused_note),

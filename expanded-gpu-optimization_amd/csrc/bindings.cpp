@@ -402,7 +402,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, module) {
              pybind11::arg("backward_version"), pybind11::arg("save_layers"),
              pybind11::arg("parameters"));
   module.def("_forward_saving", &forward_saving,
-             "Forward that also keeps the hidden layers' outputs for _backward(saved=...)",
+             "Forward with the saved-layer pair's buffer for _backward(saved=...)",
              pybind11::arg("coordinates"), pybind11::arg("parameters"),
              pybind11::arg("version") = 2);
   module.def("fused_forward_laplacian", &fused_forward_laplacian,

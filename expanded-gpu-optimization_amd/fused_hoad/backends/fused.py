@@ -211,7 +211,7 @@ def fused_laplacian(
                 return FlattenedFusedLaplacian.apply(coordinates, flat, version, *tensors)
         elif flat is not None:
             return fused_forward_laplacian(coordinates, flat, version)
-    else:
+    elif "_fused_hoad_packed" in model.__dict__:
         # Inference: a flattened model's buffer, without building the list of its parameters that
         # the pack cache compares (a program that evaluates several models missed it on each call).
         flat = flattened_poisson_parameters(model)
