@@ -1736,7 +1736,7 @@ __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, cons
     __syncthreads();
     // hbar of this wave's rows of the layer below, before dW: the next adjoint waits for it alone, and
     // its VALU work runs behind dW's MFMAs (kHbarFirst holds the compiler to it: backward call at
-    // 1,000 points 18.2 -> 17.1 us; in backward_kernel<false, true> it made the 64-point tiles spill,
+    // 1,000 points 18.2 -> 17.1 us; in backward_kernel<false, true, false> it made the 64-point tiles spill,
     // 50,021 points 93.7 -> 96.1 us).
     get_components<C>(sc.z, entry, op);
     const u4* wt = w_t + layer * kLayerU4 + (w >> 1) * kParts * kWave;
@@ -1893,12 +1893,18 @@ struct PhaseClock {
 //
 // kLoss: grad_output and grad_laplacian are unused and the seed comes from `seed` (above);
 // grad_coordinates may be null.
-template <bool kLoss, bool kRest>
+//
+// kBoundary: with boundary tiles in it, the fused step's kernel spills more registers in its 64-point
+// tiles (step of 16,384 points 39.1 -> 37.4 us without them, 65,536 109.3 -> 106.6, 262,144 400 ->
+// 395), so steps of whole rounds without boundary points run a form without; with a rest of split
+// tiles the form without spills more (50,021 points 93.5 -> 95.9), so that one always has them.
+template <bool kLoss, bool kRest, bool kBoundary>
 __global__ void __launch_bounds__(kBwdWaves * kWave, 1)
 backward_kernel(const float* __restrict__ coordinates, const float* __restrict__ params,
                 const float* __restrict__ grad_output, const float* __restrict__ grad_laplacian,
                 float* __restrict__ grad_coordinates, float* __restrict__ partials,
                 int64_t batch, int64_t whole, int64_t tiles, int slots, LossSeed seed) {
+  static_assert(kLoss || !kBoundary, "boundary points belong to the fused step's loss");
   constexpr int kCombined = 7;  // point sums combined over the waves: w0x, w0y, b0, wout, bh[3]
   union Scratch {
     DwStage stage;
@@ -2194,7 +2200,7 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
       }
       clock.mark(kClockRest);
     }
-    if (kLoss && tile < tiles) {  // boundary tiles (uniform per workgroup)
+    if (kBoundary && tile < tiles) {  // boundary tiles (uniform per workgroup)
       __syncthreads();
       for (; tile < tiles; tile += slots, ++round) {
         keep_lds_reads_in_loop();
@@ -2972,11 +2978,11 @@ int launch_backward(const float* coordinates, const float* parameters, const flo
     const InteriorTiles it = interior_tiles_for(batch, slots);
     const dim3 block(kBwdWaves * kWave);
     if (it.whole != it.total) {
-      hipLaunchKernelGGL((backward_kernel<false, true>), dim3(grid), block, 0, hs, coordinates,
+      hipLaunchKernelGGL((backward_kernel<false, true, false>), dim3(grid), block, 0, hs, coordinates,
                          parameters, grad_output, grad_laplacian, grad_coordinates, partials, batch,
                          it.whole, it.total, slots, LossSeed{});
     } else {
-      hipLaunchKernelGGL((backward_kernel<false, false>), dim3(grid), block, 0, hs, coordinates,
+      hipLaunchKernelGGL((backward_kernel<false, false, false>), dim3(grid), block, 0, hs, coordinates,
                          parameters, grad_output, grad_laplacian, grad_coordinates, partials, batch,
                          it.whole, it.total, slots, LossSeed{});
     }
@@ -3040,11 +3046,15 @@ extern "C" int fhoad_poisson_adam_step(const float* coordinates, const float* so
     if (int st = check_launch("backward_split_kernel")) return st;
   } else {
     if (it.whole != it.total) {
-      hipLaunchKernelGGL((backward_kernel<true, true>), dim3(grid), dim3(kBwdWaves * kWave),
+      hipLaunchKernelGGL((backward_kernel<true, true, true>), dim3(grid), dim3(kBwdWaves * kWave),
+                         0, hs, coordinates, parameters, nullptr, nullptr, grad_coordinates,
+                         partials, batch, it.whole, tiles, slots, seed);
+    } else if (boundary_count > 0) {
+      hipLaunchKernelGGL((backward_kernel<true, false, true>), dim3(grid), dim3(kBwdWaves * kWave),
                          0, hs, coordinates, parameters, nullptr, nullptr, grad_coordinates,
                          partials, batch, it.whole, tiles, slots, seed);
     } else {
-      hipLaunchKernelGGL((backward_kernel<true, false>), dim3(grid), dim3(kBwdWaves * kWave),
+      hipLaunchKernelGGL((backward_kernel<true, false, false>), dim3(grid), dim3(kBwdWaves * kWave),
                          0, hs, coordinates, parameters, nullptr, nullptr, grad_coordinates,
                          partials, batch, it.whole, tiles, slots, seed);
     }
