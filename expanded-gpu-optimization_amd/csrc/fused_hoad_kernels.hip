@@ -240,29 +240,31 @@ __device__ __forceinline__ void block_product(const WeightOperand& w, const JetO
 // and s = (1 - tanh^2 z_v) / 4. With t = exp(-2 z_v) = exp2(zv) and u = 1 / (1 + t):
 //   tanh z_v = 2 u - 1,   1 - tanh^2 z_v = 4 u (1 - u),
 // so v = fma(u, c / 2, -c / 4) and s = fma(-u, u, u): 3 VALU + 2 transcendental instructions
-// (v_exp_f32, v_rcp_f32) per value. t overflows to +inf for z_v < -44 (u = 0: tanh = -1,
+// (v_exp_f32, v_rcp_f32) per value (tanh_value, tanh_slope). t overflows to +inf for z_v < -44 (u = 0: tanh = -1,
 // s = 0) and flushes to 0 for z_v > 44 (u = 1: tanh = 1, s = 0). Near tanh = +1, s carries the
 // absolute rounding of u (about 6e-8), as 1 - a^2 does.
 // The four values go in stages: the four exp2, then the four rcp, then the rest (each value's
 // chain is serial).
-__device__ __forceinline__ void tanh_scaled4(const f4 zv, f4& v, f4& s) {
-  f4 u;
+__device__ __forceinline__ float tanh_value(float u) { return __builtin_fmaf(u, 0.5f * kC, -0.25f * kC); }
+__device__ __forceinline__ float tanh_slope(float u) { return __builtin_fmaf(-u, u, u); }
+
+__device__ __forceinline__ void tanh_scaled4(const f4 zv, f4& u, f4& v, f4& s) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) u[r] = __builtin_amdgcn_exp2f(zv[r]);
 #pragma unroll
   for (int r = 0; r < 4; ++r) u[r] = __builtin_amdgcn_rcpf(u[r] + 1.0f);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    v[r] = __builtin_fmaf(u[r], 0.5f * kC, -0.25f * kC);
-    s[r] = __builtin_fmaf(-u[r], u[r], u[r]);
+    v[r] = tanh_value(u[r]);
+    s[r] = tanh_slope(u[r]);
   }
 }
 
 // tanh_jet of four values (component vectors z[c][r] of one accumulator row block), the tanh
-// four at a time (tanh_scaled4): out[c][r] is the scaled output jet.
-__device__ __forceinline__ void tanh_jet4(const f4 (&z)[4], f4 (&out)[4]) {
+// four at a time (tanh_scaled4): out[c][r] is the scaled output jet, u[r] tanh_scaled4's.
+__device__ __forceinline__ void tanh_jet4(const f4 (&z)[4], f4 (&out)[4], f4& u) {
   f4 v, sl;
-  tanh_scaled4(z[0], v, sl);
+  tanh_scaled4(z[0], u, v, sl);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const float q = __builtin_fmaf(z[1][r], z[1][r], z[2][r] * z[2][r]);
@@ -271,6 +273,11 @@ __device__ __forceinline__ void tanh_jet4(const f4 (&z)[4], f4 (&out)[4]) {
     out[2][r] = sl[r] * z[2][r];
     out[3][r] = sl[r] * __builtin_fmaf(v[r], q, z[3][r]);
   }
+}
+
+__device__ __forceinline__ void tanh_jet4(const f4 (&z)[4], f4 (&out)[4]) {
+  f4 u;
+  tanh_jet4(z, out, u);
 }
 
 // Adjoint of the tanh jet (tanh_jet4, per value) in the scaled variables (the adjoint of a
@@ -498,10 +505,10 @@ __device__ __forceinline__ float layer0_zv(const Layer0Weights& w, int r, float 
 __device__ __forceinline__ void layer0_block(const float* s_small, int mb, int g, float x0,
                                              float x1, f4 (&h)[4]) {
   const Layer0Weights w = layer0_weights(s_small, mb, g);
-  f4 zv, v, s;
+  f4 zv, u, v, s;
 #pragma unroll
   for (int r = 0; r < 4; ++r) zv[r] = layer0_zv(w, r, x0, x1);
-  tanh_scaled4(zv, v, s);
+  tanh_scaled4(zv, u, v, s);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     h[0][r] = v[r];
@@ -1100,22 +1107,19 @@ __device__ __forceinline__ int owned_neuron(int m, int g) { return 16 * (m >> 2)
 //
 // The adjoint of the tanh jet (tanh_jet_adjoint_layer0) needs s', z'_J and P = z'_L + v' q' only
 // in the products the jet's output already holds: h' = (v', s' z'_J0, s' z'_J1, s' P), so
-// s' z'_J = h'_J, s' P = h'_L and s'^2 q' = |h'_J|^2. With s' from v' alone,
-//   s' = 1/4 + (kappa / 2) v'^2      (v' = (c / 4) tanh z_v, kappa = -8 / c^2: (1 - tanh^2) / 4),
-// the adjoint is
+// s' z'_J = h'_J, s' P = h'_L and s'^2 q' = |h'_J|^2. The adjoint is
 //   zbar_L' = s' Lbar',   zbar_Jd' = s' Jbar_d' + 2 Lbar' v' h'_Jd,
 //   zbar_v' = s' vbar' + kappa v' (Jbar' . h'_J + Lbar' h'_L) + Lbar' |h'_J|^2
 // (18 instructions per value). A tile therefore keeps each hidden layer's output h (which the
 // forward re-run produces anyway, and which the weight gradient of the layer above needs) and
-// evaluates no tanh in the walk back. Near |tanh| = 1, s' carries an absolute rounding of about
-// 3e-8, as 1 - a^2 does in the reference (/root/reference/csrc/fused_backward.cu:65-89).
-constexpr float kHalfKappa = 0.5f * kKappa;
-
-__device__ __forceinline__ void tanh_jet_adjoint_h(float v, float hj0, float hj1, float hl,
+// evaluates no tanh in the walk back. Of the value component it keeps tanh_scaled4's u instead of v':
+// each of v' and s' is one fma of u (tanh_value, tanh_slope), and s' = u - u^2 is relatively exact
+// where tanh nears -1, while s' from v' (1/4 + (kappa / 2) v'^2) carries an absolute rounding of 3e-8
+// there, 4 % of s' at z = -7.
+__device__ __forceinline__ void tanh_jet_adjoint_h(float u, float hj0, float hj1, float hl,
                                                    float& bv, float& bj0, float& bj1, float& bl) {
-  const float hk = kHalfKappa * v;
-  const float s = __builtin_fmaf(hk, v, 0.25f);
-  const float kv = hk + hk;
+  const float v = tanh_value(u), s = tanh_slope(u);
+  const float kv = kKappa * v;
   const float lv2 = bl * (v + v);
   const float dot = __builtin_fmaf(bj0, hj0, bj1 * hj1);
   const float q = __builtin_fmaf(hj0, hj0, hj1 * hj1);
@@ -1130,12 +1134,11 @@ __device__ __forceinline__ void tanh_jet_adjoint_h(float v, float hj0, float hj1
 // tanh_jet_adjoint_h for the output layer's seed: Jbar' = 0 and, with kZeroV (interior points
 // of the fused step), vbar' = 0; only operations on those zeros are dropped.
 template <bool kZeroV>
-__device__ __forceinline__ void tanh_jet_adjoint_h_seed(float v, float hj0, float hj1, float hl,
+__device__ __forceinline__ void tanh_jet_adjoint_h_seed(float u, float hj0, float hj1, float hl,
                                                         float& bv, float& bj0, float& bj1,
                                                         float& bl) {
-  const float hk = kHalfKappa * v;
-  const float s = __builtin_fmaf(hk, v, 0.25f);
-  const float kv = hk + hk;
+  const float v = tanh_value(u), s = tanh_slope(u);
+  const float kv = kKappa * v;
   const float lv2 = bl * (v + v);
   const float q = __builtin_fmaf(hj0, hj0, hj1 * hj1);
   const float t = bl * hl;
@@ -1182,8 +1185,9 @@ __device__ __forceinline__ void hbar_step(int j, const WeightOperand& w, const J
 }
 
 // The work on an output block after its product, in twelve stages to run one per step of the next
-// block's: the tanh jet (tanh_jet4) and, with kOperand, the split into the next operand
-// (split_block), whose remainders have a step or two to come out of the matrix cores.
+// block's: the tanh jet (tanh_jet4; out[0] keeps u, see tanh_jet_adjoint_h) and, with kOperand, the
+// split into the next operand (split_block), whose remainders have a step or two to come out of the
+// matrix cores.
 template <bool kOperand>
 struct BlockWork {
   f4 z[4], v, s, q;
@@ -1201,9 +1205,10 @@ struct BlockWork {
     } else if (j == 2) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        s[r] = __builtin_fmaf(-v[r], v[r], v[r]);
-        out[0][r] = __builtin_fmaf(v[r], 0.5f * kC, -0.25f * kC);
+        s[r] = tanh_slope(v[r]);
+        z[0][r] = tanh_value(v[r]);
       }
+      out[0] = v;
     } else if (j == 3) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -1212,9 +1217,9 @@ struct BlockWork {
       }
     } else if (j == 4) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) out[3][r] = s[r] * __builtin_fmaf(out[0][r], q[r], z[3][r]);
+      for (int r = 0; r < 4; ++r) out[3][r] = s[r] * __builtin_fmaf(z[0][r], q[r], z[3][r]);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) z[c] = out[c];
+      for (int c = 1; c < 4; ++c) z[c] = out[c];
     } else if (kOperand && (j == 5 || j == 8 || j == 11)) {
       const int p = (j - 5) / 3;
 #pragma unroll
@@ -1336,7 +1341,12 @@ __device__ __forceinline__ void backward_layer(const u4* w_t, const u4* w_after,
   sum[0] = sum[1] = zero16();
   u4 part[2][kParts];  // of the component to stage next
   {
-    const f4 x[4] = {h[0][0], h[1][0], h[2][0], h[3][0]};
+    f4 x[4];  // v' from the kept u
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[mb][r] = tanh_value(h[mb][0][r]);
+    }
     u2 p[4][kParts];
     split_block(minus_one, x, p);
 #pragma unroll
@@ -1576,12 +1586,15 @@ __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, cons
   constexpr bool kBoundary = C == 1;
   const int lane = 16 * g + m;
   const int entry = operand_entry(m, g);
-  auto tanh_rows = [&](const f4 (&z)[4], f4 (&out)[4]) {
+  // The jet's output rows, and what the walk back keeps of them: u for v' (tanh_jet_adjoint_h).
+  auto tanh_rows = [&](const f4 (&z)[4], f4 (&out)[4], f4 (&keep)[4]) {
     if (kBoundary) {
       f4 unused;
-      tanh_scaled4(z[0], out[0], unused);
+      tanh_scaled4(z[0], keep[0], out[0], unused);
     } else {
-      tanh_jet4(z, out);
+      tanh_jet4(z, out, keep[0]);
+#pragma unroll
+      for (int c = 1; c < 4; ++c) keep[c] = out[c];
     }
   };
   auto split_rows = [&](const f4 (&x)[4], u2 (&part)[4][kParts]) {
@@ -1638,16 +1651,16 @@ __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, cons
       }
     }
   }
-  f4 h[3][4];  // this wave's rows of the hidden layers' outputs
+  f4 h[3][4], out[4];  // this wave's rows of the hidden layers' outputs: as kept, and the last one's
 #pragma unroll
   for (int layer = 0; layer < 3; ++layer) {
     const f4 bias = lds4(s_small + kSmallBh + layer * kHidden + 16 * w + 4 * g);
     f4 z[4];
     product(lds_weights(w_lane + layer * kLayerU4, w), op, bias, z);
-    tanh_rows(z, h[layer]);
+    tanh_rows(z, out, h[layer]);
     if (layer < 2) {
       Exchange& x = layer ? sc.h2 : sc.h1;
-      put_rows(x, h[layer]);
+      put_rows(x, out);
       __syncthreads();
       get_components<C>(x, entry, op);
     }
@@ -1660,17 +1673,17 @@ __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, cons
       const f4 wo = lds4(s_small + (kBoundary ? kSmallWoutV : kSmallWoutL) + 16 * w + 4 * g);
       float t = 0.0f;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) t = __builtin_fmaf(wo[r], h[2][kBoundary ? 0 : 3][r], t);
+      for (int r = 0; r < 4; ++r) t = __builtin_fmaf(wo[r], out[kBoundary ? 0 : 3][r], t);
       terms[w * kWave + lane] = t;
     }
     __syncthreads();
-    float out = terms[lane];
+    float total = terms[lane];
 #pragma unroll
-    for (int mb = 1; mb < 4; ++mb) out += terms[mb * kWave + lane];
-    out = sum_lane_groups(out);
+    for (int mb = 1; mb < 4; ++mb) total += terms[mb * kWave + lane];
+    total = sum_lane_groups(total);
     __syncthreads();  // sc.z is free again
     // u (boundary) or the residual lap - f (interior).
-    const float e = active ? (kBoundary ? out + s_small[kSmallBout] : out - f) : 0.0f;
+    const float e = active ? (kBoundary ? total + s_small[kSmallBout] : total - f) : 0.0f;
     const float sq = sum_row16(e * e);
     if (kBoundary) {
       gu = sign * (seed.boundary_scale * (2.0f * e));
@@ -1694,7 +1707,7 @@ __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, cons
     f4 terms;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      terms[r] = kBoundary ? gu_c * h[2][0][r] : __builtin_fmaf(gu_c, h[2][0][r], gl_l * h[2][3][r]);
+      terms[r] = kBoundary ? gu_c * out[0][r] : __builtin_fmaf(gu_c, out[0][r], gl_l * out[3][r]);
       hb[0][r] = gu * wv[r];
       if (!kBoundary) {
         hb[1][r] = 0.0f;
@@ -1713,12 +1726,11 @@ __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, cons
     f4 zb[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const float v = h[layer][0][r];
       if (kBoundary) {
-        zb[0][r] = __builtin_fmaf(kHalfKappa * v, v, 0.25f) * hb[0][r];
+        zb[0][r] = tanh_slope(h[layer][0][r]) * hb[0][r];
       } else {
         float bv = hb[0][r], bj0 = hb[1][r], bj1 = hb[2][r], bl = hb[3][r];
-        tanh_jet_adjoint_h(v, h[layer][1][r], h[layer][2][r], h[layer][3][r], bv, bj0, bj1, bl);
+        tanh_jet_adjoint_h(h[layer][0][r], h[layer][1][r], h[layer][2][r], h[layer][3][r], bv, bj0, bj1, bl);
         zb[0][r] = bv;
         zb[1][r] = bj0;
         zb[2][r] = bj1;
@@ -1774,10 +1786,10 @@ __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, cons
     const Layer0Weights w0 = layer0_weights(s_small, w, g);
     const float cx0 = kHalfC * x0, cx1 = kHalfC * x1;
     float gx0 = 0.f, gx1 = 0.f;
-    f4 zv4, v4, s4, tx, ty, tb;
+    f4 zv4, unused, v4, s4, tx, ty, tb;
 #pragma unroll
     for (int r = 0; r < 4; ++r) zv4[r] = layer0_zv(w0, r, x0, x1);
-    tanh_scaled4(zv4, v4, s4);
+    tanh_scaled4(zv4, unused, v4, s4);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float bv = hb[0][r];
@@ -2054,7 +2066,7 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             wout_terms[4 * mb + r] = kLoss ? gl_l * h3[mb][3][r]
-                                           : __builtin_fmaf(gu_c, h3[mb][0][r], gl_l * h3[mb][3][r]);
+                                           : __builtin_fmaf(gu_c, tanh_value(h3[mb][0][r]), gl_l * h3[mb][3][r]);
             float bv = kLoss ? 0.0f : gu * wv[r], bj0, bj1, bl = gl * wl[r];
             tanh_jet_adjoint_h_seed<kLoss>(h3[mb][0][r], h3[mb][1][r], h3[mb][2][r], h3[mb][3][r],
                                            bv, bj0, bj1, bl);
@@ -2113,19 +2125,19 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
       // grad_x = (c W0)^T bv, dW0[o][d] = sum_p bv (c x_d) + 2 bj_d = 2 sum_p (bv (c x_d / 2) + bj_d)
       // (the row takes the 2), db0 = c sum_p bv.
       {
-        f4 h0[4][4], s0[4];
+        f4 h0[4][4];
 #pragma unroll
         for (int mb = 0; mb < 4; ++mb) {
           const Layer0Weights w0 = layer0_weights(s_small, mb, g);
-          f4 zv;
+          f4 zv, v, s;
 #pragma unroll
           for (int r = 0; r < 4; ++r) zv[r] = layer0_zv(w0, r, x0, x1);
-          tanh_scaled4(zv, h0[mb][0], s0[mb]);
+          tanh_scaled4(zv, h0[mb][0], v, s);
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            h0[mb][1][r] = s0[mb][r] * w0.wx[r];
-            h0[mb][2][r] = s0[mb][r] * w0.wy[r];
-            h0[mb][3][r] = s0[mb][r] * (h0[mb][0][r] * w0.q[r]);
+            h0[mb][1][r] = s[r] * w0.wx[r];
+            h0[mb][2][r] = s[r] * w0.wy[r];
+            h0[mb][3][r] = s[r] * (v[r] * w0.q[r]);
           }
         }
         float gx0 = 0.f, gx1 = 0.f, tx[16], ty[16], tb[16];
@@ -2134,7 +2146,8 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
         Layer0Weights lw = layer0_weights(s_small, 0, g);  // of the block at hand, read a block ahead
         backward_layer(w_t, w_t, sp, minus_one, zb, h0, sums, wt, [&](int ib, int r, const f4 (&hb)[4]) {
           float bv = hb[0][r], bj0 = hb[1][r], bj1 = hb[2][r], bl = hb[3][r];
-          tanh_jet_adjoint_layer0(h0[ib][0][r], s0[ib][r], lw.wx[r], lw.wy[r], lw.q[r], bv, bj0, bj1, bl);
+          const float u = h0[ib][0][r];
+          tanh_jet_adjoint_layer0(tanh_value(u), tanh_slope(u), lw.wx[r], lw.wy[r], lw.q[r], bv, bj0, bj1, bl);
           gx0 = __builtin_fmaf(lw.cwx[r], bv, gx0);
           gx1 = __builtin_fmaf(lw.cwy[r], bv, gx1);
           tx[4 * ib + r] = __builtin_fmaf(bv, cx0, bj0);  // dW0[o][0] / 2
