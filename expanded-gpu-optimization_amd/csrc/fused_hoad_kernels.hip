@@ -95,7 +95,9 @@ __device__ __forceinline__ f4 lds4(const float* p) { return *reinterpret_cast<co
 // of random values is off by 0.9e-7 of its norm this way and by 1.45e-7 with
 // v_mfma_f32_16x16x4f32 (fewer roundings along the accumulation).
 // An infinite value, or one that rounds to an infinite bf16 (above 3.39e38), has an infinite hi
-// and a NaN remainder: what follows from it is NaN.
+// and a NaN remainder: what follows from it is NaN. The forward kernels therefore form a NaN result
+// again from float32 products (float32_outputs). The gradient kernels do not: a hidden weight's
+// gradient is NaN where float32 products could give an infinity.
 typedef unsigned u4 __attribute__((ext_vector_type(4)));  // 8 bf16 values, two to a register
 typedef unsigned u2 __attribute__((ext_vector_type(2)));
 typedef float f2 __attribute__((ext_vector_type(2)));
@@ -711,6 +713,86 @@ __device__ __forceinline__ void get_exchange(const Exchange& x, int entry, JetOp
   }
 }
 
+// (u - b_out, lap) of a tile's points from float32 products (v_mfma_f32_16x16x4f32, k-step 16 ib + j
+// taking inputs 16 ib + 4 g + j from the lane groups), the weights read from global memory. For
+// results that split products cannot give: with an infinite hidden weight the tanh saturates and u is
+// finite, and a Laplacian can be infinite rather than NaN.
+__device__ __forceinline__ f2 float32_outputs(const float* __restrict__ params, const float* s_small, int m,
+                                              int g, float x0, float x1) {
+  f4 h[4][4];
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb) layer0_block(s_small, mb, g, x0, x1, h[mb]);
+  f2 out{0.0f, 0.0f};
+#pragma unroll 1
+  for (int layer = 0; layer < 3; ++layer) {
+    const float* row = params + kHiddenBase + layer * kHiddenStride + m * kHidden + 4 * g;
+    f4 next[4][4];
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) {
+      f4 z[4];
+      z[0] = lds4(s_small + kSmallBh + layer * kHidden + 16 * mb + 4 * g);
+      z[1] = z[2] = z[3] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ib = 0; ib < 4; ++ib) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float w = 4.0f * row[16 * mb * kHidden + 16 * ib + j];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) z[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w, h[ib][c][j], z[c], 0, 0, 0);
+        }
+      }
+      tanh_jet4(z, next[mb]);
+    }
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) h[mb][c] = next[mb][c];
+    }
+  }
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb) {
+    const f2 terms = output_terms(s_small, mb, g, h[mb]);
+    out[0] = mb ? out[0] + terms[0] : terms[0];
+    out[1] = mb ? out[1] + terms[1] : terms[1];
+  }
+  return f2{sum_lane_groups(out[0]), sum_lane_groups(out[1])};
+}
+
+__device__ __forceinline__ bool is_nan(float a, float b) { return a != a || b != b; }
+
+// At a forward kernel's end, after some tile of the workgroup (blockIdx.x + k gridDim.x) came out
+// NaN: its waves read the tiles' results back and write the NaN ones, and only those, again from
+// float32_outputs. Here nothing else is live (the lane's indexes are formed anew and the wave's is a
+// scalar); inside the tile loops the same work cost registers. A NaN parameter makes every result NaN
+// whatever the products, so then nothing is tried (s_nan = 2): 1,000,003 points of a network that has
+// diverged take 380 us, 1,194 without that look at the parameters.
+template <int kWaves>
+__device__ __forceinline__ void retry_nan_tiles(const float* __restrict__ coordinates, const float* __restrict__ params,
+                                                const float* s_small, float* __restrict__ output,
+                                                float* __restrict__ laplacian, int64_t batch, int64_t tiles,
+                                                int wave, unsigned& s_nan) {
+  bool hopeless = false;
+  for (int k = threadIdx.x; k < kOutputBase + kHidden; k += kWaves * kWave) hopeless |= params[k] != params[k];
+  if (hopeless) s_nan = 2;
+  __syncthreads();
+  if (s_nan == 2) return;
+  const int lane = opaque(__lane_id());
+  const int m = lane & 15, g = lane >> 4;
+  for (int64_t tile = blockIdx.x + static_cast<int64_t>(wave) * gridDim.x; tile < tiles;
+       tile += static_cast<int64_t>(kWaves) * gridDim.x) {
+    const int64_t point = tile * kTile + m;
+    const bool active = point < batch;
+    const float u = active ? output[point] : 0.0f, lap = active ? laplacian[point] : 0.0f;
+    if (!__any(is_nan(u, lap))) continue;
+    const float x0 = active ? coordinates[2 * point] : 0.0f, x1 = active ? coordinates[2 * point + 1] : 0.0f;
+    const f2 again = float32_outputs(params, s_small, m, g, x0, x1);
+    if (g == 0 && active) {
+      if (u != u) output[point] = again[0] + s_small[kSmallBout];
+      if (lap != lap) laplacian[point] = again[1];
+    }
+  }
+}
+
 template <int kWaves>
 __global__ void __launch_bounds__(kWaves * kWave)
 forward_kernel(const float* __restrict__ coordinates, const float* __restrict__ params,
@@ -721,6 +803,7 @@ forward_kernel(const float* __restrict__ coordinates, const float* __restrict__ 
   __shared__ Exchange s_x[2];  // split tiles
   __shared__ unsigned s_quad;  // split tiles: quad_sync counter
   __shared__ unsigned s_next;  // the next k to take
+  __shared__ unsigned s_nan;   // some result is NaN
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int g = lane >> 4;
@@ -739,7 +822,10 @@ forward_kernel(const float* __restrict__ coordinates, const float* __restrict__ 
   if (threadIdx.x == 0) {
     s_quad = 0;
     s_next = kWaves;
+    s_nan = 0;
   }
+  bool nan = false;
+  const int wave_index = __builtin_amdgcn_readfirstlane(wave);
   const SmallLoads small = load_small<kWaves * kWave>(params, threadIdx.x);
   stage_operand_weights<kWaves * kWave>(params, s_wa, threadIdx.x);
   store_small(s_small, threadIdx.x, small);
@@ -798,6 +884,7 @@ forward_kernel(const float* __restrict__ coordinates, const float* __restrict__ 
               out[1] += more[1];
             }
             const float u = sum_lane_groups(out[0]), lap = sum_lane_groups(out[1]);
+            if (met) nan |= active && is_nan(u, lap);
             if (g == 0 && active) {
               // A tile whose meetings gave up read stale rows: its outputs are NaN (and the
               // device status word says why).
@@ -853,10 +940,16 @@ forward_kernel(const float* __restrict__ coordinates, const float* __restrict__ 
     next_x0 = opaque(next_x0);
     next_x1 = opaque(next_x1);
     const float u = sum_lane_groups(out[0]), lap = sum_lane_groups(out[1]);
+    nan |= active && is_nan(u, lap);
     if (g == 0 && active) {
       output[point] = u + s_small[kSmallBout];
       laplacian[point] = lap;
     }
+  }
+  if (nan) s_nan = 1;
+  __syncthreads();  // also: the workgroup's results are written
+  if (s_nan) {
+    retry_nan_tiles<kWaves>(coordinates, params, s_small, output, laplacian, batch, tiles, wave_index, s_nan);
   }
 }
 
@@ -878,10 +971,14 @@ forward_split_kernel(const float* __restrict__ coordinates, const float* __restr
                      int64_t tiles) {
   __shared__ Exchange s_x[2];
   __shared__ __attribute__((aligned(16))) float s_small[kSmallFloats];
+  __shared__ unsigned s_nan;  // some result is NaN
   const int lane = threadIdx.x & (kWave - 1);
   const int w = threadIdx.x / kWave;
   const int m = lane & 15;
   const int g = lane >> 4;
+  if (threadIdx.x == 0) s_nan = 0;
+  bool nan = false;
+  const int wave_index = __builtin_amdgcn_readfirstlane(w);
   // The small parameters are staged first and this wave's operands loaded after (they are needed
   // only after the barrier and the first tile's coordinates): issued together, the operand loads
   // were waited for before the barrier and a 1K-point call took 0.4 us longer.
@@ -951,6 +1048,7 @@ forward_split_kernel(const float* __restrict__ coordinates, const float* __restr
             out[1] += more[1];
           }
           const float u = sum_lane_groups(out[0]), lap = sum_lane_groups(out[1]);
+          nan |= active && is_nan(u, lap);
           if (g == 0 && active) {
             output[point] = u + s_small[kSmallBout];
             laplacian[point] = lap;
@@ -958,6 +1056,11 @@ forward_split_kernel(const float* __restrict__ coordinates, const float* __restr
         }
       }
     }
+  }
+  if (nan) s_nan = 1;
+  __syncthreads();  // also: the workgroup's results are written
+  if (s_nan) {
+    retry_nan_tiles<kSplitWaves>(coordinates, params, s_small, output, laplacian, batch, tiles, wave_index, s_nan);
   }
 }
 
