@@ -1678,7 +1678,7 @@ __device__ __forceinline__ void get_components(const Exchange& x, int entry, Jet
 // the value one is exactly zero at every layer. The weight-gradient terms reduce to
 // zbar_v h_v^T, and the forward's J and L components feed nothing. A boundary tile therefore
 // runs the value channel only; the terms it skips are exact zeros.
-template <int kComponents, bool kLoss, bool kHbarFirst>
+template <int kComponents, bool kLoss>
 __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, const float* s_small,
                                            SplitScratch& sc, u2 minus_one, int w, int g, int m,
                                            float x0, float x1, float gu, float gl, float f,
@@ -1850,9 +1850,9 @@ __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, cons
     }
     __syncthreads();
     // hbar of this wave's rows of the layer below, before dW: the next adjoint waits for it alone, and
-    // its VALU work runs behind dW's MFMAs (kHbarFirst holds the compiler to it: backward call at
-    // 1,000 points 18.2 -> 17.1 us; in backward_kernel<false, true, false> it made the 64-point tiles spill,
-    // 50,021 points 93.7 -> 96.1 us).
+    // its VALU work runs behind dW's MFMAs (the region's end holds the compiler to it). Backward call at
+    // 1,000 points 18.2 -> 17.1 us; with a rest of split tiles, 30,000 points 74.5 -> 70.4, 70,001
+    // 127.4 -> 122.6.
     get_components<C>(sc.z, entry, op);
     const u4* wt = w_t + layer * kLayerU4 + (w >> 1) * kParts * kWave;
     WeightOperand a;
@@ -1869,7 +1869,7 @@ __device__ __forceinline__ void split_tile(const u4* w_lane, const u4* w_t, cons
       }
     }
     product(a, op, zero4(), hb);
-    if (kHbarFirst) region_end();
+    region_end();
     // dW += sum over (c, points) of zbar h_prev^T.
     {
       const Exchange& hx = layer == 1 ? sc.h1 : sc.h2;
@@ -2291,8 +2291,8 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
       }
     };
     // kRest: interior points past the last whole round of 64-point tiles, as 16-point tiles
-    // whose rows are split over the 4 waves (split_tile), so a round that is not whole costs a
-    // quarter tile on the slots that have one instead of a whole tile on some. The scratch
+    // whose rows are split over the 4 waves (split_tile); one takes 9.7 us, a 64-point tile 22 (see
+    // interior_tiles_for). The scratch
     // overlays the dW staging buffer: the barrier waits for the last 64-point tile's readers.
     // (A separate instantiation: with this loop in the kernel the compiler schedules the
     // 64-point loop differently, so whole rounds run without it.)
@@ -2308,7 +2308,7 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
         }
         const int64_t point = whole * kBwdTile + (tile - whole) * kTile + m;
         SplitSums s{};
-        split_tile<4, kLoss, kLoss>(w_lane, w_t, s_small, s_x.split, minus_one, w, g, m_pick, in.x0, in.x1,
+        split_tile<4, kLoss>(w_lane, w_t, s_small, s_x.split, minus_one, w, g, m_pick, in.x0, in.x1,
                              kLoss ? 0.f : in.a, kLoss ? 0.f : in.b, kLoss ? in.a : 0.f,
                              point < batch, walk_sign(slot, round), point, grad_coordinates, seed, dw, s);
         add_split(s, m_pick);
@@ -2328,7 +2328,7 @@ backward_kernel(const float* __restrict__ coordinates, const float* __restrict__
         }
         const int64_t point = (tile - seed.interior_tiles) * kTile + m;
         SplitSums s{};
-        split_tile<1, kLoss, kLoss>(w_lane, w_t, s_small, s_x.split, minus_one, w, g, m_pick, in.x0, in.x1, 0.f,
+        split_tile<1, kLoss>(w_lane, w_t, s_small, s_x.split, minus_one, w, g, m_pick, in.x0, in.x1, 0.f,
                              0.f, 0.f, point < seed.boundary_count, walk_sign(slot, round), point, nullptr, seed, dw, s);
         add_split(s, m_pick);
         deliver(next);
@@ -2446,7 +2446,7 @@ backward_split_kernel(const float* __restrict__ coordinates, const float* __rest
                                              seed, tile + slots, w, m);
       }
       const int64_t point = tile * kTile + m;
-      split_tile<4, kLoss, true>(w_lane, w_t, s_small, s_x, minus_one, w, g, m, in.x0, in.x1,
+      split_tile<4, kLoss>(w_lane, w_t, s_small, s_x, minus_one, w, g, m, in.x0, in.x1,
                            kLoss ? 0.f : in.a, kLoss ? 0.f : in.b, kLoss ? in.a : 0.f, point < batch,
                            walk_sign(slot, round), point, grad_coordinates, seed, dw, sums);
       deliver(next);
@@ -2460,7 +2460,7 @@ backward_split_kernel(const float* __restrict__ coordinates, const float* __rest
                                                seed, tile + slots, w, m);
         }
         const int64_t point = (tile - seed.interior_tiles) * kTile + m;
-        split_tile<1, kLoss, true>(w_lane, w_t, s_small, s_x, minus_one, w, g, m, in.x0, in.x1, 0.f, 0.f, 0.f,
+        split_tile<1, kLoss>(w_lane, w_t, s_small, s_x, minus_one, w, g, m, in.x0, in.x1, 0.f, 0.f, 0.f,
                              point < seed.boundary_count, walk_sign(slot, round), point, nullptr, seed, dw,
                              sums);
         deliver(next);
@@ -2734,7 +2734,10 @@ int64_t split_tiles(int64_t points) { return (points + kTile - 1) / kTile; }
 // Interior tiles of backward_kernel for `batch` points over `slots` slots: 64-point tiles in
 // whole rounds of `slots` (`whole` of them), then the remaining points as 16-point tiles whose
 // rows are split over the waves (`total` counts both). Below one whole round, or when the
-// rounds are whole, every tile is a 64-point one.
+// rounds are whole, every tile is a 64-point one. A split tile takes 0.43 of a 64-point tile's time, so
+// a rest of one or two a slot costs less than a round of 64-point tiles would, one of three or four
+// more (backward call of 16,384 points 36.4 us, 16,400 44.2, 24,000 57.5, 28,000 67, 32,000 77, and
+// 32,768, two whole rounds, 58.6).
 struct InteriorTiles {
   int64_t whole, total;
 };
