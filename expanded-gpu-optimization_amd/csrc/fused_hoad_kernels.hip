@@ -2010,9 +2010,9 @@ struct PhaseClock {
 // grad_coordinates may be null.
 //
 // kBoundary: with boundary tiles in it, the fused step's kernel spills more registers in its 64-point
-// tiles (step of 16,384 points 39.1 -> 37.4 us without them, 65,536 109.3 -> 106.6, 262,144 400 ->
-// 395), so steps of whole rounds without boundary points run a form without; with a rest of split
-// tiles the form without spills more (50,021 points 93.5 -> 95.9), so that one always has them.
+// tiles, so a step of whole rounds without boundary points runs a form without them (262,144 points
+// 396.5 -> 389.3 us). With a rest of split tiles the two forms are within 2 % either way (30,000 points
+// 74.1 against 72.6 without, 250,001 386 against 387.5), so that one always has them.
 template <bool kLoss, bool kRest, bool kBoundary>
 __global__ void __launch_bounds__(kBwdWaves * kWave, 1)
 backward_kernel(const float* __restrict__ coordinates, const float* __restrict__ params,

@@ -62,7 +62,7 @@ def test_backward_through_saturated_units(batch: int, first: int) -> None:
     assert (got_x.double() - want_x).norm() < BOUND * want_x.norm()
 
 
-@pytest.mark.parametrize("batch,boundary", [(1000, 0), (1000, 100), (16384, 1024), (70001, 500)])
+@pytest.mark.parametrize("batch,boundary", [(1000, 0), (1000, 100), (16384, 0), (16384, 1024), (16400, 0), (70001, 0), (70001, 500)])
 def test_step_through_saturated_units(batch: int, boundary: int) -> None:
     """The fused step's kernels. With boundary points the source is the network's own Laplacian and
     the boundary term's weight is large, so the gradient is the boundary tiles' alone."""
