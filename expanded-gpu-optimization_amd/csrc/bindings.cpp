@@ -99,50 +99,15 @@ std::vector<torch::Tensor> fused_forward_laplacian_backward(torch::Tensor coordi
   return {grad_parameters, grad_coordinates};
 }
 
-// The saved-layer pair's forward: (u, Laplacian, buffer), the last an opaque uint8 buffer of
-// fhoad_saved_layers_size(batch) bytes for backward_for_autograd.
-std::vector<torch::Tensor> forward_saving(torch::Tensor coordinates, torch::Tensor parameters,
-                                          int64_t version) {
-  TORCH_CHECK(version >= 0 && version <= 5, "version must be 0 to 5");
-  check_inputs(coordinates, parameters);
-  const c10::DeviceGuard device_guard(coordinates.device());
-  const int64_t batch = coordinates.size(0);
-  auto output = torch::empty({batch, 1}, coordinates.options());
-  auto laplacian = torch::empty({batch, 1}, coordinates.options());
-  const size_t saved_bytes = fhoad_saved_layers_size(batch);
-  TORCH_CHECK(saved_bytes <= static_cast<size_t>(INT64_MAX),
-              "the saved layers of ", batch, " points do not fit in memory");
-  auto saved = torch::empty({static_cast<int64_t>(saved_bytes)},
-                            coordinates.options().dtype(torch::kUInt8));
-  if (batch == 0) {
-    return {output, laplacian, saved};
-  }
-  check_status(fhoad_forward_laplacian_saving(
-      coordinates.data_ptr<float>(), parameters.data_ptr<float>(), output.data_ptr<float>(),
-      laplacian.data_ptr<float>(), saved.data_ptr(), saved_bytes, batch,
-      static_cast<int>(version), current_stream(coordinates)));
-  return {output, laplacian, saved};
-}
-
 // The backward for the autograd glue (no counterpart among the reference's bindings): either
 // upstream gradient may be None (zero, so no zeros tensor is made), and grad_coordinates is
 // computed only when want_coordinates is set (otherwise None is returned and nothing is
-// written). Same checks and kernels as fused_forward_laplacian_backward. saved:
-// forward_saving's buffer for the same coordinates and parameters (checked, not read), or None.
+// written). Same checks and kernels as fused_forward_laplacian_backward.
 std::vector<c10::optional<torch::Tensor>> backward_for_autograd(
     torch::Tensor coordinates, torch::Tensor parameters, c10::optional<torch::Tensor> grad_output,
-    c10::optional<torch::Tensor> grad_laplacian, bool want_coordinates, int64_t version,
-    c10::optional<torch::Tensor> saved) {
+    c10::optional<torch::Tensor> grad_laplacian, bool want_coordinates, int64_t version) {
   TORCH_CHECK(version >= 1 && version <= 6, "backward version must be 1 to 6");
   check_inputs(coordinates, parameters);
-  if (saved.has_value()) {
-    TORCH_CHECK(saved->is_cuda() && saved->is_contiguous() && saved->scalar_type() == torch::kUInt8,
-                "saved layers must be a contiguous uint8 CUDA tensor");
-    TORCH_CHECK(saved->device() == coordinates.device(),
-                "saved layers must be on the coordinates' device");
-    TORCH_CHECK(static_cast<size_t>(saved->numel()) >= fhoad_saved_layers_size(coordinates.size(0)),
-                "saved layers do not cover the batch");
-  }
   for (const auto* grad : {&grad_output, &grad_laplacian}) {
     if (!grad->has_value()) continue;
     const torch::Tensor& g = **grad;
@@ -166,18 +131,10 @@ std::vector<c10::optional<torch::Tensor>> backward_for_autograd(
   const float* gu = grad_output.has_value() ? grad_output->data_ptr<float>() : nullptr;
   const float* gl = grad_laplacian.has_value() ? grad_laplacian->data_ptr<float>() : nullptr;
   float* gx = want_coordinates ? grad_coordinates->data_ptr<float>() : nullptr;
-  if (saved.has_value()) {
-    check_status(fhoad_forward_laplacian_backward_saved(
-        coordinates.data_ptr<float>(), parameters.data_ptr<float>(), saved->data_ptr(),
-        static_cast<size_t>(saved->numel()), gu, gl, grad_parameters.data_ptr<float>(), gx,
-        workspace.data_ptr(), workspace_bytes, batch, static_cast<int>(version),
-        current_stream(coordinates)));
-  } else {
-    check_status(fhoad_forward_laplacian_backward(
-        coordinates.data_ptr<float>(), parameters.data_ptr<float>(), gu, gl,
-        grad_parameters.data_ptr<float>(), gx, workspace.data_ptr(), workspace_bytes, batch,
-        static_cast<int>(version), current_stream(coordinates)));
-  }
+  check_status(fhoad_forward_laplacian_backward(
+      coordinates.data_ptr<float>(), parameters.data_ptr<float>(), gu, gl,
+      grad_parameters.data_ptr<float>(), gx, workspace.data_ptr(), workspace_bytes, batch,
+      static_cast<int>(version), current_stream(coordinates)));
   return {grad_parameters, grad_coordinates};
 }
 
@@ -206,20 +163,18 @@ static_assert(fhoad::kOutputBase + fhoad::kHidden + 1 == kParameterCount, "packe
 // per-step host work (the Python apply, the backward's Python frame, the differentiable
 // torch.cat pack and its backward, or the ten gradient views built in Python). Inputs:
 // coordinates; the packed buffer when the model's parameters are its views
-// (flatten_poisson_parameters_), else None; the forward and backward versions; save_layers (the
-// "saved" mode; nothing is kept, since the backward re-runs the forward faster than it could read
-// the layers back); and the ten parameters in layout order (weight
-// then bias of each linear layer), the Function's differentiable inputs. Without a buffer the
-// parameters are packed into a new one (one copy kernel, outside autograd). Each parameter gets
-// a view of the packed gradient with its own shape. An unused output's gradient arrives
-// undefined and is read as zero; the coordinate gradient is computed only when the coordinates
-// need it.
+// (flatten_poisson_parameters_), else None; the forward and backward versions; and the ten
+// parameters in layout order (weight then bias of each linear layer), the Function's
+// differentiable inputs. Without a buffer the parameters are packed into a new one (one copy
+// kernel, outside autograd). Each parameter gets a view of the packed gradient with its own
+// shape. An unused output's gradient arrives undefined and is read as zero; the coordinate
+// gradient is computed only when the coordinates need it.
 struct ModelLaplacian : public torch::autograd::Function<ModelLaplacian> {
   static torch::autograd::variable_list forward(torch::autograd::AutogradContext* ctx,
                                                 const torch::Tensor& coordinates,
                                                 const c10::optional<torch::Tensor>& packed,
                                                 int64_t version, int64_t backward_version,
-                                                bool /*save_layers*/, torch::TensorList parameters) {
+                                                torch::TensorList parameters) {
     TORCH_CHECK(backward_version >= 1 && backward_version <= 6, "backward version must be 1 to 6");
     TORCH_CHECK(parameters.size() == kPackedSlices.size(), "expected the model's 10 parameters");
     for (size_t k = 0; k < kPackedSlices.size(); ++k) {
@@ -251,9 +206,8 @@ struct ModelLaplacian : public torch::autograd::Function<ModelLaplacian> {
     ctx->saved_data["backward_version"] = backward_version;
     ctx->saved_data["packed_given"] = packed.has_value();
     std::vector<torch::Tensor> out = fused_forward_laplacian(coordinates, flat, version);
-    // Saved: coordinates, the packed buffer and, when the
-    // buffer is the model's (its parameters are views of it), the ten parameters as well: each
-    // view has its own version counter, so an in-place update of a parameter between this
+    // Saved: coordinates, the packed buffer and, when the buffer is the model's (its parameters
+    // are views of it), the ten parameters as well: each view has its own version counter, so an in-place update of a parameter between this
     // forward and the backward (an optimizer step before a retain_graph backward) leaves the
     // buffer's counter alone; saving the views makes autograd's check of their counters raise
     // PyTorch's in-place-modification error there, as nn.Linear would. Saving copies nothing.
@@ -266,9 +220,9 @@ struct ModelLaplacian : public torch::autograd::Function<ModelLaplacian> {
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  torch::autograd::variable_list grads) {
     // One gradient per forward argument: coordinates, packed, version, backward_version,
-    // save_layers, then the ten parameters (undefined where none). The differentiable inputs
-    // are the coordinates (input 0), the packed buffer when given, and the parameters.
-    torch::autograd::variable_list result(5 + kPackedSlices.size());
+    // then the ten parameters (undefined where none). The differentiable inputs are the
+    // coordinates (input 0), the packed buffer when given, and the parameters.
+    torch::autograd::variable_list result(4 + kPackedSlices.size());
     if (!grads[0].defined() && !grads[1].defined()) return result;
     const auto saved = ctx->get_saved_variables();
     const size_t first_parameter = ctx->saved_data["packed_given"].toBool() ? 2 : 1;
@@ -283,14 +237,14 @@ struct ModelLaplacian : public torch::autograd::Function<ModelLaplacian> {
     };
     const auto out = backward_for_autograd(
         saved[0], saved[1], upstream(grads[0]), upstream(grads[1]), needs_coordinates,
-        ctx->saved_data["backward_version"].toInt(), c10::nullopt);
+        ctx->saved_data["backward_version"].toInt());
     if (needs_coordinates) result[0] = *out[1];
     if (needs_parameters) {
       const torch::Tensor& grad_flat = *out[0];
       for (size_t k = 0; k < kPackedSlices.size(); ++k) {
         if (!ctx->needs_input_grad(first_parameter + k)) continue;
         const PackedSlice& slice = kPackedSlices[k];
-        result[5 + k] = slice.cols ? grad_flat.as_strided({slice.rows, slice.cols}, {slice.cols, 1}, slice.offset)
+        result[4 + k] = slice.cols ? grad_flat.as_strided({slice.rows, slice.cols}, {slice.cols, 1}, slice.offset)
                                    : grad_flat.as_strided({slice.rows}, {1}, slice.offset);
       }
     }
@@ -301,9 +255,8 @@ struct ModelLaplacian : public torch::autograd::Function<ModelLaplacian> {
 torch::autograd::variable_list model_laplacian(const torch::Tensor& coordinates,
                                                const c10::optional<torch::Tensor>& packed,
                                                int64_t version, int64_t backward_version,
-                                               bool save_layers,
                                                const std::vector<torch::Tensor>& parameters) {
-  return ModelLaplacian::apply(coordinates, packed, version, backward_version, save_layers,
+  return ModelLaplacian::apply(coordinates, packed, version, backward_version,
                                torch::TensorList(parameters));
 }
 
@@ -394,17 +347,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, module) {
              "optional coordinate gradient",
              pybind11::arg("coordinates"), pybind11::arg("parameters"),
              pybind11::arg("grad_output"), pybind11::arg("grad_laplacian"),
-             pybind11::arg("want_coordinates"), pybind11::arg("version") = 6,
-             pybind11::arg("saved") = pybind11::none());
+             pybind11::arg("want_coordinates"), pybind11::arg("version") = 6);
   module.def("_model_laplacian", &model_laplacian,
              "(u, Laplacian) of the model's ten parameters through the C++ autograd Function",
              pybind11::arg("coordinates"), pybind11::arg("packed"), pybind11::arg("version"),
-             pybind11::arg("backward_version"), pybind11::arg("save_layers"),
-             pybind11::arg("parameters"));
-  module.def("_forward_saving", &forward_saving,
-             "Forward with the saved-layer pair's buffer for _backward(saved=...)",
-             pybind11::arg("coordinates"), pybind11::arg("parameters"),
-             pybind11::arg("version") = 2);
+             pybind11::arg("backward_version"), pybind11::arg("parameters"));
   module.def("fused_forward_laplacian", &fused_forward_laplacian,
              "Fixed MLP forward pass and input Laplacian (MI355X HIP kernel)",
              pybind11::arg("coordinates"), pybind11::arg("parameters"),

@@ -172,15 +172,15 @@ def test_model_laplacian_function_checks_its_parameters() -> None:
     flat, tensors = flattened_poisson_binding(model)
     x = coordinates(100, seed=33)
     with pytest.raises(RuntimeError, match="must have the shape of layout slice 0"):
-        _C._model_laplacian(x, flat, 2, 6, False, [tensors[2], *tensors[1:]])
+        _C._model_laplacian(x, flat, 2, 6, [tensors[2], *tensors[1:]])
     with pytest.raises(RuntimeError, match="parameter 3 is not the packed buffer's view"):
-        _C._model_laplacian(x, flat, 2, 6, False, [*tensors[:3], tensors[3].clone(), *tensors[4:]])
+        _C._model_laplacian(x, flat, 2, 6, [*tensors[:3], tensors[3].clone(), *tensors[4:]])
     with pytest.raises(RuntimeError, match="expected the model's 10 parameters"):
-        _C._model_laplacian(x, flat, 2, 6, False, tensors[:9])
-    u, lap = _C._model_laplacian(x, flat, 2, 6, False, tensors)
+        _C._model_laplacian(x, flat, 2, 6, tensors[:9])
+    u, lap = _C._model_laplacian(x, flat, 2, 6, tensors)
     ref_u, ref_lap = fused_forward_laplacian(x, flat, 2)
     twin = _model(7)
-    packed_u, packed_lap = _C._model_laplacian(x, None, 2, 6, False, list(twin.parameters()))
+    packed_u, packed_lap = _C._model_laplacian(x, None, 2, 6, list(twin.parameters()))
     torch.cuda.synchronize()
     assert torch.equal(pack_poisson_parameters(twin), flat)
     assert torch.equal(u, ref_u) and torch.equal(lap, ref_lap)
@@ -337,9 +337,8 @@ def test_graph_captured_training_step_matches_eager_step() -> None:
 
 @pytest.mark.parametrize("mode", ["cuda", "saved"])
 def test_graph_captured_flattened_step_matches_eager_at_64k(mode: str) -> None:
-    """The drop-in step bench.py times as train_step_autograd_graphed_ms (and, with
-    backward="saved", as ..._saved_ms): a flattened model at 65,536 points (BASELINE config 3's
-    size, where torch's mean reduces over many blocks), captured whole and replayed 10 times
+    """The drop-in step bench.py times as train_step_autograd_graphed_ms, and the same with
+    backward="saved": a flattened model at 65,536 points (BASELINE config 3's size, where torch's mean reduces over many blocks), captured whole and replayed 10 times
     with a host sync between replays, against the same steps run eagerly: every replay's loss
     (rtol 1e-4) and the weights after."""
     announce(f"whole-step graph capture vs eager, flattened model, batch=65536, backward={mode}")
