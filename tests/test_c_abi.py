@@ -106,7 +106,7 @@ def test_workspace_size_covers_either_gradient_kernel() -> None:
     assert lib.fhoad_backward_workspace_size(1) == per_slot
     assert lib.fhoad_backward_workspace_size(65536) == 256 * per_slot
     assert lib.fhoad_backward_workspace_size(1 << 20) == 256 * per_slot
-    for batch in (1, 16, 17, 64, 65, 1000, 4096, 12288, 12289, 20000):
+    for batch in (1, 16, 17, 64, 65, 1000, 4096, 8192, 8193, 12288, 12289, 20000):
         assert lib.fhoad_backward_workspace_size(batch) == _expected_workspace(batch), batch
     assert lib.fhoad_poisson_adam_step_workspace_size(0, 5) == 0
     for batch, boundary in ((64, 0), (65, 1), (1000, 200), (16384, 1024), (12000, 300)):

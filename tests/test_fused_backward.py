@@ -158,9 +158,9 @@ def test_backward_past_the_last_whole_round() -> None:
         assert torch.equal(gp, ref_p) and torch.equal(gx, ref_x), f"changed with {blocks} blocks"
 
 
-@pytest.mark.parametrize("batch", [1, 17, 1000, 4096, 12288])
+@pytest.mark.parametrize("batch", [1, 17, 1000, 4096, 8192, 12288])
 def test_split_backward_agrees_with_the_tiled_kernel(batch: int) -> None:
-    """Up to 768 16-point tiles the backward runs backward_split_kernel (rows split over a
+    """Up to 512 16-point tiles (8,192 points) the backward runs backward_split_kernel (rows split over a
     workgroup's waves). It does backward_kernel's arithmetic with the sums over points grouped
     differently, so the two agree to rounding: 1e-5 of each block's scale, ten times tighter
     than the parity bar."""
@@ -177,15 +177,20 @@ def test_split_backward_agrees_with_the_tiled_kernel(batch: int) -> None:
     assert_scaled_close(sx, tx, 1e-5, "grad_coordinates")
 
 
-@pytest.mark.parametrize("batch", [12288, 12289])
-def test_backward_on_both_sides_of_the_kernel_threshold(batch: int) -> None:
-    """12,288 points (768 16-point tiles) still run backward_split_kernel, 12,289 run
-    backward_kernel; both meet the parity bar against the recompute backward."""
-    announce(f"backward at the split-kernel threshold, batch={batch}, vs recompute")
+@pytest.mark.parametrize("batch,split", [(8192, "1"), (8193, "0")])
+def test_backward_on_both_sides_of_the_kernel_threshold(batch: int, split: str) -> None:
+    """8,192 points (512 16-point tiles) still run backward_split_kernel, 8,193 run
+    backward_kernel: bitwise what the forced kernel gives and not what the other one does. Both
+    meet the parity bar against the recompute backward."""
+    announce(f"backward at the split-kernel threshold, batch={batch}, vs forced kernels and recompute")
     (gp, gx), (ep, ex) = _pair(batch, seed=8)
     for name, lo, hi in BLOCKS:
         assert_scaled_close(gp[lo:hi], ep[lo:hi], 1e-4, name)
     assert_scaled_close(gx, ex, 1e-4, "grad_coordinates")
+    for value in "01":
+        with knobs(FUSED_HOAD_BWD_SPLIT=value):
+            (fp, _), _ = _pair(batch, seed=8)
+        assert torch.equal(fp, gp) == (value == split), f"FUSED_HOAD_BWD_SPLIT={value}"
 
 
 def test_split_backward_many_tiles_per_slot_and_saturated_tanh() -> None:

@@ -270,8 +270,8 @@ def _boundary(count: int, seed: int):
 
 @pytest.mark.parametrize(
     "batch,nb",
-    [(1000, 100), (100, 1), (100, 63), (64, 64), (100, 65), (12000, 288), (12000, 289), (20000, 1024),
-     (65537, 1025)],
+    [(1000, 100), (100, 1), (100, 63), (64, 64), (100, 65), (8000, 192), (8000, 193), (12000, 288), (12000, 289),
+     (20000, 1024), (65537, 1025)],
 )
 def test_pinn_step_with_boundary_matches_the_oracle(batch: int, nb: int) -> None:
     announce(f"fused PINN+Adam step (boundary term) vs float64 oracle, batch={batch}, boundary={nb}")
@@ -367,3 +367,25 @@ def test_split_gradient_kernel_agrees_with_the_tiled_one(batch: int, nb: int) ->
     assert loss_s == pytest.approx(loss_t, rel=1e-6)
     for name, start, end in _blocks():
         assert_scaled_close(grad_s[start:end], grad_t[start:end], 1e-5, name)
+
+
+@pytest.mark.parametrize("batch,nb,split", [(8192, 0, "1"), (8193, 0, "0"), (8000, 192, "1"), (8000, 193, "0")])
+def test_step_on_both_sides_of_the_kernel_threshold(batch: int, nb: int, split: str) -> None:
+    """512 16-point tiles, boundary tiles counted, still run backward_split_kernel and 513 run
+    backward_kernel: bitwise what the forced kernel gives and not what the other one does."""
+    announce(f"fused step at the split-kernel threshold, batch={batch}, boundary={nb}, vs forced kernels")
+    from fused_hoad.training import FusedPoissonAdam
+
+    x = coordinates(batch, seed=18)
+    xb = _boundary(nb, 18) if nb else None
+
+    def gradient(**knob: str):
+        trainer = FusedPoissonAdam(_model(3), x, boundary=xb)
+        with knobs(**knob):
+            trainer.step()
+        torch.cuda.synchronize()
+        return trainer.grad.clone()
+
+    default = gradient()
+    for value in "01":
+        assert torch.equal(gradient(FUSED_HOAD_BWD_SPLIT=value), default) == (value == split), value
