@@ -1,10 +1,10 @@
 """Benchmark of the fused forward-Laplacian path on one MI355X.
 
-Metric (BASELINE.json): residual points/s (u, Laplacian u) at 64K points plus train-step ms at
+Metric: residual points/s (u, Laplacian u) at 64K points plus train-step ms at
 64K points, FP32, 1 GPU. One "step" is one fused residual evaluation of 65,536 points
 (coordinates already in HBM). The training step (forward jet, loss mean((Laplacian u - f)^2)
 with f = -2 pi^2 sin(pi x) sin(pi y), adjoint jet, Adam lr 1e-3) is timed the same way at 65,536
-points with all of BASELINE config 3's outputs (gradients of every weight and bias and of the
+points with all of the step's outputs (gradients of every weight and bias and of the
 input coordinates): ``train_step_ms`` is the fused step (FusedPoissonAdam: one gradient kernel
 that re-runs the forward and seeds itself from the loss, one reduction kernel with the Adam
 update), ``train_step_graphed_ms`` the same replayed from a HIP graph, and
@@ -450,7 +450,7 @@ def main() -> None:
                 f"{ms:.3f} ms wall/step (flattened model; {note})")
 
     # ---- training step (b): the fused step, FusedPoissonAdam (2 kernels) ----
-    # All of config 3's outputs: the gradients of every weight and bias and of the input
+    # All of the step's outputs: the gradients of every weight and bias and of the input
     # coordinates (they require grad, so each step writes trainer.grad_coordinates, as the
     # reference's backward always writes grad_coordinates, csrc/fused_backward.cu:830-831).
     torch.manual_seed(0)

@@ -10,7 +10,7 @@ Behaviour of /root/reference/benchmarks/train_poisson.py:
 
 Backends are the reference's registry names that are trainable here (`eager`,
 `forward_laplacian`, `fused_cuda`, `fused_cuda_bwd_v1`, `fused_cuda_recompute`), all stepped
-through autograd and torch.optim.Adam. `fused_step` is this build's fused training step
+through autograd and torch.optim.Adam. `fused_step` is the fused training step
 (`FusedPoissonAdam`: loss, gradients and Adam in two kernels).
 
     python -m fused_hoad.train_poisson --backends fused_step fused_cuda --seeds 0 1 2

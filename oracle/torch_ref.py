@@ -4,7 +4,7 @@ TEST INFRASTRUCTURE ONLY (checker and CPU baseline). Only ``tests/``,
 ``__graft_entry__.smoke()`` and the ``cpu_baseline`` leg of ``bench.py`` may use it; the product
 never imports it.
 
-* ``forward_laplacian``: the PyTorch forward Laplacian the north star's forward tolerance
+* ``forward_laplacian``: the PyTorch forward Laplacian the forward kernels' tolerance
   (atol 1e-5 / rtol 1e-4) is stated against, /root/reference/src/fused_hoad/backends/
   forward_laplacian.py:28-132. The reference stacks (v, J, L) into one [batch, 4, 64] tensor;
   this restatement keeps the four components as separate [batch, 64] tensors, which is the

@@ -215,8 +215,7 @@ def test_forward_laplacian_matches_oracle_jet() -> None:
 
 @pytest.mark.parametrize("batch", [256, 1024])
 def test_forward_laplacian_matches_eager_in_float32(batch: int) -> None:
-    """1,024 points is BASELINE.json config 1 (the CPU residual), checked at its stated size
-    with the north star's FP32 tolerance."""
+    """1,024 points on the CPU, with the kernels' FP32 tolerance."""
     model, x = _model_and_coordinates(DEFAULT_POISSON_MLP, batch=batch, dtype=torch.float32)
     eu, expected = get_backend("eager")(model, x)
     u, actual = forward_laplacian(model, x)

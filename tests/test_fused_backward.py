@@ -1,7 +1,7 @@
 """GPU parity of the gfx950 backward kernels (through fused_hoad._C and the C ABI).
 
 Tolerance: max |error| <= 1e-4 x max |expected| for the whole parameter gradient, for each of
-the 10 weight/bias blocks separately, and for the coordinate gradient (the north star's bar;
+the 10 weight/bias blocks separately, and for the coordinate gradient (the parity bar;
 the reference's test_fused.py:185-218). Expected values come from the PyTorch reference
 backward (autograd through the jet, oracle/torch_ref.py) in FP32 on the GPU, and from the
 float64 closed-form oracle (oracle/jet.py).

@@ -1,7 +1,7 @@
 """GPU parity of the gfx950 forward kernel (through fused_hoad._C and the C ABI).
 
 Tolerances: against the PyTorch forward Laplacian in FP32 (oracle/torch_ref.py, the
-reference's forward_laplacian.py restated) atol 1e-5 / rtol 1e-4, the north star's bar and
+reference's forward_laplacian.py restated) atol 1e-5 / rtol 1e-4, the parity bar and
 the reference's test_fused.py:27-35; against the float64 oracle with saturating weights
 max |error| <= 1e-4 max |expected| (test_fused.py:38-49).
 """
@@ -32,7 +32,7 @@ def _fused(x, p, version=2):
 
 # the reference's tile edges (test_fused.py:28) plus this kernel's: 16-point wave tiles, and
 # ragged large batches (a partial last tile, workgroups with unequal tile counts); 1,024 and
-# 16,384 are BASELINE.json configs 1 and 2
+# 16,384 points are among the benchmark's sizes
 @pytest.mark.parametrize(
     "batch",
     [1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 1000, 1024, 4097, 16384, 16401, 65536, 65537,

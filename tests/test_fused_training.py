@@ -338,9 +338,9 @@ def test_graph_captured_training_step_matches_eager_step() -> None:
 @pytest.mark.parametrize("mode", ["cuda", "saved"])
 def test_graph_captured_flattened_step_matches_eager_at_64k(mode: str) -> None:
     """The drop-in step bench.py times as train_step_autograd_graphed_ms, and the same with
-    backward="saved": a flattened model at 65,536 points (BASELINE config 3's size, where torch's mean reduces over many blocks), captured whole and replayed 10 times
-    with a host sync between replays, against the same steps run eagerly: every replay's loss
-    (rtol 1e-4) and the weights after."""
+    backward="saved": a flattened model at 65,536 points (where torch's mean reduces over many
+    blocks), captured whole and replayed 10 times with a host sync between replays, against the
+    same steps run eagerly: every replay's loss (rtol 1e-4) and the weights after."""
     announce(f"whole-step graph capture vs eager, flattened model, batch=65536, backward={mode}")
     from fused_hoad import manufactured_source
     from fused_hoad.backends.fused import fused_laplacian
